@@ -5,6 +5,9 @@
 // materialised transpose (the reference transposes then multiplies,
 // functions/matrix_ops.cpp:8-24, with a SIMT kernel, matrix.cu:21-145).
 //
+// Most products with K > 32 run on the bf16 matrix cores instead, each operand
+// in three parts (gemm_bf3.hpp; bf3_ok says which).
+//
 // Tiling.  A workgroup of 4 waves owns a BM x BN tile of C; the waves form a
 // WGM x WGN grid and each wave owns TM x TN blocks of 32x32, accumulated by
 // one MFMA chain per block.  K advances BK = 32 at a time through two LDS
@@ -82,8 +85,8 @@ struct GemmArgs {
   const float* bias;   // per-column bias added to the final output (or null)
   int vec_out;         // C (and the bias) take 128-bit stores: n, ldc % 4 == 0, 16-byte aligned
   int relu;            // with a bias: ReLU after it (Linear followed by ReLU)
-  float* colsum;       // column sums of op(B) (+)= into it (or null): tiny kernel and LDS
-                       // tiles with B untransposed and K unsplit
+  float* colsum;       // column sums of op(B) (+)= into it (or null): tiny and short-K kernels,
+                       // bf16 path with B untransposed, LDS tiles with K unsplit as well
   int colsum_acc;
   const float* bmask;  // tiny kernel, B untransposed: B[k][j] counts only where
                        // 0 < bmask[k][j] < +inf (ReLU's backward mask; same layout as B)
@@ -407,6 +410,14 @@ int launch_fold(Runtime* rt, float* c, const float* part, int m, int n, int ldc,
   LMP_LAUNCH_CHECK("fold_splits");
   return LMP_OK;
 }
+
+}  // namespace
+}  // namespace lmp_hip
+
+#include "gemm_bf3.hpp"
+
+namespace lmp_hip {
+namespace {
 
 // ------------------------------------------------------------------ direct
 //
@@ -1287,28 +1298,6 @@ __global__ __launch_bounds__(NT, MINB) void gemm_f32_lds(GemmArgs g) {
   gemm_f32_lds_tile<C, TA, TB>(g, int(blockIdx.x), int(blockIdx.z), gridDim.z > 1, smem);
 }
 
-// Two independent products in one launch (a Linear's weight gradient A and
-// input gradient B): workgroups [0, tiles_a * splits_a) compute product A in
-// the order of its own launch (split-major, as blockIdx.z then x), the rest
-// product B, so every tile and partial holds the bits the product's own
-// launch gives.  The CUs product A frees start B's first loads while A's last
-// stores drain, where two launches would drain and refill one after the other.
-template <int NT, int MINB, class CA, bool TAA, bool TBA, class CB, bool TAB, bool TBB>
-__global__ __launch_bounds__(NT, MINB) void gemm_f32_lds_pair(GemmArgs ga, int splits_a,
-                                                              GemmArgs gb, int splits_b) {
-  static_assert(NT == CA::THREADS && NT == CB::THREADS, "one workgroup size for both");
-  constexpr int FA = CA::STAGES * CA::STAGE, FB = CB::STAGES * CB::STAGE;
-  __shared__ __attribute__((aligned(1024))) float smem[FA > FB ? FA : FB];
-  const int tiles_a = ga.tiles_m * ga.tiles_n, tiles_b = gb.tiles_m * gb.tiles_n;
-  const int i = int(blockIdx.x);
-  if (i < tiles_a * splits_a) {
-    gemm_f32_lds_tile<CA, TAA, TBA>(ga, i % tiles_a, i / tiles_a, splits_a > 1, smem);
-  } else {
-    const int j = i - tiles_a * splits_a;
-    gemm_f32_lds_tile<CB, TAB, TBB>(gb, j % tiles_b, j / tiles_b, splits_b > 1, smem);
-  }
-}
-
 // ------------------------------------------------------------------ rows
 //
 // M <= 32 with B transposed and enough columns to give every CU a block of
@@ -1837,21 +1826,23 @@ int launch_rows(Runtime* rt, const GemmArgs& g0) {
   return LMP_OK;
 }
 
-// Kernel choice (measured on MI355X, fp32), in order: the tiny kernel for
-// small latency-bound products (K <= 512, at most 2^21 multiply-adds); the
+// Kernel choice (measured on MI355X), in order: the tiny kernel for small
+// latency-bound products (K <= 512, at most 2^21 multiply-adds); the
 // persistent short-K kernel (A transposed, K <= 32); whole rows of B per
 // workgroup (M <= 32, B transposed, a 32-column block per CU); the
-// register-direct kernel (M <= 32) and 32 x 256 tiles (M <= 64); then, with
-// 16-byte operand rows, the LDS-DMA configurations (256 x 256 when they cover
-// the CUs, 256 x 128 split for M >= 512, N >= 2048, K >= 2048, 128 x 64 split
-// when 128 x 128 tiles would not cover the CUs); otherwise 64 x 64 register
-// tiles without a split for a short K (<= 2048) with too few 128 x 128 tiles,
-// else 128 x 128 (on LDS-DMA tiles when the rows allow) with split K.  Single
-// and paired launches take their kernel from this one function.
-enum class Route { Tiny, Short, Rows, Direct, Skinny, Big, Wide, Mid, Small64, Large };
+// register-direct kernel (M <= 32); the bf16 matrix cores (bf3_ok below, tiles
+// and split of K by bf3_plan); then the fp32 MFMAs: 32 x 256 tiles (M <= 64)
+// and, with 16-byte operand rows, the LDS-DMA configurations (256 x 256 when
+// they cover the CUs, 256 x 128 split for M >= 512, N >= 2048, K >= 2048,
+// 128 x 64 split when 128 x 128 tiles would not cover the CUs); otherwise 64 x
+// 64 register tiles without a split for a short K (<= 2048) with too few 128 x
+// 128 tiles, else 128 x 128 (on LDS-DMA tiles when the rows allow) with split
+// K.  Single and paired launches take their kernel from these functions.
+enum class Route { Tiny, Short, Rows, Direct, Bf3, Skinny, Big, Wide, Mid, Small64, Large };
 
+// The choice among the fp32 kernels.
 template <bool TA, bool TB>
-Route gemm_route(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok) {
+Route gemm_route_f32(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok) {
   if (tiny_ok(g)) return Route::Tiny;
   // K <= 32 with A transposed (a Linear's weight gradient at a small batch):
   // the persistent short-K kernel, whose tiles and orders are those of the
@@ -1888,6 +1879,31 @@ Route gemm_route(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok) {
   return Route::Large;
 }
 
+// Whether the product may run on the bf16 matrix cores (in place of any fp32
+// kernel but the tiny, short-K and M <= 32 ones):
+//   K > 32, where the error against float64 is no larger than the fp32 MFMAs'
+//     (512 x 512 outputs, normal operands, unsplit: 7.4e-8 fp32 and 8.3e-8
+//     here at K = 16, 1.02e-7 and 1.04e-7 at 32, 1.44e-7 and 1.35e-7 at 64;
+//     4096^3: 1.15e-6 and 1.01e-6);
+//   not a forward product X * W (neither transposed) of up to 512 rows.  Those
+//     are a training step's, and any other rounding of them moves the ReLU
+//     inputs that lie within it of zero to the other side: a step of the wide
+//     net (512 rows) on these products as well took 690 us instead of 755 us,
+//     but its updated weights then differed by up to 1.7e-5 from the fp32
+//     kernels' (themselves 1.5e-5 from float64 for the same reason), more than
+//     the 1e-5 that perf/cases.py holds a training step to.
+template <bool TA, bool TB>
+bool bf3_ok(const GemmArgs& g) {
+  return g.k > kBK && (TA || TB || g.m > 512);
+}
+
+template <bool TA, bool TB>
+Route gemm_route(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok) {
+  const Route r = gemm_route_f32<TA, TB>(rt, g, vec, direct_ok);
+  const bool own = r == Route::Tiny || r == Route::Short || r == Route::Rows || r == Route::Direct;
+  return !own && bf3_ok<TA, TB>(g) ? Route::Bf3 : r;
+}
+
 template <bool TA, bool TB>
 int launch_gemm(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok, const Workspace& ws,
                 bool* colsum_done = nullptr) {
@@ -1900,96 +1916,56 @@ int launch_gemm(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok, const 
     // With B transposed a wave's loads touch more cache lines per byte, so
     // three fragments in flight instead of two.
     case Route::Direct: return launch_direct<TA, TB, TB ? 3 : 2>(rt, g, ws);
+    case Route::Bf3: return launch_bf3_planned<TA, TB>(rt, g, ws, colsum_done);
     case Route::Skinny: return launch_gemm_cfg<CfgSkinny, TA, TB>(rt, g, vec, ws);
-    case Route::Big: return launch_lds<LdsBig, TA, TB>(rt, g, ws, colsum_done);
-    case Route::Wide: return launch_lds<LdsWide, TA, TB>(rt, g, ws, colsum_done);
-    case Route::Mid: return launch_lds<LdsMid, TA, TB>(rt, g, ws, colsum_done);
     case Route::Small64: return launch_gemm_cfg<CfgSmall, TA, TB>(rt, g, vec, ws, 1);
     case Route::Large: return launch_gemm_cfg<CfgLarge, TA, TB>(rt, g, vec, ws, 0, colsum_done);
+    // These three take K >= 256, where only X * W stays on the fp32 MFMAs.
+    case Route::Big:
+      if constexpr (!TA && !TB) return launch_lds<LdsBig, TA, TB>(rt, g, ws, colsum_done);
+      break;
+    case Route::Wide:
+      if constexpr (!TA && !TB) return launch_lds<LdsWide, TA, TB>(rt, g, ws, colsum_done);
+      break;
+    case Route::Mid:
+      if constexpr (!TA && !TB) return launch_lds<LdsMid, TA, TB>(rt, g, ws, colsum_done);
+      break;
   }
   return fail(LMP_ERR_RUNTIME, "gemm: no kernel for this product");
 }
 
+// Bytes of split-K partials by which the no-allocation entry point decides
+// whether it serves a product of the bf16 path.  The set of products it
+// accepts is part of its interface and was fixed by the fp32 kernels' splits;
+// the bf16 path's own partials always fit the workspace.
+template <bool TA, bool TB>
+int64_t noalloc_bytes(Runtime* rt, GemmArgs g, bool vec, bool direct_ok) {
+  if (gemm_route<TA, TB>(rt, g, vec, direct_ok) != Route::Bf3) return 0;  // checked at the launch
+  int splits = 1;
+  switch (gemm_route_f32<TA, TB>(rt, g, vec, direct_ok)) {
+    case Route::Skinny: splits = set_split(rt, g, CfgSkinny::BM, CfgSkinny::BN, 0); break;
+    case Route::Big: splits = set_split_lds<LdsBig>(rt, g); break;
+    case Route::Wide: splits = set_split_lds<LdsWide>(rt, g); break;
+    case Route::Mid: splits = set_split_lds<LdsMid>(rt, g); break;
+    case Route::Large: splits = set_split(rt, g, CfgLarge::BM, CfgLarge::BN, 0); break;
+    default: break;
+  }
+  return splits > 1 ? int64_t(splits) * g.m * g.n * int64_t(sizeof(float)) : 0;
+}
+
 // ------------------------------------------------------ weight + input pair
 
-// The LDS configuration a product's own launch would use, with its tiles and
-// split set in g: 0 (not an LDS-tile launch), else the configuration's id
-// (1 Big, 2 Wide, 3 Mid, 4 the 128 x 128 LDS tiles of the Large route).
-template <bool TA, bool TB>
-int lds_config_of(Runtime* rt, GemmArgs& g, bool vec, bool direct_ok, int* splits) {
-  switch (gemm_route<TA, TB>(rt, g, vec, direct_ok)) {
-    case Route::Big: *splits = set_split_lds<LdsBig>(rt, g); return 1;
-    case Route::Wide: *splits = set_split_lds<LdsWide>(rt, g); return 2;
-    case Route::Mid: *splits = set_split_lds<LdsMid>(rt, g); return 3;
-    case Route::Large:
-      if (!vec) return 0;
-      *splits = set_split(rt, g, CfgLarge::BM, CfgLarge::BN, 0);
-      return 4;
-    default: return 0;
-  }
-}
-
-template <class CW, class CX>
-int launch_pair(Runtime* rt, GemmArgs gw, int sw, GemmArgs gx, int sx) {
-  static_assert(CW::THREADS == CX::THREADS, "one workgroup size for both");
-  const Workspace ws{};
-  float* pw = nullptr;
-  float* px = nullptr;
-  float* const cw = gw.c;
-  float* const cx = gx.c;
-  if (sw > 1) {
-    const int rc = ws.take(size_t(sw) * size_t(gw.m) * size_t(gw.n) * sizeof(float), &pw);
-    if (rc != LMP_OK) return rc;
-    gw.c = pw;
-  }
-  if (sx > 1) {
-    const int rc = ws.take(size_t(sx) * size_t(gx.m) * size_t(gx.n) * sizeof(float), &px);
-    if (rc != LMP_OK) {
-      if (pw) ws.give(pw);
-      return rc;
-    }
-    gx.c = px;
-  }
-  constexpr int kMinB = CW::MINB > CX::MINB ? CW::MINB : CX::MINB;
-  const int64_t wgs = int64_t(gw.tiles_m) * gw.tiles_n * sw + int64_t(gx.tiles_m) * gx.tiles_n * sx;
-  hipLaunchKernelGGL((gemm_f32_lds_pair<CW::THREADS, kMinB, CW, true, false, CX, false, true>),
-                     dim3(uint32_t(wgs)), dim3(CW::THREADS), 0, rt->stream, gw, sw, gx, sx);
-  LMP_LAUNCH_CHECK("gemm_f32_lds_pair");
-  int rc = LMP_OK;
-  if (sw > 1) rc = launch_fold(rt, cw, pw, gw.m, gw.n, gw.ldc, sw, gw.accumulate, nullptr, 0);
-  if (rc == LMP_OK && sx > 1)
-    rc = launch_fold(rt, cx, px, gx.m, gx.n, gx.ldc, sx, gx.accumulate, nullptr, 0);
-  if (pw) ws.give(pw);  // stream-ordered: the folds read them first
-  if (px) ws.give(px);
-  return rc;
-}
-
 // dW = X^T G (with db, the column sums of G, when gw.colsum is set) and
-// dX = G W^T in one launch when both take LDS tiles of one workgroup size,
-// each with the configuration and split of its own launch (so the same bits
-// as lmp_k_gemm_colsum_f32 and lmp_k_gemm_f32); the column sums must then ride
-// in the dW tiles (dW unsplit).  Returns false, with nothing launched, when
-// the pair does not apply.
-bool try_linear_backward_pair(Runtime* rt, GemmArgs gw, bool vec_w, bool direct_w, GemmArgs gx,
-                              bool vec_x, bool direct_x, int* rc) {
-  int sw = 1, sx = 1;
-  const int kw = lds_config_of<true, false>(rt, gw, vec_w, direct_w, &sw);
-  const int kx = lds_config_of<false, true>(rt, gx, vec_x, direct_x, &sx);
-  if (kw == 0 || kx == 0) return false;
-  if (gw.colsum && sw > 1) return false;
-  const bool wide_w = kw <= 2, wide_x = kx <= 2;  // 512-thread configurations
-  if (wide_w != wide_x) return false;
-  switch (kw * 8 + kx) {
-    case 1 * 8 + 1: *rc = launch_pair<LdsBig, LdsBig>(rt, gw, sw, gx, sx); return true;
-    case 1 * 8 + 2: *rc = launch_pair<LdsBig, LdsWide>(rt, gw, sw, gx, sx); return true;
-    case 2 * 8 + 1: *rc = launch_pair<LdsWide, LdsBig>(rt, gw, sw, gx, sx); return true;
-    case 2 * 8 + 2: *rc = launch_pair<LdsWide, LdsWide>(rt, gw, sw, gx, sx); return true;
-    case 3 * 8 + 3: *rc = launch_pair<LdsMid, LdsMid>(rt, gw, sw, gx, sx); return true;
-    case 3 * 8 + 4: *rc = launch_pair<LdsMid, LdsSmall>(rt, gw, sw, gx, sx); return true;
-    case 4 * 8 + 3: *rc = launch_pair<LdsSmall, LdsMid>(rt, gw, sw, gx, sx); return true;
-    case 4 * 8 + 4: *rc = launch_pair<LdsSmall, LdsSmall>(rt, gw, sw, gx, sx); return true;
-    default: return false;
-  }
+// dX = G W^T in one launch when both run on the bf16 path with one workgroup
+// size, each with the tiles and split of its own launch (so the same bits as
+// lmp_k_gemm_colsum_f32 and lmp_k_gemm_f32).  Returns false, with nothing
+// launched, when the pair does not apply.
+bool try_linear_backward_pair(Runtime* rt, const GemmArgs& gw, bool vec_w, bool direct_w,
+                              const GemmArgs& gx, bool vec_x, bool direct_x, int* rc) {
+  if (gemm_route<true, false>(rt, gw, vec_w, direct_w) != Route::Bf3 ||
+      gemm_route<false, true>(rt, gx, vec_x, direct_x) != Route::Bf3)
+    return false;
+  return launch_bf3_pair_planned(rt, gw, gx, rc);
 }
 
 bool aligned16(const void* p) {
@@ -2126,6 +2102,15 @@ int gemm_f32_entry(int trans_a, int trans_b, size_t m, size_t n, size_t k,
   g.colsum_acc = colsum_acc ? 1 : 0;
   bool vec = false, direct_ok = false;
   gemm_flags(g, trans_a, trans_b, &vec, &direct_ok);
+  if (ws.fixed) {
+    const int64_t need =
+        !trans_a ? (!trans_b ? noalloc_bytes<false, false>(rt, g, vec, direct_ok)
+                             : noalloc_bytes<false, true>(rt, g, vec, direct_ok))
+                 : (!trans_b ? noalloc_bytes<true, false>(rt, g, vec, direct_ok)
+                             : noalloc_bytes<true, true>(rt, g, vec, direct_ok));
+    float* unused = nullptr;
+    if (const int wrc = ws.take(size_t(need), &unused); wrc != LMP_OK) return wrc;
+  }
   bool* cd = colsum_done;
   int rc;
   if (!trans_a && !trans_b) rc = launch_gemm<false, false>(rt, g, vec, direct_ok, ws, cd);

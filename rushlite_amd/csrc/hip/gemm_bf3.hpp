@@ -1,0 +1,763 @@
+// fp32 GEMM on the bf16 matrix cores, each operand split into three bf16 parts.
+//
+// Why.  v_mfma_f32_32x32x2_f32 does 64 flop per cycle and SIMD (157 TFLOP/s on
+// the chip); v_mfma_f32_32x32x16_bf16 does 1024.  An fp32 value x scaled by
+// 2^24 is h + m + l exactly (h = bf16(x), m = bf16(x - h), l = x - h - m: 8
+// bits each, round to nearest), so
+//   a*b = ah*bh + ah*bm + am*bh + am*bm + ah*bl + al*bh + (terms below 2^-26)
+// takes six bf16 MFMAs with fp32 accumulation: 2.5 PFLOP/s / 6 = 419 TFLOP/s.
+// The error against float64 is that of the accumulation: six roundings per 16
+// values of k here, eight or more on the fp32 MFMAs (4096^3, normal operands:
+// 1.01e-6 against 1.15e-6; 512^3: 3.5e-7 against 4.0e-7).  At K = 32 and
+// below the dropped terms show, and those products stay on the fp32 MFMAs.
+//
+// Range.  The scaling makes the split exact for every finite fp32 value,
+// subnormals included (the last bit of one, 2^-149, becomes 2^-125, a normal
+// bf16), up to 2^103 for operands and 2^80 for results.  Whatever exceeds
+// that, and every infinity and NaN of the operands, leaves a non-finite value
+// in the accumulator (an infinite h has m = NaN), so a workgroup that finds
+// one after its K loop computes its tile again with fp32 MFMAs on the
+// unscaled operands (fallback below): infinities, NaN and overflow come out as
+// fp32 products give them, and no other value takes that path unnoticed.
+//
+// What bounds it: power.  4096^3 takes 575-607 us on normal operands (227-239
+// TFLOP/s = 1.36-1.43 PFLOP/s of bf16, where a bf16 product of 8192^3 through
+// the vendor library reached 1.26) and 395-420 us on zeros: the clock falls
+// under the MFMAs of random operands.  The fp32 MFMA kernel it replaced took
+// 965 us (143 TFLOP/s); a Linear's backward of 1000 x 2047 x 1531 (odd rows,
+// register-staged fp32 tiles and a separate column reduction) 212 -> 84 us;
+// the two backward products of 512 x 4096 x 4096 281 -> 181 us.
+//
+// Structure.  A workgroup owns a BM x BN tile of C, its waves TM x TN blocks
+// of 32 x 32 each; K advances 16 at a time through two LDS stages with one
+// barrier per step.  Loads go through registers (any alignment, any
+// orientation, one step ahead), are split there and stored to LDS as three
+// planes of 16-byte octets, [plane][k / 8][row], in which a fragment of one
+// MFMA is one conflict-free 128-bit read per lane; 64 bytes between the two
+// octets keep the stores of k-contiguous operands off each other's banks.
+// Each operand value is converted once per workgroup (13 VALU operations per
+// pair, spread over the MFMAs by hand: a pair, then MPC MFMAs), and a fragment
+// feeds TN (or TM) x 2 MFMAs per plane, so neither the VALU nor the LDS is
+// near its limit.  The last of the six products is held past the barrier: it
+// reads registers only and covers the first fragment reads of the next step.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdint>
+#include <type_traits>
+
+namespace lmp_hip {
+namespace {
+
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+constexpr int kBf3K = 16;                               // k values per step
+constexpr float kBf3Scale = 16777216.0f;                // 2^24, on each operand
+constexpr float kBf3Unscale = 3.552713678800501e-15f;   // 2^-48, on the result
+
+// Kept out of the templates, as lds_dma16 is: a target builtin inside a kernel
+// template keeps the host pass from emitting the kernel's launch stub.
+__device__ __forceinline__ v16f mfma_bf16(bf8 a, bf8 b, v16f c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ v16f mfma_f32(float a, float b, v16f c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{x, y}, bf2));
+}
+__device__ __forceinline__ float bf16_low(uint32_t u) {
+  return __builtin_bit_cast(float, u << 16);
+}
+__device__ __forceinline__ float bf16_high(uint32_t u) {
+  return __builtin_bit_cast(float, u & 0xffff0000u);
+}
+// Two values into the three parts, packed.
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32_t& m,
+                                           uint32_t& l) {
+  const float xs = x * kBf3Scale, ys = y * kBf3Scale;
+  h = pack_bf16(xs, ys);
+  const float xr = xs - bf16_low(h), yr = ys - bf16_high(h);
+  m = pack_bf16(xr, yr);
+  l = pack_bf16(xr - bf16_low(m), yr - bf16_high(m));
+}
+
+// DEPTH: steps of loads in flight ahead of the one being split.
+template <int WM_, int WN_, int TM_, int TN_, int DEPTH_, int MINB_>
+struct Bf3Cfg {
+  static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, DEPTH = DEPTH_, MINB = MINB_;
+  static constexpr int NW = WM * WN, THREADS = 64 * NW;
+  static constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
+  static constexpr int A_OCT = BM * 16 + 64, B_OCT = BN * 16 + 64;  // bytes
+  static constexpr int A_PLANE = 2 * A_OCT, B_PLANE = 2 * B_OCT;
+  static constexpr int STAGE = 3 * (A_PLANE + B_PLANE);
+  static constexpr int SMEM = 2 * STAGE + 16;  // the stages and the fallback's flag
+  static_assert(2 * STAGE >= NW * 32 * 36 * 4, "the epilogue's wave tiles fit");
+};
+
+// One operand's panel of R rows (of m or n) x 16 k on its way from memory to
+// LDS.  A thread holds ITEMS items of W consecutive k values of one row, in
+// SETS register sets (steps in flight).  KMAJOR: k is contiguous in memory.
+// Rows past the matrix read its last row (their results are never stored).
+template <int R, int THREADS, bool KMAJOR, int SETS>
+struct Bf3Panel {
+  static constexpr int W = R * 2 >= THREADS ? 8 : 4;
+  static constexpr int PER_ROW = kBf3K / W;
+  static constexpr int ITEMS = R * PER_ROW / THREADS;
+  static constexpr int PAIRS = ITEMS * (W / 2);  // of this thread, per step
+  static_assert(ITEMS * THREADS == R * PER_ROW, "items split evenly over the threads");
+  const float* p[ITEMS];
+  int ld, k[ITEMS], off[ITEMS];
+  float v[SETS][ITEMS][W];
+  float cs[ITEMS];  // column sums (bias gradient), where they are asked for
+
+  // `k0`: the first k that load() reads.
+  __device__ __forceinline__ void init(const float* base, int ld_, int r0, int rows, int k0,
+                                       int oct_bytes) {
+    ld = ld_;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int q = int(threadIdx.x) + i * THREADS;
+      const int row = KMAJOR ? q / PER_ROW : q % R;
+      k[i] = W * (KMAJOR ? q % PER_ROW : q / R);
+      const int64_t r = min(r0 + row, rows - 1);
+      p[i] = base + (KMAJOR ? r * ld + (k0 + k[i]) : int64_t(k0 + k[i]) * ld + r);
+      off[i] = (k[i] / 8) * oct_bytes + row * 16 + (k[i] % 8) * 2;
+      cs[i] = 0.0f;
+    }
+  }
+  // The item's values of a whole step; the next load reads `advance` k on.
+  __device__ __forceinline__ void load(int set, int i, int advance) {
+    if constexpr (KMAJOR) {
+#pragma unroll
+      for (int j = 0; j < W; j += 4) {
+        const v4f_any x = *reinterpret_cast<const v4f_any*>(p[i] + j);
+        v[set][i][j] = x.x; v[set][i][j + 1] = x.y; v[set][i][j + 2] = x.z; v[set][i][j + 3] = x.w;
+      }
+      p[i] += advance;
+    } else {
+#pragma unroll
+      for (int j = 0; j < W; ++j) v[set][i][j] = p[i][int64_t(j) * ld];
+      p[i] += int64_t(advance) * ld;
+    }
+  }
+  __device__ __forceinline__ void load_all(int set, int advance) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) load(set, i, advance);
+  }
+  // A step of `left` values of k that starts `at` k past the pointers, zeros
+  // after them.
+  __device__ __forceinline__ void load_tail(int set, int at, int left) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i)
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        v[set][i][j] = 0.0f;
+        if (k[i] + j < left)
+          v[set][i][j] = KMAJOR ? p[i][at + j] : p[i][int64_t(at + j) * ld];
+      }
+  }
+  __device__ __forceinline__ void add_cs(int set) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i)
+#pragma unroll
+      for (int j = 0; j < W; ++j) cs[i] += v[set][i][j];
+  }
+  // Stores an item's parts (h, m, l: W / 2 packed pairs) into the three planes.
+  __device__ __forceinline__ void put(int i, char* lds, int plane, const uint32_t (&h)[4],
+                                      const uint32_t (&m)[4], const uint32_t (&l)[4]) const {
+    char* q = lds + off[i];
+    if constexpr (W == 8) {
+      *reinterpret_cast<u4*>(q) = u4{h[0], h[1], h[2], h[3]};
+      *reinterpret_cast<u4*>(q + plane) = u4{m[0], m[1], m[2], m[3]};
+      *reinterpret_cast<u4*>(q + 2 * plane) = u4{l[0], l[1], l[2], l[3]};
+    } else {
+      *reinterpret_cast<u2*>(q) = u2{h[0], h[1]};
+      *reinterpret_cast<u2*>(q + plane) = u2{m[0], m[1]};
+      *reinterpret_cast<u2*>(q + 2 * plane) = u2{l[0], l[1]};
+    }
+  }
+  __device__ __forceinline__ void store_all(int set, char* lds, int plane) const {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      uint32_t h[4], m[4], l[4];
+#pragma unroll
+      for (int j = 0; j < W / 2; ++j)
+        split_pair(v[set][i][2 * j], v[set][i][2 * j + 1], h[j], m[j], l[j]);
+      put(i, lds, plane, h, m, l);
+    }
+  }
+};
+
+struct Bf3Args {
+  GemmArgs g;
+  int splits, steps_per_split;  // K splits, and 16-wide k steps in each
+  // Partials of split s (splits > 1): C's m * n values at part + s *
+  // part_stride and, with column sums, their n values cs_at after it; both
+  // start on 16 bytes.
+  float* part;
+  int64_t part_stride, cs_at;
+};
+
+// Work item `id` of the product (in [0, tiles * splits)) for this workgroup.
+template <class C, bool TA, bool TB>
+__device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char* smem) {
+  const GemmArgs& g = args.g;
+  constexpr int TM = C::TM, TN = C::TN, MM = TM * TN;
+  // Consecutive ids go round the eight XCDs: give each XCD a contiguous run of
+  // (split, tile), so its L2 sees one range of k and neighbouring tiles.
+  const int ntiles = g.tiles_m * g.tiles_n, total = ntiles * args.splits;
+  {
+    const int q = total / 8, r = total % 8, x = id % 8;
+    id = x * q + min(x, r) + id / 8;
+  }
+  const int split = id / ntiles, tile = id - split * ntiles;
+  constexpr int kGroup = 8;  // tile rows walked together
+  const int per_group = kGroup * g.tiles_n, group = tile / per_group;
+  const int gsize = min(g.tiles_m - group * kGroup, kGroup);
+  const int in_group = tile - group * per_group;
+  const int tile_m = group * kGroup + in_group % gsize;
+  const int m0 = tile_m * C::BM, n0 = (in_group / gsize) * C::BN;
+
+  const int k_begin = split * args.steps_per_split * kBf3K;
+  const int k_len = min(g.k - k_begin, args.steps_per_split * kBf3K);
+  const int full = k_len / kBf3K, left = k_len % kBf3K, steps = full + (left ? 1 : 0);
+  const bool partial = args.splits > 1;
+  int* flag = reinterpret_cast<int*>(smem + 2 * C::STAGE);
+  if (threadIdx.x == 0) *flag = 0;  // set after the K loop's barriers
+  const bool do_cs = !TB && g.colsum != nullptr && tile_m == 0;  // uniform
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / C::WN, wn = wave % C::WN;
+  const int li = lane & 31, lh = lane >> 5;
+
+  using PA = Bf3Panel<C::BM, C::THREADS, !TA, C::DEPTH>;
+  using PB = Bf3Panel<C::BN, C::THREADS, TB, C::DEPTH>;
+  PA pa;
+  PB pb;
+  // Loads past the last whole step repeat it (and are not used); a split
+  // without a whole step reads the 16 k before the end of K for them (K > 32).
+  const int k_load = min(k_begin, g.k - kBf3K);
+  pa.init(g.a, g.lda, m0, g.m, k_load, C::A_OCT);
+  pb.init(g.b, g.ldb, n0, g.n, k_load, C::B_OCT);
+
+  v16f acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = v16f(0.0f);
+
+  const int a_at = lh * C::A_OCT + (wm * TM * 32 + li) * 16;
+  const int b_at = 3 * C::A_PLANE + lh * C::B_OCT + (wn * TN * 32 + li) * 16;
+  bf8 fa[3][TM], fb[3][TN];
+  auto read_a = [&](const char* s, int p) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      fa[p][i] = *reinterpret_cast<const bf8*>(s + p * C::A_PLANE + a_at + i * 512);
+  };
+  auto read_b = [&](const char* s, int p) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      fb[p][j] = *reinterpret_cast<const bf8*>(s + p * C::B_PLANE + b_at + j * 512);
+  };
+  auto mma = [&](int p, int q) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma_bf16(fa[p][i], fb[q][j], acc[i][j]);
+  };
+
+  // The step with the end of K first (when 16 does not divide it), then the
+  // whole ones.  Stage t % 2 holds step t, the register sets the DEPTH steps
+  // after it: step u in set u % DEPTH.
+  int ahead = full;  // whole steps not loaded yet
+  auto advance = [&]() { return ahead > 1 ? kBf3K : 0; };
+  if (left) {
+    pa.load_tail(0, k_begin - k_load + full * kBf3K, left);
+    pb.load_tail(0, k_begin - k_load + full * kBf3K, left);
+  } else {
+    pa.load_all(0, advance());
+    pb.load_all(0, advance());
+    --ahead;
+  }
+  if constexpr (!TB)
+    if (do_cs) pb.add_cs(0);
+  pa.store_all(0, smem, C::A_PLANE);
+  pb.store_all(0, smem + 3 * C::A_PLANE, C::B_PLANE);
+#pragma unroll
+  for (int d = 1; d <= C::DEPTH; ++d) {
+    const int adv = advance();
+    pa.load_all(d % C::DEPTH, adv);
+    pb.load_all(d % C::DEPTH, adv);
+    --ahead;
+  }
+  // Product (1, 1) of the step before is held past the barrier; zeros at first.
+#pragma unroll
+  for (int i = 0; i < TM; ++i) fa[1][i] = bf8(0);
+#pragma unroll
+  for (int j = 0; j < TN; ++j) fb[1][j] = bf8(0);
+  constexpr int PA_OF[5] = {0, 0, 2, 1, 0}, PB_OF[5] = {0, 2, 0, 0, 1};
+  constexpr int PAIRS = PA::PAIRS + PB::PAIRS;
+  constexpr int MPC = (5 * MM - MM / 2) / PAIRS > 0 ? (5 * MM - MM / 2) / PAIRS : 1;
+  // One step: STAGE holds it, SET the next one.
+  auto step = [&](auto stage_c, auto set_c, int t) {
+    constexpr int stage = decltype(stage_c)::value, set = decltype(set_c)::value;
+    const char* s = smem + stage * C::STAGE;
+    char* d = smem + (stage ^ 1) * C::STAGE;
+    __syncthreads();
+    if constexpr (!TB)
+      if (do_cs && t + 1 < steps) pb.add_cs(set);
+    const int adv = advance();
+    --ahead;
+    read_a(s, 0);
+    read_b(s, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    read_b(s, 2);
+    uint32_t h[4], m[4], l[4];
+#pragma unroll
+    for (int c = 0; c < PAIRS; ++c) {
+      // The next product's fragments, half a product or more ahead of it.
+      const int q0 = c * MPC, q1 = c == PAIRS - 1 ? 5 * MM : q0 + MPC;
+      auto covers = [&](int q) { return q0 <= q && q < q1; };
+      if (covers(MM / 2)) read_a(s, 2);
+      if (covers(MM + MM / 2)) read_a(s, 1);
+      if (covers(3 * MM - 1)) read_b(s, 1);
+      const bool of_a = c < PA::PAIRS;
+      const int ca = of_a ? c : c - PA::PAIRS;
+      const int it = of_a ? ca / (PA::W / 2) : ca / (PB::W / 2);
+      const int pr = of_a ? ca % (PA::W / 2) : ca % (PB::W / 2);
+      if (of_a)
+        split_pair(pa.v[set][it][2 * pr], pa.v[set][it][2 * pr + 1], h[pr], m[pr], l[pr]);
+      else
+        split_pair(pb.v[set][it][2 * pr], pb.v[set][it][2 * pr + 1], h[pr], m[pr], l[pr]);
+#pragma unroll
+      for (int q = q0; q < q1; ++q)
+        if (q < 5 * MM) {
+          const int pp = q / MM, i = (q % MM) / TN, j = q % TN;
+          acc[i][j] = mfma_bf16(fa[PA_OF[pp]][i], fb[PB_OF[pp]][j], acc[i][j]);
+        }
+      if (of_a && pr == PA::W / 2 - 1) {
+        pa.put(it, d, C::A_PLANE, h, m, l);
+        pa.load(set, it, adv);
+      }
+      if (!of_a && pr == PB::W / 2 - 1) {
+        pb.put(it, d + 3 * C::A_PLANE, C::B_PLANE, h, m, l);
+        pb.load(set, it, adv);
+      }
+      // Masks: 0x8 MFMA, 0x100 LDS read, 0x2 VALU.
+#pragma unroll
+      for (int q = 0; q < MPC; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, (13 + MPC - 1) / MPC, 0);
+      }
+      if (c < PAIRS - 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  constexpr int D = C::DEPTH;
+  static_assert(D == 1 || D == 2, "steps are unrolled by two");
+#define LMP_BF3_STEP(U) \
+  step(std::integral_constant<int, (U) % 2>{}, std::integral_constant<int, ((U) + 1) % D>{}, t)
+  for (int t = 0;;) {
+    LMP_BF3_STEP(0);
+    if (++t == steps) break;
+    LMP_BF3_STEP(1);
+    if (++t == steps) break;
+  }
+#undef LMP_BF3_STEP
+  mma(1, 1);
+  __syncthreads();
+
+  // Column sums: the parts of a column (its items' k ranges) in k order.
+  if constexpr (!TB) {
+    if (do_cs) {
+      float* sums = reinterpret_cast<float*>(smem);
+#pragma unroll
+      for (int i = 0; i < PB::ITEMS; ++i) sums[int(threadIdx.x) + i * C::THREADS] = pb.cs[i];
+      __syncthreads();
+      for (int c = threadIdx.x; c < C::BN; c += C::THREADS) {
+        float v = sums[c];
+#pragma unroll
+        for (int q = 1; q < PB::PER_ROW; ++q) v += sums[q * C::BN + c];
+        const int col = n0 + c;
+        if (col < g.n) {
+          if (partial)
+            args.part[split * args.part_stride + args.cs_at + col] = v;
+          else
+            g.colsum[col] = g.colsum_acc ? g.colsum[col] + v : v;
+        }
+      }
+      __syncthreads();
+    }
+  }
+
+  // Unscale; a value that is not finite sends the workgroup to the fallback.
+  uint32_t top = 0;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float v = acc[i][j][r];
+        top = max(top, __builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
+        acc[i][j][r] = v * kBf3Unscale;
+      }
+  if (top >= 0x7f800000u) *flag = 1;
+  __syncthreads();
+  if (*flag) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = v16f(0.0f);
+    for (int k = 0; k < k_len; k += 2) {
+      const bool in = k + lh < k_len;
+      const int64_t kk = k_begin + k + (in ? lh : 0);
+      float xa[TM], xb[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int64_t r = min(m0 + (wm * TM + i) * 32 + li, g.m - 1);
+        const float x = g.a[TA ? kk * g.lda + r : r * g.lda + kk];
+        xa[i] = in ? x : 0.0f;
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int64_t c = min(n0 + (wn * TN + j) * 32 + li, g.n - 1);
+        const float x = g.b[TB ? c * g.ldb + kk : kk * g.ldb + c];
+        xb[j] = in ? x : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma_f32(xa[i], xb[j], acc[i][j]);
+    }
+  }
+
+  float* out = partial ? args.part + split * args.part_stride : g.c;
+  const int64_t ld = partial ? g.n : g.ldc;
+  const float* bias = partial ? nullptr : g.bias;
+  const bool acc_out = !partial && g.accumulate;
+  if (g.vec_out) {
+    // Whole float4s of C's rows through a wave-private 32 x 36 LDS tile (LDS
+    // requests of one wave complete in order).  Every wave is past its reads of
+    // the stages (the flag's barrier).
+    float* w = reinterpret_cast<float*>(smem) + wave * (32 * 36);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          w[((r / 4) * 8 + lh * 4 + (r % 4)) * 36 + li] = acc[i][j][r];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const int row0 = m0 + (wm * TM + i) * 32, col0 = n0 + (wn * TN + j) * 32;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int at = lane + 64 * q, rr = at >> 3, cc = (at & 7) * 4;
+          const v4f v = *reinterpret_cast<const v4f*>(w + rr * 36 + cc);
+          const int row = row0 + rr, col = col0 + cc;
+          if (row < g.m && col < g.n) {
+            v4f* p = reinterpret_cast<v4f*>(out + row * ld + col);
+            if (acc_out) *p = *p + v;
+            else if (bias) *p = lin_epi4(v, *reinterpret_cast<const v4f*>(bias + col), g.relu);
+            else *p = v;
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int col = n0 + (wn * TN + j) * 32 + li;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = m0 + (wm * TM + i) * 32 + (r / 4) * 8 + lh * 4 + (r % 4);
+        if (row < g.m && col < g.n) {
+          float* p = out + row * ld + col;
+          const float v = acc[i][j][r];
+          if (acc_out) *p = *p + v;
+          else if (bias) *p = lin_epi(v, bias[col], g.relu);
+          else *p = v;
+        }
+      }
+    }
+}
+
+template <int NT, int MINB, class C, bool TA, bool TB>
+__global__ __launch_bounds__(NT, MINB) void gemm_bf3(Bf3Args args) {
+  static_assert(NT == C::THREADS, "one lane per thread of the configuration");
+  __shared__ __attribute__((aligned(1024))) char smem[C::SMEM];
+  gemm_bf3_tile<C, TA, TB>(args, int(blockIdx.x), smem);
+}
+
+// A Linear's weight gradient (`w`: A transposed) and input gradient (`x`: B
+// transposed) in one grid, the first product's workgroups first: the CUs it
+// frees start the second's first loads while its last stores drain, and the
+// bits are those of two launches.
+template <int NT, int MINB, class CW, class CX>
+__global__ __launch_bounds__(NT, MINB) void gemm_bf3_pair(Bf3Args w, Bf3Args x) {
+  static_assert(NT == CW::THREADS && NT == CX::THREADS, "one workgroup size for both");
+  __shared__ __attribute__((aligned(1024))) char smem[CW::SMEM > CX::SMEM ? CW::SMEM : CX::SMEM];
+  const int of_w = w.g.tiles_m * w.g.tiles_n * w.splits;
+  const int id = int(blockIdx.x);
+  if (id < of_w) gemm_bf3_tile<CW, true, false>(w, id, smem);
+  else gemm_bf3_tile<CX, false, true>(x, id - of_w, smem);
+}
+
+// C (and the column sums) from the partials of one product, or of two (`b`,
+// from workgroup `blocks_a` on), added in split order, with the epilogue of
+// the final output.  Four consecutive values per lane, counted through C as
+// one run of m * n: the loads are 128-bit whatever n is, and so are the stores
+// when C's rows are contiguous or all 16-byte aligned (g.vec_out).  The last
+// workgroups of a product add its column sums.
+struct Bf3Fold {
+  Bf3Args a;
+  int blocks_c, blocks;  // workgroups for C, and with the column sums
+};
+
+__device__ __forceinline__ void fold_bf3_block(const Bf3Args& a, int block, int blocks_c) {
+  const GemmArgs& g = a.g;
+  const bool is_cs = block >= blocks_c;
+  const int count = is_cs ? g.n : g.m * g.n;  // below 2^23: the partials are bounded
+  const int i = 4 * ((block - (is_cs ? blocks_c : 0)) * 256 + int(threadIdx.x));
+  if (i >= count) return;
+  const float* src = a.part + (is_cs ? a.cs_at : 0) + i;
+  v4f v = *reinterpret_cast<const v4f*>(src);
+  int s = 1;
+  for (; s + 4 <= a.splits; s += 4) {
+    v4f x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const v4f*>(src + (s + u) * a.part_stride);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v = v + x[u];
+  }
+  for (; s < a.splits; ++s) v = v + *reinterpret_cast<const v4f*>(src + s * a.part_stride);
+  if (is_cs) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (i + e < count) g.colsum[i + e] = g.colsum_acc ? g.colsum[i + e] + v[e] : v[e];
+    return;
+  }
+  int row = i / g.n, col = i - row * g.n;
+  if (g.vec_out) {
+    v4f* p = reinterpret_cast<v4f*>(g.c + int64_t(row) * g.ldc + col);
+    if (g.accumulate) *p = *p + v;
+    else *p = g.bias ? lin_epi4(v, *reinterpret_cast<const v4f*>(g.bias + col), g.relu) : v;
+    return;
+  }
+  if (g.ldc == g.n && !g.accumulate && i + 4 <= count) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (g.bias) v[e] = lin_epi(v[e], g.bias[col], g.relu);
+      if (++col == g.n) col = 0;
+    }
+    *reinterpret_cast<v4f_any*>(g.c + i) = v;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (i + e < count) {
+      float* p = g.c + int64_t(row) * g.ldc + col;
+      if (g.accumulate) *p = *p + v[e];
+      else *p = g.bias ? lin_epi(v[e], g.bias[col], g.relu) : v[e];
+    }
+    if (++col == g.n) {
+      col = 0;
+      ++row;
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void fold_bf3(Bf3Fold a, Bf3Fold b) {
+  const int block = int(blockIdx.x);
+  if (block < a.blocks) fold_bf3_block(a.a, block, a.blocks_c);
+  else fold_bf3_block(b.a, block - a.blocks, b.blocks_c);
+}
+
+// ------------------------------------------------------------------- host
+
+using Bf3Big = Bf3Cfg<2, 4, 4, 2, 1, 1>;     // 256 x 256, 8 waves of 128 x 64
+using Bf3Wide = Bf3Cfg<4, 2, 2, 2, 1, 1>;    // 256 x 128, 8 waves of 64 x 64
+using Bf3Mid = Bf3Cfg<4, 2, 1, 2, 2, 1>;     // 128 x 128, 8 waves of 32 x 64
+using Bf3Flat = Bf3Cfg<1, 4, 2, 1, 2, 2>;    // 64 x 128, 4 waves of 64 x 32
+using Bf3Small = Bf3Cfg<2, 2, 1, 1, 2, 2>;   // 64 x 64, 4 waves of 32 x 32
+
+struct Bf3Plan {
+  int cfg = 0;  // index into kBf3Tiles
+  int splits = 1;
+};
+
+// Time of one 16-wide k step of a workgroup, in us: `alone` on its CU, and
+// `shared` per workgroup where several take turns (medians of a sweep of 25
+// shapes, random operands, on one MI355X).  A larger tile moves and splits
+// each value fewer times: 4096^3 takes 574, 637, 700, 792 and about 980 us on
+// the five, 512 x 1000 x 4096 (K split) 44.0, 34.4, 34.4, 36.7, 39.4 and
+// 256 x 1024 x 1024 25.9, 19.8, 15.9, 14.5, 13.7.
+struct Bf3Tile {
+  int bm, bn;
+  float alone, shared;
+};
+constexpr Bf3Tile kBf3Tiles[] = {{256, 256, 2.2f, 2.2f},
+                                 {256, 128, 1.25f, 1.25f},
+                                 {128, 128, 0.69f, 0.68f},
+                                 {64, 128, 0.42f, 0.39f},
+                                 {64, 64, 0.34f, 0.235f}};
+
+// Tiles and split of K with the least modelled time: workgroups go round the
+// CUs, each takes 4.5 us besides its steps (first loads, C), and a split costs
+// a second launch (2 us) and a round trip of the partials (5 TB/s).  The
+// partials stay within the fixed workspace whichever entry point is called, so
+// that all of them give the same bits; a split keeps at least 64 k.
+Bf3Plan bf3_plan(Runtime* rt, const GemmArgs& g) {
+  const int64_t steps = (g.k + kBf3K - 1) / kBf3K, mn = int64_t(g.m) * g.n;
+  const int64_t most =
+      std::min<int64_t>(std::max<int64_t>(1, steps / 4),
+                        int64_t(LMP_NOALLOC_SCRATCH_BYTES) / int64_t(sizeof(float)) /
+                            (mn + g.n + 8));  // room for column sums, asked for or not
+  Bf3Plan plan;
+  float best = 0.0f;
+  for (int c = 0; c < 5; ++c) {
+    const Bf3Tile& t = kBf3Tiles[c];
+    const int64_t tiles = int64_t((g.m + t.bm - 1) / t.bm) * ((g.n + t.bn - 1) / t.bn);
+    for (int s : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+      if (s > 1 && s > most) break;
+      const float load = float((tiles * s + rt->cu_count - 1) / rt->cu_count);
+      const float per_step = std::max(t.alone, load * t.shared);
+      float us = 4.5f + float((steps + s - 1) / s) * per_step;
+      if (s > 1) us += 2.0f + float(s + 1) * float(mn) * (4.0f / 5e6f);
+      if (best == 0.0f || us < best) {
+        best = us;
+        plan.cfg = c;
+        plan.splits = s;
+      }
+      if (tiles * s > 8 * int64_t(rt->cu_count)) break;  // more splits only add partials
+    }
+  }
+  return plan;
+}
+
+// Calls f with the configuration's type.
+template <class F>
+int with_bf3_cfg(int cfg, F&& f) {
+  switch (cfg) {
+    case 0: return f(Bf3Big{});
+    case 1: return f(Bf3Wide{});
+    case 2: return f(Bf3Mid{});
+    case 3: return f(Bf3Flat{});
+    default: return f(Bf3Small{});
+  }
+}
+
+// The launch arguments of `g` under `plan`, without the partials' memory.
+Bf3Args bf3_args(const GemmArgs& g, const Bf3Plan& plan) {
+  Bf3Args a{};
+  a.g = g;
+  const Bf3Tile& t = kBf3Tiles[plan.cfg];
+  a.g.tiles_m = (g.m + t.bm - 1) / t.bm;
+  a.g.tiles_n = (g.n + t.bn - 1) / t.bn;
+  const int steps = (g.k + kBf3K - 1) / kBf3K;
+  a.steps_per_split = (steps + plan.splits - 1) / plan.splits;
+  a.splits = (steps + a.steps_per_split - 1) / a.steps_per_split;
+  a.cs_at = (int64_t(g.m) * g.n + 3) / 4 * 4;
+  a.part_stride = a.cs_at + (g.colsum ? (int64_t(g.n) + 3) / 4 * 4 : 0);
+  return a;
+}
+
+int bf3_take_partials(Bf3Args& a, const Workspace& ws) {
+  if (a.splits == 1) return LMP_OK;
+  return ws.take(size_t(a.splits) * size_t(a.part_stride) * sizeof(float), &a.part);
+}
+
+uint32_t bf3_workgroups(const Bf3Args& a) {
+  return uint32_t(int64_t(a.g.tiles_m) * a.g.tiles_n * a.splits);
+}
+
+// The fold of one or two products; those without a split take no workgroup.
+int launch_fold_bf3(Runtime* rt, const Bf3Args& a, const Bf3Args* b = nullptr) {
+  auto fold = [](const Bf3Args& x) {
+    Bf3Fold f{x, 0, 0};
+    if (x.splits > 1) {
+      f.blocks_c = int((int64_t(x.g.m) * x.g.n + 1023) / 1024);
+      f.blocks = f.blocks_c + (x.g.colsum ? (x.g.n + 1023) / 1024 : 0);
+    }
+    return f;
+  };
+  const Bf3Fold fa = fold(a), fb = b ? fold(*b) : Bf3Fold{};
+  if (fa.blocks + fb.blocks == 0) return LMP_OK;
+  hipLaunchKernelGGL(fold_bf3, dim3(uint32_t(fa.blocks + fb.blocks)), dim3(256), 0, rt->stream,
+                     fa, fb);
+  LMP_LAUNCH_CHECK("fold_bf3");
+  return LMP_OK;
+}
+
+template <bool TA, bool TB>
+int launch_bf3_as(Runtime* rt, GemmArgs g, const Bf3Plan& plan, const Workspace& ws) {
+  Bf3Args a = bf3_args(g, plan);
+  if (const int rc = bf3_take_partials(a, ws); rc != LMP_OK) return rc;
+  const int rc = with_bf3_cfg(plan.cfg, [&](auto cfg) {
+    using C = decltype(cfg);
+    hipLaunchKernelGGL((gemm_bf3<C::THREADS, C::MINB, C, TA, TB>), dim3(bf3_workgroups(a)),
+                       dim3(C::THREADS), 0, rt->stream, a);
+    LMP_LAUNCH_CHECK("gemm_bf3");
+    return launch_fold_bf3(rt, a);
+  });
+  if (a.part) ws.give(a.part);  // stream-ordered: the fold reads it first
+  return rc;
+}
+
+template <bool TA, bool TB>
+int launch_bf3_planned(Runtime* rt, GemmArgs g, const Workspace& ws, bool* colsum_done) {
+  if (TB) g.colsum = nullptr;  // the sums ride where B's rows run along n
+  if (g.colsum && colsum_done) *colsum_done = true;
+  return launch_bf3_as<TA, TB>(rt, g, bf3_plan(rt, g), ws);
+}
+
+// A weight gradient (A transposed, with its column sums) and an input gradient
+// (B transposed) as one launch and, where either is split, one fold; false,
+// with nothing launched, if their workgroups differ in size.
+bool launch_bf3_pair_planned(Runtime* rt, const GemmArgs& gw, const GemmArgs& gx, int* rc) {
+  const Bf3Plan pw = bf3_plan(rt, gw), px = bf3_plan(rt, gx);
+  if ((pw.cfg <= 2) != (px.cfg <= 2)) return false;
+  Bf3Args w = bf3_args(gw, pw), x = bf3_args(gx, px);
+  const Workspace ws{};
+  if ((*rc = bf3_take_partials(w, ws)) != LMP_OK) return true;
+  if ((*rc = bf3_take_partials(x, ws)) != LMP_OK) {
+    if (w.part) ws.give(w.part);
+    return true;
+  }
+  *rc = with_bf3_cfg(pw.cfg, [&](auto cw) {
+    return with_bf3_cfg(px.cfg, [&](auto cx) {
+      using CW = decltype(cw);
+      using CX = decltype(cx);
+      if constexpr (CW::THREADS == CX::THREADS) {
+        constexpr int kMinB = CW::MINB < CX::MINB ? CW::MINB : CX::MINB;
+        hipLaunchKernelGGL((gemm_bf3_pair<CW::THREADS, kMinB, CW, CX>),
+                           dim3(bf3_workgroups(w) + bf3_workgroups(x)), dim3(CW::THREADS), 0,
+                           rt->stream, w, x);
+        LMP_LAUNCH_CHECK("gemm_bf3_pair");
+        return launch_fold_bf3(rt, w, &x);
+      } else {
+        return fail(LMP_ERR_RUNTIME, "linear_backward: workgroup sizes differ");
+      }
+    });
+  });
+  if (w.part) ws.give(w.part);  // stream-ordered: the fold reads them first
+  if (x.part) ws.give(x.part);
+  return true;
+}
+
+}  // namespace
+}  // namespace lmp_hip

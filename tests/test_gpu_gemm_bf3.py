@@ -1,0 +1,147 @@
+"""The fp32 GEMM that runs on the bf16 matrix cores, each operand in three
+parts (K > 32 and M > 32, with an operand transposed or M > 512), through the C
+ABI: tile edges, K remainders, splits of K, unaligned rows, the whole range of
+fp32, and values that are not finite."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24  # half an ulp of fp32, relative
+
+
+def _run(hip, A, B, ta, tb, pad=(0, 0), c0=None, acc=0, colsum=False):
+    """C = op(A) op(B) with `pad` extra values in each stored row (poisoned)
+    and C's rows; the column sums of op(B) beside it when asked for."""
+    m, k = A.shape[::-1] if ta else A.shape
+    n = B.shape[0] if tb else B.shape[1]
+    bufs = []
+    for x, p in ((A, pad[0]), (B, pad[1])):
+        y = np.full((x.shape[0], x.shape[1] + p), np.nan, np.float32)
+        y[:, :x.shape[1]] = x
+        bufs.append((hip.DeviceBuffer.from_numpy(y), y.shape[1]))
+    ldc = n + pad[1]
+    c = np.full((m, ldc), 7.0, np.float32)
+    if c0 is not None:
+        c[:, :n] = c0
+    dc = hip.DeviceBuffer.from_numpy(c)
+    (da, lda), (db, ldb) = bufs
+    if colsum:
+        cs = hip.DeviceBuffer.from_numpy(np.full(n, 3.0, np.float32))
+        hip.check(hip.lib().lmp_k_gemm_colsum_f32(ta, tb, m, n, k, da.ptr, lda, db.ptr, ldb,
+                                                  dc.ptr, ldc, acc, cs.ptr, 0))
+        got = dc.numpy()
+        assert np.all(got[:, n:] == 7.0)
+        return got[:, :n], cs.numpy()
+    hip.check(hip.lib().lmp_k_gemm_f32(ta, tb, m, n, k, da.ptr, lda, db.ptr, ldb, dc.ptr, ldc, acc))
+    got = dc.numpy()
+    assert np.all(got[:, n:] == 7.0)  # nothing outside C
+    return got[:, :n]
+
+
+def _operands(m, n, k, ta, tb, seed):
+    rng = np.random.default_rng(seed)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    b = rng.standard_normal((k, n), dtype=np.float32)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    return (np.ascontiguousarray(a.T) if ta else a), (np.ascontiguousarray(b.T) if tb else b), a64, b64
+
+
+# Tile edges of the five tile sizes, K around one, two and three steps of 16
+# and around the ends of K splits; the last five take the 256 x 256, 256 x 128,
+# 128 x 128, 64 x 128 and 64 x 64 tiles.
+SHAPES = [(33, 1, 33), (64, 65, 47), (65, 64, 48), (129, 127, 49), (257, 255, 63), (255, 130, 64),
+          (40, 1000, 1003), (200, 200, 2049), (4096, 4000, 49), (512, 2050, 2083), (1000, 1027, 1531),
+          (64, 2048, 1030), (300, 700, 260)]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES, ids=str)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_against_float64(hip, m, n, k, ta, tb):
+    """Rounding errors only: a step of 16 k adds six bf16 products, each with
+    at most two roundings of half an ulp of the running sum, independent of
+    each other, so the 2-norm of the error is below sqrt(12 ceil(K / 16))
+    half-ulps of the result's (a missing part of a split, 2^-17 of a term, is
+    over it).  Aligned and odd row pitches give the same bits."""
+    if not ta and not tb:
+        m += 512  # up to 512 rows X * W stays on the fp32 MFMAs
+    A, B, a64, b64 = _operands(m, n, k, ta, tb, m * 31 + n * 7 + k)
+    want = a64 @ b64
+    got = _run(hip, A, B, ta, tb)
+    steps = -(-k // 16)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert err <= np.sqrt(12 * steps + 2) * U, err
+    # every element, against the terms' magnitudes
+    assert np.all(np.abs(got - want) <= (12 * steps + 70) * U * (np.abs(a64) @ np.abs(b64)))
+    padded = _run(hip, A, B, ta, tb, pad=(1, 3))
+    assert np.array_equal(padded.view(np.uint32), got.view(np.uint32))
+    c0 = np.random.default_rng(1).standard_normal((m, n), dtype=np.float32)
+    acc = _run(hip, A, B, ta, tb, pad=(3, 1), c0=c0, acc=1)
+    assert np.array_equal(acc.view(np.uint32), (c0 + got).view(np.uint32))
+
+
+@pytest.mark.parametrize("m,n,k", [(129, 127, 49), (1000, 1027, 1531), (200, 200, 2049), (300, 700, 260)],
+                         ids=str)
+def test_column_sums(hip, m, n, k):
+    """The column sums beside the product (whole and split K, odd pitches):
+    within K half-ulps of the terms' magnitudes, the product unchanged."""
+    A, B, a64, b64 = _operands(m, n, k, 1, 0, 11)
+    for pad in ((0, 0), (1, 3)):
+        got, cs = _run(hip, A, B, 1, 0, pad=pad, colsum=True)
+        assert np.array_equal(got.view(np.uint32), _run(hip, A, B, 1, 0).view(np.uint32))
+        assert np.all(np.abs(cs - b64.sum(0)) <= k * U * np.abs(b64).sum(0))
+
+
+@pytest.mark.parametrize("m,k", [(64, 64), (200, 96), (300, 256)], ids=str)
+@pytest.mark.parametrize("ta,tb", [(0, 1), (1, 1), (1, 0)])
+def test_every_finite_value_survives(hip, m, k, ta, tb):
+    """Random bit patterns of finite fp32 values, subnormals and the largest
+    included, times the identity (its own transpose): each row exactly, through
+    either operand."""
+    rng = np.random.default_rng(m + k)
+    bits = rng.integers(0, 1 << 32, (m, k), dtype=np.uint64).astype(np.uint32)
+    bits[(bits & 0x7f800000) == 0x7f800000] ^= 0x00800000  # no infinity, no NaN
+    bits[::3] &= np.uint32(0x807fffff)                      # whole rows of subnormals
+    x = bits.view(np.float32)
+    x = np.where(x == 0, np.float32(1e-45), x)
+    eye = np.eye(k, dtype=np.float32)
+    got = _run(hip, np.ascontiguousarray(x.T) if ta else x, eye, ta, tb)
+    assert np.array_equal(got.view(np.uint32), x.view(np.uint32))
+    y = np.ascontiguousarray(x.T)  # [k, m]
+    got = _run(hip, eye, np.ascontiguousarray(y.T) if tb else y, ta, tb)
+    assert np.array_equal(got.view(np.uint32), y.view(np.uint32))
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 70, 40), (300, 270, 200), (200, 200, 2049)], ids=str)
+@pytest.mark.parametrize("kind", ["inf", "nan", "large", "overflow"])
+def test_values_that_are_not_finite(hip, m, n, k, kind):
+    """One infinity, NaN, row near the top of the range, or row whose results
+    overflow, alone in its tile: C is as float64 has it (rounded to fp32)."""
+    A, B, _, _ = _operands(m, n, k, 0, 0, 5)
+    row = m - 3
+    if kind == "inf":
+        A[row, 1] = np.inf
+    elif kind == "nan":
+        A[row, 1] = np.nan
+    elif kind == "large":
+        A[row] *= np.float32(1e33)
+    else:
+        A[row] = (np.abs(A[row]) + 1) * np.float32(1e37)
+        B[:, 2] = np.abs(B[:, 2]) + 1
+    with np.errstate(all="ignore"):
+        want = A.astype(np.float64) @ B.astype(np.float64)
+        want32 = want.astype(np.float32)
+    got = _run(hip, np.ascontiguousarray(A.T), B, 1, 0)
+    if kind == "overflow":  # the other columns' terms overflow one by one, with either sign
+        keep = np.ones((m, n), bool)
+        keep[row] = False
+        keep[row, 2] = True
+    else:
+        keep = np.ones((m, n), bool)
+    assert np.array_equal(np.isnan(got)[keep], np.isnan(want32)[keep])
+    inf = np.isinf(want32) & keep
+    assert np.array_equal(got[inf], want32[inf])
+    fin = np.isfinite(want32) & keep
+    scale = np.abs(np.where(np.isfinite(A), A, 0)).astype(np.float64) @ np.abs(B).astype(np.float64)
+    # the fallback's fp32 products round once per value of k
+    assert np.all(np.abs(got[fin] - want[fin]) <= (2 * k + 70) * U * scale[fin])
