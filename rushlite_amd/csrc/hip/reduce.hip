@@ -9,21 +9,26 @@
 //                      a row is split over several workgroups only when
 //                      there are too few rows to fill 256 CUs, and the
 //                      partials are folded by a second pass in fixed order.
+//   other long rows -> (odd lengths, other types) the same with units of
+//                      one value, or of 16 bytes where the type, length and
+//                      alignment allow.
 //   short rows      -> one wave per row (softmax/loss rows like [512,1000]),
 //                      float4 loads when rows are 16-byte multiples, four
-//                      loads in flight per lane.
+//                      loads in flight per lane; rows of at most 32 units
+//                      share a wave, 8 to 32 lanes each.
 // Column case (inner > 1, e.g. sum over dim 0, the bias-gradient reduction):
-//   each lane owns four adjacent columns (one float4); the four waves of a
-//   workgroup share a 256-column strip and take every fourth row of a chunk
-//   of the reduced axis (8 loads in flight per lane), then combine in LDS in
-//   fixed wave order.  The axis is cut into S chunks so the grid holds about
-//   four workgroups per CU; chunk partials [outer, S, inner] are folded by a
-//   second pass, S float4 loads per lane issued together.  An axis of at
-//   most 4096 rows that would need chunks (bias gradients: [batch, out] with
-//   a batch of a few hundred) is reduced in one pass instead: a workgroup
-//   owns a narrow strip of float4 columns and every row, its lanes split into
-//   row groups that combine in LDS, so there is no second launch.  No
-//   atomics: results are deterministic.
+//   units of 16 bytes along the columns where the type, inner extent and
+//   alignment allow, one value otherwise.  A workgroup owns a strip of up to
+//   64 units of one outer slice (the strips of a slice evenly wide) and a chunk
+//   of the reduced axis; its 256 lanes are row groups that take every rg-th row
+//   (8 loads in flight per lane) and combine in LDS by halving in fixed order.
+//   The axis is cut into S chunks so the grid holds about four workgroups per
+//   CU; the same kernel folds the chunk partials [outer, S, inner].  A short
+//   axis that would need chunks (bias gradients: [batch, out] with a batch of a
+//   few hundred) takes narrower strips instead, down to 64 bytes, so there is
+//   no second launch.
+//   Slices of at most 128 units take a lane per output.  No atomics: results
+//   are deterministic.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -74,6 +79,34 @@ template <bool NT>
 __device__ __forceinline__ v4f load4(const v4f* p) {
   if constexpr (NT) return __builtin_nontemporal_load(p);
   else return *p;
+}
+
+// V consecutive values, loaded and stored at once.
+template <typename T, int V>
+struct alignas(sizeof(T) * V) Pack {
+  T x[V];
+};
+template <int OP, typename T, int V>
+__device__ __forceinline__ Pack<T, V> combine_pack(Pack<T, V> a, const Pack<T, V>& b) {
+#pragma unroll
+  for (int i = 0; i < V; ++i) a.x[i] = Reducer<OP, T>::combine(a.x[i], b.x[i]);
+  return a;
+}
+template <int OP, typename T, int V>
+__device__ __forceinline__ Pack<T, V> identity_pack() {
+  Pack<T, V> p;
+#pragma unroll
+  for (int i = 0; i < V; ++i) p.x[i] = Reducer<OP, T>::identity();
+  return p;
+}
+template <bool NT, typename T, int V>
+__device__ __forceinline__ Pack<T, V> load_pack(const Pack<T, V>* p) {
+  if constexpr (NT) {
+    const v4f v = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p));
+    return __builtin_bit_cast(Pack<T, V>, v);
+  } else {
+    return *p;
+  }
 }
 
 // Block (row, part) reduces float4 [part*seg4, min(len4, (part+1)*seg4)) of
@@ -192,6 +225,75 @@ __global__ __launch_bounds__(kBlock) void row_reduce_wave_f32(
   if (lane == 0) out[row] = v;
 }
 
+// Long rows of any type: row_reduce_f32 with units of V values (len, a multiple
+// of V, counted in units).  [2048, 10001] fp32 (one wave a row before) 23.5 ->
+// 15.3 us, 5.35 TB/s.
+template <int OP, typename T, int V>
+__global__ __launch_bounds__(kBlock) void row_reduce_block(T* __restrict__ out,
+                                                           const T* __restrict__ in, uint32_t units,
+                                                           uint32_t seg, FastDiv parts) {
+  using R = Reducer<OP, T>;
+  using P = Pack<T, V>;
+  const uint32_t row = parts.div(blockIdx.x);
+  const uint32_t part = blockIdx.x - row * parts.d;
+  const P* src = reinterpret_cast<const P*>(in) + uint64_t(row) * units;
+  const uint32_t end = min(units, (part + 1) * seg);
+  P acc[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) acc[u] = identity_pack<OP, T, V>();
+  uint32_t i = part * seg + threadIdx.x;
+  for (; i + 3 * kBlock < end; i += 4 * kBlock) {
+    P x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = src[i + u * kBlock];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc[u] = combine_pack<OP>(acc[u], x[u]);
+  }
+  for (; i < end; i += kBlock) acc[0] = combine_pack<OP>(acc[0], src[i]);
+  P a = combine_pack<OP>(combine_pack<OP>(acc[0], acc[1]), combine_pack<OP>(acc[2], acc[3]));
+#pragma unroll
+  for (int w = 1; w < V; w *= 2)
+#pragma unroll
+    for (int j = 0; j + w < V; j += 2 * w) a.x[j] = R::combine(a.x[j], a.x[j + w]);
+  const T v = wave_reduce<OP, T>(a.x[0]);
+  __shared__ T lds[kWaves];
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    T r = lds[0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) r = R::combine(r, lds[w]);
+    out[blockIdx.x] = r;
+  }
+}
+
+// Rows of at most 32 units, G = 8, 16 or 32 lanes each (64 / G rows per wave):
+// a lane holds at most one unit, so the butterfly's first steps, which stay
+// inside the G lanes, give the bits of the one-wave kernels (whose other lanes
+// hold the identity).  [65536, 8] fp32: 8.3 -> 3.7 us.
+template <int OP, typename T, int V, int G>
+__global__ __launch_bounds__(kBlock) void row_reduce_small(T* __restrict__ out,
+                                                           const T* __restrict__ in, uint64_t rows,
+                                                           uint32_t units) {
+  using R = Reducer<OP, T>;
+  const uint64_t row = (uint64_t(blockIdx.x) * kBlock + threadIdx.x) / G;
+  const uint32_t lane = threadIdx.x % G;
+  Pack<T, V> a = identity_pack<OP, T, V>();
+  if (row < rows && lane < units)
+    a = combine_pack<OP>(a, reinterpret_cast<const Pack<T, V>*>(in)[row * units + lane]);
+#pragma unroll
+  for (int w = 1; w < V; w *= 2)
+#pragma unroll
+    for (int j = 0; j + w < V; j += 2 * w) a.x[j] = R::combine(a.x[j], a.x[j + w]);
+  T v = a.x[0];
+  v = R::combine(v, lmp_swap<1>(v));
+  v = R::combine(v, lmp_swap<2>(v));
+  v = R::combine(v, lmp_swap<4>(v));
+  if constexpr (G > 8) v = R::combine(v, lmp_swap<8>(v));
+  if constexpr (G > 16) v = R::combine(v, lmp_swap<16>(v));
+  if (lane == 0 && row < rows) out[row] = v;
+}
+
 // Fold `parts` consecutive partials per output in order.
 template <int OP, typename T>
 __global__ __launch_bounds__(kBlock) void fold_parts(T* __restrict__ out,
@@ -206,146 +308,98 @@ __global__ __launch_bounds__(kBlock) void fold_parts(T* __restrict__ out,
   out[i] = acc;
 }
 
-// Column reduction, fp32.  grid = (ceil(inner4/64), S, outer); lane owns
-// float4 column c4 = blockIdx.x*64 + lane, wave w takes rows r0+w, r0+w+4, ...
-// of chunk s = [s*chunk, min(len, (s+1)*chunk)).  dst layout [outer, S, inner]
-// (S == 1 writes the final result).
+// Column reduction, V values per unit.  Workgroup (o, s, b) owns units
+// [b * cw, b * cw + cw) of slice o and rows [s * chunk, s * chunk + chunk);
+// lane t takes unit t % cw and, of rg = 256 / cw row groups, rows t / cw +
+// rg * i, eight loads in flight.  dst layout [outer, S, units] (S == 1 writes
+// the final result).  HBM-bound: sum over the middle axis of [256, 197, 768]
+// 51.6 -> 28.8 us (5.4 TB/s; fp32 strips were sized without the outer extent:
+// 64-byte rows), over dim 0 of [16384, 16384] 160 -> 157 us (6.8 TB/s), float64
+// 352 -> 317 us and int32 184 -> 164 us (units of one value before), of
+// [200000, 64] fp32 59 -> 14 us, float64 272 -> 21 us (the partials folded by one
+// lane per column), [16384, 3] 27.6 -> 6.5 us (three lanes of 256).
 constexpr int kColUnroll = 8;
-template <int OP, bool NT>
-__global__ __launch_bounds__(kBlock) void col_reduce_f32(
-    float* __restrict__ dst, const float* __restrict__ in, uint32_t inner4,
-    uint32_t len, uint32_t chunk) {
-  using R = Reducer<OP, float>;
-  const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint32_t c4 = blockIdx.x * 64 + lane;
-  const uint32_t s = blockIdx.y, S = gridDim.y, o = blockIdx.z;
-  const uint32_t r0 = s * chunk;
-  const uint32_t r1 = min(len, r0 + chunk);
-  const v4f id = v4f(R::identity());
-  v4f acc[kColUnroll];
+template <int OP, typename T, int V, bool NT>
+__global__ __launch_bounds__(kBlock) void col_reduce_tile(T* __restrict__ dst,
+                                                          const T* __restrict__ in, uint32_t units,
+                                                          uint32_t len, uint32_t chunk, FastDiv cw,
+                                                          FastDiv strips, FastDiv S) {
+  using P = Pack<T, V>;
+  const uint32_t q = strips.div(blockIdx.x), b = blockIdx.x - q * strips.d;
+  const uint32_t o = S.div(q), s = q - o * S.d;
+  const uint32_t g = cw.div(threadIdx.x), col = threadIdx.x - g * cw.d;
+  const uint32_t rg = cw.div(uint32_t(kBlock)), c = b * cw.d + col;
+  const uint32_t r1 = min(len, (s + 1) * chunk);
+  P acc[kColUnroll];
 #pragma unroll
-  for (int u = 0; u < kColUnroll; ++u) acc[u] = id;
-  if (c4 < inner4) {
-    const v4f* src = reinterpret_cast<const v4f*>(in) + uint64_t(o) * len * inner4 + c4;
-    uint32_t r = r0 + w;
-    for (; r + 4 * (kColUnroll - 1) < r1; r += 4 * kColUnroll) {
-      v4f x[kColUnroll];
+  for (int u = 0; u < kColUnroll; ++u) acc[u] = identity_pack<OP, T, V>();
+  if (c < units && g < rg) {
+    const P* src = reinterpret_cast<const P*>(in) + uint64_t(o) * len * units + c;
+    uint32_t r = s * chunk + g;
+    for (; r + rg * (kColUnroll - 1) < r1; r += rg * kColUnroll) {
+      P x[kColUnroll];
 #pragma unroll
-      for (int u = 0; u < kColUnroll; ++u) x[u] = load4<NT>(src + uint64_t(r + 4 * u) * inner4);
+      for (int u = 0; u < kColUnroll; ++u) x[u] = load_pack<NT>(src + uint64_t(r + rg * u) * units);
 #pragma unroll
-      for (int u = 0; u < kColUnroll; ++u) acc[u] = combine4<OP>(acc[u], x[u]);
+      for (int u = 0; u < kColUnroll; ++u) acc[u] = combine_pack<OP>(acc[u], x[u]);
     }
-    for (; r < r1; r += 4) acc[0] = combine4<OP>(acc[0], load4<NT>(src + uint64_t(r) * inner4));
-  }
-  v4f a = acc[0];
+    if (r < r1) {  // at most seven rows remain: their loads go out together too
+      P x[kColUnroll - 1];
 #pragma unroll
-  for (int u = 1; u < kColUnroll; ++u) a = combine4<OP>(a, acc[u]);
-  __shared__ v4f lds[kWaves][64];
-  lds[w][lane] = a;
-  __syncthreads();
-  if (w == 0 && c4 < inner4) {
-    v4f t = lds[0][lane];
+      for (int u = 0; u < kColUnroll - 1; ++u) {
+        x[u] = identity_pack<OP, T, V>();
+        if (r + rg * u < r1) x[u] = load_pack<NT>(src + uint64_t(r + rg * u) * units);
+      }
 #pragma unroll
-    for (int k = 1; k < kWaves; ++k) t = combine4<OP>(t, lds[k][lane]);
-    reinterpret_cast<v4f*>(dst)[(uint64_t(o) * S + s) * inner4 + c4] = t;
-  }
-}
-
-// Column reduction in one pass for a short axis.  grid = (ceil(inner4/cw),
-// 1, outer), cw = 1 << cw_log2 float4 columns per workgroup; the 256/cw row
-// groups take rows g, g + 256/cw, ... (eight loads in flight per lane), then
-// fold in LDS by halving in fixed order.  out layout [outer, inner4].
-constexpr uint32_t kStripMaxLen = 4096;
-template <int OP>
-__global__ __launch_bounds__(kBlock) void col_reduce_strip_f32(
-    float* __restrict__ out, const float* __restrict__ in, uint32_t inner4, uint32_t len,
-    uint32_t cw_log2) {
-  using R = Reducer<OP, float>;
-  const uint32_t t = threadIdx.x;
-  const uint32_t cw = 1u << cw_log2, rg = uint32_t(kBlock) >> cw_log2;
-  const uint32_t col = t & (cw - 1), g = t >> cw_log2;
-  const uint32_t c4 = blockIdx.x * cw + col;
-  const uint32_t o = blockIdx.z;
-  const v4f id = v4f(R::identity());
-  v4f acc[kColUnroll];
-#pragma unroll
-  for (int u = 0; u < kColUnroll; ++u) acc[u] = id;
-  if (c4 < inner4) {
-    const v4f* src = reinterpret_cast<const v4f*>(in) + uint64_t(o) * len * inner4 + c4;
-    uint32_t r = g;
-    for (; r + rg * (kColUnroll - 1) < len; r += rg * kColUnroll) {
-      v4f x[kColUnroll];
-#pragma unroll
-      for (int u = 0; u < kColUnroll; ++u) x[u] = src[uint64_t(r + rg * u) * inner4];
-#pragma unroll
-      for (int u = 0; u < kColUnroll; ++u) acc[u] = combine4<OP>(acc[u], x[u]);
+      for (int u = 0; u < kColUnroll - 1; ++u) acc[u] = combine_pack<OP>(acc[u], x[u]);
     }
-    for (; r < len; r += rg) acc[0] = combine4<OP>(acc[0], src[uint64_t(r) * inner4]);
   }
-  v4f a = acc[0];
+  P a = acc[0];
 #pragma unroll
-  for (int u = 1; u < kColUnroll; ++u) a = combine4<OP>(a, acc[u]);
-  __shared__ v4f lds[kBlock];
-  lds[t] = a;  // row group g, column col
-  for (uint32_t half = rg >> 1; half >= 1; half >>= 1) {
+  for (int u = 1; u < kColUnroll; ++u) a = combine_pack<OP>(a, acc[u]);
+  __shared__ P lds[kBlock];
+  lds[threadIdx.x] = a;
+  for (uint32_t n = rg; n > 1;) {
+    const uint32_t half = (n + 1) / 2;
     __syncthreads();
-    if (g < half) {
-      a = combine4<OP>(a, lds[t + half * cw]);
-      lds[t] = a;
+    if (g < n - half) {
+      a = combine_pack<OP>(a, lds[threadIdx.x + half * cw.d]);
+      lds[threadIdx.x] = a;
     }
+    n = half;
   }
-  if (g == 0 && c4 < inner4) reinterpret_cast<v4f*>(out)[uint64_t(o) * inner4 + c4] = a;
+  if (g == 0 && c < units)
+    reinterpret_cast<P*>(dst)[(uint64_t(o) * S.d + s) * units + c] = a;
 }
 
-// Fold S chunk partials [outer, S, inner4] -> [outer, inner4], float4 lanes,
-// in chunk order with the loads of eight chunks issued before their combines.
-template <int OP>
-__global__ __launch_bounds__(kBlock) void fold_chunks_f32(
-    float* __restrict__ out, const float* __restrict__ part, uint64_t outer,
-    uint32_t inner4, uint32_t S) {
-  using R = Reducer<OP, float>;
+// One lane per output unit of [outer, units]: short slices, or an axis whose
+// outputs alone fill the chip.  Eight accumulators as above.
+template <int OP, typename T, int V>
+__global__ __launch_bounds__(kBlock) void col_reduce_lane(T* __restrict__ out,
+                                                          const T* __restrict__ in, uint64_t n,
+                                                          uint32_t units, uint32_t len) {
+  using P = Pack<T, V>;
   const uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= outer * inner4) return;
-  const uint64_t o = i / inner4, c = i - o * inner4;
-  const v4f* src = reinterpret_cast<const v4f*>(part) + o * S * inner4 + c;
-  v4f acc = v4f(R::identity());
-  uint32_t s = 0;
-  for (; s + 8 <= S; s += 8) {
-    v4f x[8];
+  if (i >= n) return;
+  const uint64_t o = i / units, c = i - o * units;
+  const P* src = reinterpret_cast<const P*>(in) + o * len * units + c;
+  P acc[kColUnroll];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = src[uint64_t(s + u) * inner4];
+  for (int u = 0; u < kColUnroll; ++u) acc[u] = identity_pack<OP, T, V>();
+  uint32_t r = 0;
+  for (; r + kColUnroll <= len; r += kColUnroll) {
+    P x[kColUnroll];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) acc = combine4<OP>(acc, x[u]);
+    for (int u = 0; u < kColUnroll; ++u) x[u] = src[uint64_t(r + u) * units];
+#pragma unroll
+    for (int u = 0; u < kColUnroll; ++u) acc[u] = combine_pack<OP>(acc[u], x[u]);
   }
-  for (; s < S; ++s) acc = combine4<OP>(acc, src[uint64_t(s) * inner4]);
-  reinterpret_cast<v4f*>(out)[i] = acc;
-}
-
-// Column reduction for any dtype / alignment: one lane per column.
-template <int OP, typename T>
-__global__ __launch_bounds__(kBlock) void col_reduce_scalar(
-    T* __restrict__ dst, const T* __restrict__ in, uint64_t inner,
-    uint64_t len, uint64_t chunk) {
-  using R = Reducer<OP, T>;
-  const uint64_t c = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (c >= inner) return;
-  const uint64_t s = blockIdx.y, S = gridDim.y, o = blockIdx.z;
-  const uint64_t r0 = s * chunk;
-  const uint64_t r1 = min(len, r0 + chunk);
-  const T* src = in + (o * len + r0) * inner + c;
-  // Eight loads in flight, combined in row order (the result is the
-  // sequential fold, as without the batching).
-  T acc = R::identity();
-  uint64_t r = r0;
-  for (; r + 8 <= r1; r += 8, src += 8 * inner) {
-    T x[8];
+  for (; r < len; ++r) acc[0] = combine_pack<OP>(acc[0], src[uint64_t(r) * units]);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = src[u * inner];
+  for (int w = kColUnroll / 2; w >= 1; w /= 2)
 #pragma unroll
-    for (int u = 0; u < 8; ++u) acc = R::combine(acc, x[u]);
-  }
-  for (; r < r1; ++r, src += inner) acc = R::combine(acc, *src);
-  dst[(o * S + s) * inner + c] = acc;
+    for (int u = 0; u < w; ++u) acc[u] = combine_pack<OP>(acc[u], acc[u + w]);
+  reinterpret_cast<P*>(out)[i] = acc[0];
 }
 
 // Column reduction with one lane per output element (o, c) of [outer, inner],
@@ -378,26 +432,11 @@ __global__ __launch_bounds__(kBlock) void col_reduce_flat(T* __restrict__ out,
   }
 }
 
-// Fold S chunk partials [outer, S, inner] -> [outer, inner] in chunk order.
-template <int OP, typename T>
-__global__ __launch_bounds__(kBlock) void fold_chunks(T* __restrict__ out,
-                                                      const T* __restrict__ part,
-                                                      uint64_t outer,
-                                                      uint64_t inner,
-                                                      uint32_t S) {
-  using R = Reducer<OP, T>;
-  const uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= outer * inner) return;
-  const uint64_t o = i / inner, c = i - o * inner;
-  const T* src = part + o * S * inner + c;
-  T acc = R::identity();
-  for (uint32_t s = 0; s < S; ++s) acc = R::combine(acc, src[uint64_t(s) * inner]);
-  out[i] = acc;
-}
-
 bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
+
+constexpr uint64_t kStripMaxLen = 4096;
 
 uint32_t blocks_for(uint64_t n) { return uint32_t((n + kBlock - 1) / kBlock); }
 
@@ -407,47 +446,91 @@ uint32_t blocks_for(uint64_t n) { return uint32_t((n + kBlock - 1) / kBlock); }
 // (columns) or more take the 64-bit kernels instead.
 constexpr uint64_t kMaxU32Extent = 0x7fffffffull;
 
+// Units of 16 bytes where the type, the contiguous extent and the address
+// allow, else of one value.
+template <typename T>
+constexpr int kPackOf = sizeof(T) >= 2 ? int(16 / sizeof(T)) : 1;
+template <typename T>
+bool packs(const void* p, uint64_t extent) {
+  return kPackOf<T> > 1 && extent % kPackOf<T> == 0 && aligned16(p);
+}
+
+// Workgroups per row of a long row: enough to fill the chip twice over, more
+// than one only when the rows alone cannot.
+uint64_t row_parts(Runtime* rt, uint64_t rows, uint64_t units) {
+  const uint64_t target = uint64_t(rt->cu_count) * 8;
+  if (rows >= target) return 1;
+  return std::min<uint64_t>((target + rows - 1) / rows, std::max<uint64_t>(1, units / 1024));
+}
+
+template <int OP, typename T, int V, int G>
+int launch_small_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t units) {
+  hipLaunchKernelGGL((row_reduce_small<OP, T, V, G>), dim3(blocks_for(rows * G)), dim3(kBlock), 0,
+                     rt->stream, out, in, rows, uint32_t(units));
+  LMP_LAUNCH_CHECK("row_reduce_small");
+  return LMP_OK;
+}
+
+// Rows of V-value units: short ones several to a wave, long ones a workgroup
+// (or several) each; *done false where neither applies.
+template <int OP, typename T, int V>
+int reduce_rows_as(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len, bool* done) {
+  const uint64_t units = len / V;
+  *done = true;
+  if (units <= 32 && rows <= 0x7fffffffull) {
+    if (units <= 8) return launch_small_rows<OP, T, V, 8>(rt, out, in, rows, units);
+    if (units <= 16) return launch_small_rows<OP, T, V, 16>(rt, out, in, rows, units);
+    return launch_small_rows<OP, T, V, 32>(rt, out, in, rows, units);
+  }
+  if (len >= 2048 && units <= kMaxU32Extent) {
+    uint64_t parts = row_parts(rt, rows, units);
+    const uint64_t seg = (units + parts - 1) / parts;
+    parts = (units + seg - 1) / seg;
+    if (rows * parts > 0x7fffffffull) return fail(LMP_ERR_UNSUPPORTED, "reduce: too many rows");
+    T* dst = out;
+    T* tmp = nullptr;
+    if (parts > 1) {
+      tmp = static_cast<T*>(scratch_alloc(rows * parts * sizeof(T)));
+      if (!tmp) return LMP_ERR_OOM;
+      dst = tmp;
+    }
+    const dim3 grid{uint32_t(rows * parts)};
+    if constexpr (std::is_same_v<T, float> && V == 4) {
+      // Enough workgroups in flight, and the nontemporal hint for inputs that
+      // cannot stay in the MALL.
+      if (rows * len * sizeof(T) >= kStreamBytes)
+        hipLaunchKernelGGL((row_reduce_f32<OP, true>), grid, dim3(kBlock), 0, rt->stream, dst, in,
+                           uint32_t(units), uint32_t(seg), FastDiv(uint32_t(parts)));
+      else
+        hipLaunchKernelGGL((row_reduce_f32<OP, false>), grid, dim3(kBlock), 0, rt->stream, dst,
+                           in, uint32_t(units), uint32_t(seg), FastDiv(uint32_t(parts)));
+      LMP_LAUNCH_CHECK("row_reduce_f32");
+    } else {
+      hipLaunchKernelGGL((row_reduce_block<OP, T, V>), grid, dim3(kBlock), 0, rt->stream, dst, in,
+                         uint32_t(units), uint32_t(seg), FastDiv(uint32_t(parts)));
+      LMP_LAUNCH_CHECK("row_reduce_block");
+    }
+    if (parts > 1) {
+      hipLaunchKernelGGL((fold_parts<OP, T>), dim3(blocks_for(rows)), dim3(kBlock), 0, rt->stream,
+                         out, tmp, rows, uint32_t(parts));
+      LMP_LAUNCH_CHECK("fold_parts");
+      scratch_free(tmp);
+    }
+    return LMP_OK;
+  }
+  *done = false;
+  return LMP_OK;
+}
+
 template <int OP, typename T>
 int reduce_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len) {
-  if constexpr (std::is_same_v<T, float>) {
-    if (len >= 2048 && len % 4 == 0 && aligned16(in) && len / 4 <= kMaxU32Extent) {
-      const uint64_t len4 = len / 4;
-      // Enough workgroups to fill the chip twice over; split long rows only
-      // when rows alone cannot.
-      const uint64_t target = uint64_t(rt->cu_count) * 8;
-      uint64_t parts = 1;
-      if (rows < target) parts = std::min<uint64_t>((target + rows - 1) / rows,
-                                                    std::max<uint64_t>(1, len4 / 1024));
-      const uint64_t seg4 = (len4 + parts - 1) / parts;
-      parts = (len4 + seg4 - 1) / seg4;
-      if (rows * parts > 0x7fffffffull)
-        return fail(LMP_ERR_UNSUPPORTED, "reduce: too many rows");
-      float* dst = out;
-      float* tmp = nullptr;
-      if (parts > 1) {
-        tmp = static_cast<float*>(scratch_alloc(rows * parts * sizeof(float)));
-        if (!tmp) return LMP_ERR_OOM;
-        dst = tmp;
-      }
-      if (rows * len4 * 16 >= kStreamBytes)
-        hipLaunchKernelGGL((row_reduce_f32<OP, true>), dim3(uint32_t(rows * parts)),
-                           dim3(kBlock), 0, rt->stream, dst, in, uint32_t(len4),
-                           uint32_t(seg4), FastDiv(uint32_t(parts)));
-      else
-        hipLaunchKernelGGL((row_reduce_f32<OP, false>), dim3(uint32_t(rows * parts)),
-                           dim3(kBlock), 0, rt->stream, dst, in, uint32_t(len4),
-                           uint32_t(seg4), FastDiv(uint32_t(parts)));
-      LMP_LAUNCH_CHECK("row_reduce_f32");
-      if (parts > 1) {
-        hipLaunchKernelGGL((fold_parts<OP, float>), dim3(blocks_for(rows)),
-                           dim3(kBlock), 0, rt->stream, out, tmp, rows,
-                           uint32_t(parts));
-        LMP_LAUNCH_CHECK("fold_parts");
-        scratch_free(tmp);
-      }
-      return LMP_OK;
-    }
-  }
+  // float64 rows stay in units of one value up to 2048, as the fused row
+  // kernels take them.
+  bool done = false;
+  const bool pack = packs<T>(in, len) && !(std::is_same_v<T, double> && len < 2048);
+  const int rc = pack ? reduce_rows_as<OP, T, kPackOf<T>>(rt, out, in, rows, len, &done)
+                      : reduce_rows_as<OP, T, 1>(rt, out, in, rows, len, &done);
+  if (done) return rc;
   const uint64_t blocks = (rows + kWaves - 1) / kWaves;
   if (blocks > 0x7fffffffull) return fail(LMP_ERR_UNSUPPORTED, "reduce: too many rows");
   if constexpr (std::is_same_v<T, float>) {
@@ -464,20 +547,99 @@ int reduce_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len) {
   return LMP_OK;
 }
 
+template <int OP, typename T, int V>
+int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t len,
+                   uint64_t inner, bool second = false) {
+  constexpr uint64_t kUnit = sizeof(T) * V;
+  const uint64_t units = inner / V, cus = uint64_t(rt->cu_count);
+  const uint64_t n = outer * units;
+  // A lane per output where a slice is too short to share a workgroup
+  // ([30000, 16, 16] fp32 34.6 -> 6.0 us), or where the outputs give every CU
+  // two workgroups of lanes of one 4-byte value, rows are 128 bytes or more and
+  // the axis is short ([4096, 64, 33] fp32: 7.0 us, 7.6 us in strips; float64
+  // 15.3 and 12.2).
+  if ((len * units <= 128 || (n >= cus * 2 * kBlock && units * kUnit >= 128 && len <= 64 && kUnit == 4)) &&
+      n <= uint64_t(0x7fffffff) * kBlock) {
+    hipLaunchKernelGGL((col_reduce_lane<OP, T, V>), dim3(blocks_for(n)), dim3(kBlock), 0,
+                       rt->stream, out, in, n, uint32_t(units), uint32_t(len));
+    LMP_LAUNCH_CHECK("col_reduce_lane");
+    return LMP_OK;
+  }
+  // Strips of equal width, at most 64 units; narrower (256 bytes or more) for an
+  // axis of 128 rows or more while there are not four workgroups per CU
+  // ([16384,16384]: 176 us at 4/CU, 196 us at 8/CU; [256, 197, 768] at 3/CU 31.7
+  // us, at 4/CU 28.8; but [64, 151296] 7.5 us at 2.3/CU, 8.2 at 4/CU).
+  const uint64_t target = cus * 4;
+  const auto width = [&](uint64_t count) { return (units + count - 1) / count; };
+  uint64_t strips = (units + 63) / 64, S = 1;
+  while (len >= 128 && strips * outer < target && width(strips + 1) * kUnit >= 256) ++strips;
+  uint64_t cw = width(strips);
+  strips = (units + cw - 1) / cw;
+  if (strips * outer < target) {
+    // One pass for an axis of at most 4096 rows, with strips of 64 bytes or
+    // more until there are 128 workgroups, while a workgroup reads at most 128
+    // KiB (more than that costs more than a second launch: [4096, 4096] 25 us
+    // in one pass, 15 us in two); the partials of a first pass always.
+    uint64_t narrow = cw;
+    while (narrow * kUnit >= 128 && (units + narrow - 1) / narrow * outer < 128)
+      narrow = (narrow + 1) / 2;
+    if (second || (len <= kStripMaxLen && len * narrow * kUnit <= (128 << 10))) {
+      cw = narrow;
+      strips = (units + cw - 1) / cw;
+    } else {
+      // Chunks of at least 64 rows and 16 KiB.
+      const uint64_t base = strips * outer;
+      S = std::min({(target + base - 1) / base, std::max<uint64_t>(1, len / 64),
+                    std::max<uint64_t>(1, len * cw * kUnit / (16 << 10))});
+    }
+  }
+  const uint64_t chunk = (len + S - 1) / S;
+  S = (len + chunk - 1) / chunk;
+  const uint64_t blocks = strips * outer * S;
+  if (blocks > 0x7fffffffull) return fail(LMP_ERR_UNSUPPORTED, "reduce: too many columns");
+  T* dst = out;
+  T* tmp = nullptr;
+  if (S > 1) {
+    tmp = static_cast<T*>(scratch_alloc(outer * S * inner * sizeof(T)));
+    if (!tmp) return LMP_ERR_OOM;
+    dst = tmp;
+  }
+  const FastDiv dcw{uint32_t(cw)}, dst_strips{uint32_t(strips)}, dS{uint32_t(S)};
+  bool nt = false;
+  if constexpr (kUnit == 16) {
+    nt = outer * len * inner * sizeof(T) >= kStreamBytes;
+    if (nt)
+      hipLaunchKernelGGL((col_reduce_tile<OP, T, V, true>), dim3(uint32_t(blocks)), dim3(kBlock),
+                         0, rt->stream, dst, in, uint32_t(units), uint32_t(len), uint32_t(chunk),
+                         dcw, dst_strips, dS);
+  }
+  if (!nt)
+    hipLaunchKernelGGL((col_reduce_tile<OP, T, V, false>), dim3(uint32_t(blocks)), dim3(kBlock), 0,
+                       rt->stream, dst, in, uint32_t(units), uint32_t(len), uint32_t(chunk), dcw,
+                       dst_strips, dS);
+  LMP_LAUNCH_CHECK("col_reduce_tile");
+  if (S > 1) {
+    const int rc = reduce_cols_as<OP, T, V>(rt, out, tmp, outer, S, inner, true);
+    scratch_free(tmp);  // stream-ordered: the second pass reads it first
+    return rc;
+  }
+  return LMP_OK;
+}
+
 template <int OP, typename T>
 int reduce_cols(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t len,
                 uint64_t inner) {
-  const bool vec = std::is_same_v<T, float> && inner % 4 == 0 && aligned16(in) &&
-                   aligned16(out) && inner / 4 <= 0x7fffffffull &&
-                   len <= kMaxU32Extent;
-  // Lanes per workgroup along the columns: 64 float4 lanes (4 waves share a
-  // strip) on the vector path, 256 scalar lanes otherwise.
-  const uint64_t lanes = vec ? inner / 4 : inner;
-  const uint64_t per_wg = vec ? 64 : kBlock;
-  const uint64_t gx = (lanes + per_wg - 1) / per_wg;
-  if (gx > 0x7fffffffull || outer > 65535) {
-    // More outer slices than the grid's z extent (or columns than its x
-    // extent): one lane per output element, grid-striding.
+  // A short axis whose outputs give every CU two to eight workgroups of lanes:
+  // a lane per 4-byte value ([64, 151296] int32 7.1 us, 7.6 in strips of 16-byte
+  // units).
+  const uint64_t per_cu = outer * inner / kBlock / uint64_t(rt->cu_count);
+  const bool lanes = sizeof(T) == 4 && len <= 64 && inner >= 32 && per_cu >= 2 && per_cu < 8;
+  const bool pack = !lanes && packs<T>(in, inner) && aligned16(out);
+  const uint64_t units = pack ? inner / kPackOf<T> : inner;
+  if (units > kMaxU32Extent || len > kMaxU32Extent || outer > 65535) {
+    // Extents past the tile kernel's 32-bit counters, and more than 65535
+    // outer slices: one lane per output element, grid-striding, the axis
+    // folded in row order.
     const uint64_t n = outer * inner;
     const uint64_t cap = uint64_t(rt->cu_count) * 64;
     const uint64_t blocks = std::min<uint64_t>((n + kBlock - 1) / kBlock, cap);
@@ -486,70 +648,8 @@ int reduce_cols(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t len,
     LMP_LAUNCH_CHECK("col_reduce_flat");
     return LMP_OK;
   }
-  // Chunk the reduced axis until the grid reaches ~4 workgroups per CU
-  // (measured best for [16384,16384]: 176 us at 4/CU vs 196 us at 8/CU),
-  // keeping at least 64 rows per chunk.
-  const uint64_t target = uint64_t(rt->cu_count) * 4;
-  uint64_t S = 1;
-  const uint64_t base = gx * outer;
-  if (base < target) S = std::min<uint64_t>((target + base - 1) / base,
-                                            std::max<uint64_t>(1, len / 64));
-  S = std::min<uint64_t>(S, 65535);
-  if constexpr (std::is_same_v<T, float>) {
-    if (vec && S > 1 && len <= kStripMaxLen) {
-      // One pass: about 128 workgroups where the columns allow, 4..64 float4
-      // columns each.
-      const uint64_t inner4 = inner / 4;
-      uint32_t cw_log2 = 2;
-      while (cw_log2 < 6 && (inner4 >> (cw_log2 + 1)) >= 128) ++cw_log2;
-      const uint64_t gx1 = (inner4 + (1u << cw_log2) - 1) >> cw_log2;
-      const dim3 grid1{uint32_t(gx1), 1u, uint32_t(outer)};
-      hipLaunchKernelGGL((col_reduce_strip_f32<OP>), grid1, dim3(kBlock), 0, rt->stream, out,
-                         in, uint32_t(inner4), uint32_t(len), cw_log2);
-      LMP_LAUNCH_CHECK("col_reduce_strip_f32");
-      return LMP_OK;
-    }
-  }
-  const uint64_t chunk = (len + S - 1) / S;
-  S = (len + chunk - 1) / chunk;
-  T* dst = out;
-  T* tmp = nullptr;
-  if (S > 1) {
-    tmp = static_cast<T*>(scratch_alloc(outer * S * inner * sizeof(T)));
-    if (!tmp) return LMP_ERR_OOM;
-    dst = tmp;
-  }
-  const dim3 grid{uint32_t(gx), uint32_t(S), uint32_t(outer)};
-  if constexpr (std::is_same_v<T, float>) {
-    if (vec) {
-      if (outer * len * inner * sizeof(float) >= kStreamBytes)
-        hipLaunchKernelGGL((col_reduce_f32<OP, true>), grid, dim3(kBlock), 0, rt->stream,
-                           dst, in, uint32_t(inner / 4), uint32_t(len), uint32_t(chunk));
-      else
-        hipLaunchKernelGGL((col_reduce_f32<OP, false>), grid, dim3(kBlock), 0, rt->stream,
-                           dst, in, uint32_t(inner / 4), uint32_t(len), uint32_t(chunk));
-      LMP_LAUNCH_CHECK("col_reduce_f32");
-      if (S > 1) {
-        const uint64_t n4 = outer * (inner / 4);
-        hipLaunchKernelGGL((fold_chunks_f32<OP>), dim3(blocks_for(n4)), dim3(kBlock), 0,
-                           rt->stream, out, tmp, outer, uint32_t(inner / 4), uint32_t(S));
-        LMP_LAUNCH_CHECK("fold_chunks_f32");
-        scratch_free(tmp);
-      }
-      return LMP_OK;
-    }
-  }
-  hipLaunchKernelGGL((col_reduce_scalar<OP, T>), grid, dim3(kBlock), 0, rt->stream, dst,
-                     in, inner, len, chunk);
-  LMP_LAUNCH_CHECK("col_reduce_scalar");
-  if (S > 1) {
-    const uint64_t n = outer * inner;
-    hipLaunchKernelGGL((fold_chunks<OP, T>), dim3(blocks_for(n)), dim3(kBlock), 0,
-                       rt->stream, out, tmp, outer, inner, uint32_t(S));
-    LMP_LAUNCH_CHECK("fold_chunks");
-    scratch_free(tmp);
-  }
-  return LMP_OK;
+  return pack ? reduce_cols_as<OP, T, kPackOf<T>>(rt, out, in, outer, len, inner)
+              : reduce_cols_as<OP, T, 1>(rt, out, in, outer, len, inner);
 }
 
 // An empty reduced axis leaves every output at the functor's identity
