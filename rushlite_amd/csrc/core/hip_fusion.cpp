@@ -21,8 +21,10 @@
 // when it reduces to rows x cols with each leaf contiguous or broadcast along
 // the row, each lane of a one-shot grid produces one float4 (a one-wave
 // workgroup owns a contiguous 1 KiB output tile) from 128-bit loads and
-// stores it, with the nontemporal hint for large outputs; otherwise it
-// decomposes the flat index with compile-time extents.  Kernels launch on the library stream without a
+// stores it, with the nontemporal hint for large outputs; other layouts, and
+// float64, produce 16 bytes per lane too, with the flat index decomposed once
+// and carried over the lane's values with compile-time extents (outputs of
+// 2^31 values or more: one value per lane in 64-bit arithmetic).  Kernels launch on the library stream without a
 // device synchronisation (the reference synchronises every launch,
 // nvrtc_backend.cpp:135-141).
 #include <cstdio>
@@ -34,6 +36,7 @@
 #include <unordered_map>
 #include <unordered_set>
 
+#include "../hip/row_split.hpp"
 #include "ops.hpp"
 
 namespace lmp::tensor::hip {
@@ -144,27 +147,48 @@ bool is_reduce(const TensorImpl* t) {
 // ------------------------------------------------------------ row regions
 //
 // A region holding reduce nodes runs as a row kernel: one wave per row of the
-// reduced shape S = [..., N], each lane holding its share of the row in
-// registers.  Every node is either full (a shape that broadcasts to S with
-// last dim N) or a row value (one that broadcasts to S with last dim 1, e.g.
-// a [1, 1] loss seed), computed for each row; a reduce node turns a full value
-// of shape S into a row value of shape S1 (S with last dim 1) with
-// exactly the order of the eager wave-per-row kernel (row_reduce_wave_f32 for
-// float32 rows with N % 4 == 0, row_reduce_wave otherwise: four interleaved
-// accumulators, their pairwise combination, then a wave butterfly), so a
-// fused softmax equals the eager one bit for bit.  Rows of 2048 or more, which
-// the eager path reduces with a workgroup per row, are not fused.
-constexpr int64_t kRowMax = 2048;
+// reduced shape S = [..., N] (N < 2048), or one 256-lane workgroup (longer
+// rows), each lane holding its share of the row in registers.  Every node is
+// either full (a shape that broadcasts to S with last dim N) or a row value
+// (one that broadcasts to S with last dim 1, e.g. a [1, 1] loss seed), computed
+// for each row; a reduce node turns a full value of shape S into a row value of
+// shape S1 (S with last dim 1) with exactly the order of the eager kernel of
+// that length (row_reduce_wave_f32, row_reduce_wave, row_reduce_f32 or
+// row_reduce_block: four interleaved accumulators of 16-byte units or single
+// values, their pairwise combination, a wave butterfly and, for a workgroup,
+// the waves in order; a long row that the eager kernel splits over workgroups
+// is walked part by part), so a fused softmax equals the eager one bit for
+// bit.  Rows of more than kLaneValues values per lane are not fused.  A long
+// row's values stay in registers between its passes: softmax over 10,000
+// classes with its loss, forward and backward, 2048 rows: 604 -> 327 us (sixteen
+// kernels before, elementwise regions around eager reductions), what the 1.9 GB
+// of leaves and held values take at 5.8 TB/s.
+constexpr int64_t kLaneValues = 64;  // float32; half as many float64
 
 struct RowPlan {
   bool ok = false;
   std::vector<size_t> S;
   int64_t R = 0, N = 0;
-  bool vec_order = false;  // float32 and N % 4 == 0: elements come in float4s
-  bool vec_load = false;   // every full leaf can be read with aligned float4s
+  int lanes = 64;          // per row: a wave or a workgroup
+  int W = 1;               // values per unit
+  int64_t parts = 1;       // of a row, each `seg` units but the last
+  int64_t seg = 0;
+  bool vec_load = false;   // every full leaf can be read a unit at a time
   std::vector<bool> full;               // per leaf: varies along the row
   std::vector<int64_t> row_stride;      // per leaf, in elements
+  int64_t units() const { return N / W; }
 };
+
+int64_t device_cus() {
+  static const int64_t cus = [] {
+    lmp_rt_info info{};
+    int n = 0;
+    if (lmp_rt_device_count(&n) != LMP_OK || n == 0) return int64_t(256);  // source only
+    hip_ok(lmp_rt_device_info(&info), "lmp_rt_device_info");
+    return int64_t(info.cu_count);
+  }();
+  return cus;
+}
 
 // `sh` broadcasts to `S` (right-aligned, each dim equal or 1).
 bool bcast_to(const std::vector<size_t>& sh, const std::vector<size_t>& S) {
@@ -199,7 +223,7 @@ RowPlan row_plan(const Region& r) {
   const size_t nd = p.S.size();
   if (nd == 0) return p;
   p.N = static_cast<int64_t>(p.S.back());
-  if (p.N < 2 || p.N >= kRowMax) return p;
+  if (p.N < 2) return p;
   p.R = static_cast<int64_t>(shape_numel(p.S)) / p.N;
   if (p.R > (int64_t(1) << 31)) return p;  // one wave per row, one-shot grid
   std::vector<size_t> S1 = p.S;
@@ -216,8 +240,18 @@ RowPlan row_plan(const Region& r) {
   const TensorImpl* root = r.nodes.back();
   if (root->shape() != p.S && root->shape() != S1) return p;
   const bool f32 = root->type() == DataType::Float32;
-  p.vec_order = f32 && p.N % 4 == 0;
-  p.vec_load = p.vec_order;
+  const bool is_long = p.N >= static_cast<int64_t>(lmp_hip::kLongRow);
+  if (f32) p.W = p.N % 4 == 0 ? 4 : 1;
+  else p.W = is_long && p.N % 2 == 0 ? 2 : 1;
+  p.lanes = is_long ? lmp_hip::kRowLanes : 64;
+  if (is_long)
+    p.parts = static_cast<int64_t>(lmp_hip::row_parts(static_cast<uint64_t>(device_cus()),
+                                                      static_cast<uint64_t>(p.R),
+                                                      static_cast<uint64_t>(p.units())));
+  p.seg = (p.units() + p.parts - 1) / p.parts;
+  if (p.parts * ((p.seg + p.lanes - 1) / p.lanes) * p.W > (f32 ? kLaneValues : kLaneValues / 2))
+    return p;
+  p.vec_load = p.W > 1;
   for (TensorImpl* leaf : r.leaves) {
     const std::vector<stride_t> st = padded_strides(leaf->shape(), nd);
     const int64_t last = st[nd - 1];
@@ -237,7 +271,7 @@ RowPlan row_plan(const Region& r) {
     }
     p.full.push_back(last == 1);
     p.row_stride.push_back(rs);
-    if (last == 1 && (rs % 4 != 0 || (reinterpret_cast<uintptr_t>(leaf->raw()) & 15u) != 0))
+    if (last == 1 && (rs % p.W != 0 || (reinterpret_cast<uintptr_t>(leaf->raw()) & 15u) != 0))
       p.vec_load = false;
   }
   p.ok = true;
@@ -347,11 +381,15 @@ std::vector<Group> coalesce(const std::vector<size_t>& shape,
 }
 
 struct Plan {
-  bool vec = false;
+  bool vec = false;    // float4s of rows x cols with cols % 4 == 0
+  bool quad = false;   // 16 bytes per lane, any layout
   std::vector<Group> groups;
   uint64_t n = 0;      // output elements
-  uint64_t nvec = 0;   // vec: output float4s
+  uint64_t nvec = 0;   // vec, quad: output units (quad: the last may be partial)
   int64_t cols4 = 0;   // vec: float4s per row
+  int W = 4;           // values per unit
+  uint64_t aligned = 0;  // bit per leaf (of the first 64): starts on 16 bytes
+  bool is_aligned(size_t l) const { return l < 64 && (aligned >> l & 1u); }
 };
 
 Plan make_plan(const Region& r, const std::vector<size_t>& shape, bool f64) {
@@ -360,21 +398,27 @@ Plan make_plan(const Region& r, const std::vector<size_t>& shape, bool f64) {
   std::vector<std::vector<stride_t>> strides;
   for (TensorImpl* leaf : r.leaves) strides.push_back(padded_strides(leaf->shape(), shape.size()));
   p.groups = coalesce(shape, strides);
-  // The float4 plan is float32 only; float64 regions use the indexed loop.
-  if (f64 || p.groups.size() > 2 || p.n / 4 >= (1ull << 31)) return p;
+  // 32-bit indices from here on; larger outputs use the indexed loop.
+  if (p.n >= (1ull << 31)) return p;
+  p.W = f64 ? 2 : 4;
+  for (size_t l = 0; l < r.leaves.size() && l < 64; ++l)
+    if ((reinterpret_cast<uintptr_t>(r.leaves[l]->raw()) & 15u) == 0) p.aligned |= uint64_t(1) << l;
   const int64_t cols = p.groups.empty() ? 1 : p.groups[0].extent;
-  if (cols % 4 != 0) return p;
-  for (size_t l = 0; l < r.leaves.size(); ++l) {
+  bool vec = !f64 && p.groups.size() <= 2 && cols % 4 == 0;
+  for (size_t l = 0; l < r.leaves.size() && vec; ++l) {
     const int64_t in = p.groups.empty() ? 0 : p.groups[0].stride[l];
-    if (in != 0 && in != 1) return p;
-    if (in == 1) {
-      if ((reinterpret_cast<uintptr_t>(r.leaves[l]->raw()) & 15u) != 0) return p;
-      if (p.groups.size() == 2 && p.groups[1].stride[l] % 4 != 0) return p;
-    }
+    if (in != 0 && in != 1) vec = false;
+    if (in == 1 && (!p.is_aligned(l) || (p.groups.size() == 2 && p.groups[1].stride[l] % 4 != 0)))
+      vec = false;
   }
-  p.vec = true;
-  p.cols4 = cols / 4;
-  p.nvec = p.n / 4;
+  if (vec) {
+    p.vec = true;
+    p.cols4 = cols / 4;
+    p.nvec = p.n / 4;
+  } else {
+    p.quad = true;
+    p.nvec = (p.n + p.W - 1) / p.W;
+  }
   return p;
 }
 
@@ -414,6 +458,7 @@ std::vector<int64_t> signature(const Region& r, const std::vector<size_t>& shape
   s.push_back(0x4c4d5046);  // tag
   s.push_back(f64 ? 8 : 4);
   s.push_back(rp.ok ? (rp.vec_load ? 3 : 2) : 0);
+  s.push_back(rp.parts);
   for (size_t d : rp.S) s.push_back(static_cast<int64_t>(d));
   s.push_back(static_cast<int64_t>(shape.size()));
   for (size_t d : shape) s.push_back(static_cast<int64_t>(d));
@@ -422,7 +467,8 @@ std::vector<int64_t> signature(const Region& r, const std::vector<size_t>& shape
     s.push_back(static_cast<int64_t>(leaf->shape().size()));
     for (size_t d : leaf->shape()) s.push_back(static_cast<int64_t>(d));
   }
-  s.push_back(p.vec ? 1 : 0);
+  s.push_back(p.vec ? 1 : p.quad ? 2 : 0);
+  if (p.quad && !rp.ok) s.push_back(static_cast<int64_t>(p.aligned));
   s.push_back(static_cast<int64_t>(r.nodes.size()));
   for (TensorImpl* n : r.nodes) {
     const auto& fn = n->lazy_op();
@@ -479,6 +525,7 @@ void emit_chain(std::ostringstream& os, const Region& r, const std::string& inde
 #define LMP_WAVE_SWAP_SRC(...) #__VA_ARGS__
 const char* kPrelude = R"(
 typedef float lmp_v4 __attribute__((ext_vector_type(4)));
+typedef double lmp_d2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float lmp_clamp(float x, float lo, float hi) {
   return x < lo ? lo : (x > hi ? hi : x);
 }
@@ -513,8 +560,8 @@ void emit_region_params(std::ostringstream& os, const Region& r, const char* T,
 }
 
 void emit_params(std::ostringstream& os, const Region& r, const std::string& name,
-                 const char* T) {
-  os << "extern \"C\" __global__ __launch_bounds__(" << kBlock << ") void " << name << "(";
+                 const char* T, int threads = kBlock) {
+  os << "extern \"C\" __global__ __launch_bounds__(" << threads << ") void " << name << "(";
   emit_region_params(os, r, T, kSingle, true);
   os << ") {\n";
 }
@@ -592,14 +639,185 @@ void emit_vec_body(std::ostringstream& os, const Region& r, const Plan& p, const
   os << "  }\n  }\n";
 }
 
+// The body of a quad region: block `block` owns output units [kBlock * block,
+// kBlock * block + kBlock) (one-shot), W consecutive values of the flat output
+// each, stored at once.  The position of the first value is decomposed over
+// the groups; the others follow by carrying, so a unit may run over the ends
+// of rows.  Leaves of the whole output are read a unit at a time; a leaf that
+// broadcasts along the row by its first and last value's rows (one change of
+// row at most, rows being W or longer); where rows are whole units, leaves
+// contiguous along them a unit at a time and broadcast ones once.  [4095, 3001]
+// exp(a) * b - relu(a) / (b + 1): 43.3 -> 16.2 us, 6.1 TB/s (a loop over single
+// values in 64-bit arithmetic before).
+void emit_quad_body(std::ostringstream& os, const Region& r, const Plan& p, const char* T,
+                    const Names& nm, const std::string& block, bool stream_stores = false) {
+  const int W = p.W;
+  const char* VT = W == 4 ? "lmp_v4" : "lmp_d2";
+  const char* comp[4] = {"x", "y", "z", "w"};
+  const size_t nl = r.leaves.size(), G = p.groups.size();
+  const bool tail = p.n % W != 0;
+  const bool whole = G > 0 && p.groups[0].extent % W == 0;  // rows are whole units
+  const size_t item = W == 4 ? sizeof(float) : sizeof(double);
+  const auto flat = [&](size_t l) { return shape_numel(r.leaves[l]->shape()) == p.n; };
+  const auto single = [&](size_t l) { return shape_numel(r.leaves[l]->shape()) == 1; };
+  bool indexed = false;  // some leaf needs the position
+  for (size_t l = 0; l < nl; ++l) indexed |= !flat(l) && !single(l);
+
+  os << "  {\n  const unsigned v = " << block << " * " << kBlock << "u + threadIdx.x;\n";
+  os << "  if (v < " << p.nvec << "u) {\n  const unsigned i0 = v * " << W << "u;\n";
+  for (int e = 1; e < W && tail; ++e)
+    os << "  const bool k" << e << " = i0 + " << e << "u < " << p.n << "u;\n";
+  const std::string full = "k" + std::to_string(W - 1);
+  if (indexed) {
+    os << "  unsigned rest = i0;\n";
+    for (size_t g = 0; g < G; ++g) {
+      const std::string x = "x0_" + std::to_string(g), E = std::to_string(p.groups[g].extent) + "u";
+      if (g + 1 < G)
+        os << "  unsigned " << x << "; { const unsigned q = rest / " << E << "; " << x
+           << " = rest - q * " << E << "; rest = q; }\n";
+      else
+        os << "  const unsigned " << x << " = rest;\n";
+    }
+    // Later values: one further along, carried over the group extents; past
+    // the output's end the first value's position, so every load is inside.
+    for (int e = 1; e < W && !whole; ++e) {
+      std::string carry = "1u";
+      for (size_t g = 0; g < G; ++g) {
+        const std::string x = "x" + std::to_string(e) + "_" + std::to_string(g);
+        os << "  unsigned " << x << " = x" << e - 1 << "_" << g << " + " << carry << ";\n";
+        if (g + 1 < G) {
+          const std::string c = "c" + std::to_string(e) + "_" + std::to_string(g);
+          os << "  const unsigned " << c << " = " << x << " == " << p.groups[g].extent
+             << "u ? 1u : 0u; " << x << " = " << c << " ? 0u : " << x << ";\n";
+          carry = c;
+        }
+      }
+      if (tail)
+        for (size_t g = 0; g < G; ++g)
+          os << "  if (!k" << e << ") x" << e << "_" << g << " = x0_" << g << ";\n";
+    }
+  }
+  // A leaf's offset at value e of the unit.
+  const auto offset = [&](size_t l, int e) {
+    std::string t;
+    for (size_t g = 0; g < G; ++g) {
+      const int64_t st = p.groups[g].stride[l];
+      if (!st) continue;
+      const int at = whole ? 0 : e;
+      t += (t.empty() ? "" : " + ") + ("(unsigned long)x" + std::to_string(at) + "_" + std::to_string(g)) +
+           " * " + std::to_string(st) + "ul";
+      if (whole && e > 0 && g == 0) t += " + " + std::to_string(st * e) + "ul";
+    }
+    return t.empty() ? std::string("0ul") : t;
+  };
+  std::vector<std::vector<std::string>> val(nl, std::vector<std::string>(W));
+  for (size_t l = 0; l < nl; ++l) {
+    const std::string in = nm.in + std::to_string(l), s = "s" + std::to_string(l);
+    const bool stream = r.leaves[l]->nbytes() >= kStreamBytes;
+    const auto unit_load = [&](const std::string& at) {
+      const std::string ptr = "reinterpret_cast<const " + std::string(VT) + "*>(" + in + " + " + at + ")";
+      return stream ? "__builtin_nontemporal_load(" + ptr + ")" : "*" + ptr;
+    };
+    if (single(l)) {
+      os << "  const " << T << " " << s << " = " << in << "[0];\n";
+      for (int e = 0; e < W; ++e) val[l][e] = s;
+      continue;
+    }
+    const bool inner1 = !flat(l) && p.groups[0].stride[l] == 1;
+    const bool inner0 = !flat(l) && p.groups[0].stride[l] == 0;
+    const bool aligned = p.is_aligned(l);
+    bool rows_aligned = aligned;
+    for (size_t g = 1; g < G; ++g) rows_aligned &= p.groups[g].stride[l] % W == 0;
+    if (flat(l) && aligned) {
+      os << "  " << VT << " " << s << ";\n  ";
+      if (tail) os << "if (" << full << ") ";
+      os << s << " = " << unit_load("i0") << ";\n";
+      if (tail) {
+        os << "  else { " << s << " = " << VT << "(0); " << s << ".x = " << in << "[i0];";
+        for (int e = 1; e + 1 < W; ++e)
+          os << " if (k" << e << ") " << s << "." << comp[e] << " = " << in << "[i0 + " << e << "u];";
+        os << " }\n";
+      }
+      for (int e = 0; e < W; ++e) val[l][e] = s + "." + comp[e];
+    } else if (flat(l)) {
+      for (int e = 0; e < W; ++e) {
+        val[l][e] = s + "_" + std::to_string(e);
+        os << "  const " << T << " " << val[l][e] << " = " << in << "[i0 + "
+           << (tail && e ? "(k" + std::to_string(e) + " ? " + std::to_string(e) + "u : 0u)"
+                         : std::to_string(e) + "u")
+           << "];\n";
+      }
+    } else if (whole && inner0) {
+      os << "  const " << T << " " << s << " = " << in << "[" << offset(l, 0) << "];\n";
+      for (int e = 0; e < W; ++e) val[l][e] = s;
+    } else if (whole && inner1 && rows_aligned) {
+      os << "  const " << VT << " " << s << " = " << unit_load(offset(l, 0)) << ";\n";
+      for (int e = 0; e < W; ++e) val[l][e] = s + "." + comp[e];
+    } else if (inner0 && p.groups[0].extent >= W) {
+      os << "  const unsigned long " << s << "f = " << offset(l, 0) << ", " << s
+         << "g = " << offset(l, W - 1) << ";\n  const " << T << " " << s << "a = " << in << "[" << s
+         << "f], " << s << "b = " << in << "[" << s << "g];\n";
+      // The tail's missing values carry the first one's position: their rows
+      // are the first's, and any change of row before them is looked up too.
+      for (int e = 0; e < W; ++e) {
+        val[l][e] = s + "_" + std::to_string(e);
+        if (tail && e > 0 && e + 1 < W)
+          os << "  const " << T << " " << val[l][e] << " = " << in << "[" << offset(l, e) << "];\n";
+        else if (e == 0)
+          os << "  const " << T << " " << val[l][e] << " = " << s << "a;\n";
+        else if (e == W - 1)
+          os << "  const " << T << " " << val[l][e] << " = " << s << "b;\n";
+        else
+          os << "  const " << T << " " << val[l][e] << " = (" << offset(l, e) << ") == " << s
+             << "f ? " << s << "a : " << s << "b;\n";
+      }
+    } else {
+      for (int e = 0; e < W; ++e) {
+        val[l][e] = s + "_" + std::to_string(e);
+        os << "  const " << T << " " << val[l][e] << " = " << in << "[" << offset(l, e) << "];\n";
+      }
+    }
+  }
+  os << "  " << VT << " o;\n";
+  for (size_t k = 0; k < r.outputs.size(); ++k) os << "  " << VT << " y" << k << ";\n";
+  for (int e = 0; e < W; ++e) {
+    os << "  {\n";
+    emit_chain(os, r, "    ", std::string("o.") + comp[e], T, [&](int l) { return val[l][e]; });
+    for (size_t k = 0; k < r.outputs.size(); ++k)
+      os << "    y" << k << "." << comp[e] << " = t" << r.node_of.at(r.outputs[k]) << ";\n";
+    os << "  }\n";
+  }
+  const bool stream_out = stream_stores || p.n * item > kStreamStoreBytes;
+  const auto store = [&](const std::string& x, const std::string& dst) {
+    os << "  ";
+    if (tail) os << "if (" << full << ") ";
+    if (stream_out)
+      os << "__builtin_nontemporal_store(" << x << ", reinterpret_cast<" << VT << "*>(" << dst
+         << ") + v);\n";
+    else
+      os << "reinterpret_cast<" << VT << "*>(" << dst << ")[v] = " << x << ";\n";
+    if (tail) {
+      os << "  else { " << dst << "[i0] = " << x << ".x;";
+      for (int e = 1; e + 1 < W; ++e)
+        os << " if (k" << e << ") " << dst << "[i0 + " << e << "u] = " << x << "." << comp[e] << ";";
+      os << " }\n";
+    }
+  };
+  for (size_t k = 0; k < r.outputs.size(); ++k)
+    store("y" + std::to_string(k), nm.xo + std::to_string(k));
+  store("o", nm.out);
+  os << "  }\n  }\n";
+}
+
 std::string codegen(const Region& r, const Plan& p, const std::string& name, bool f64) {
   const char* T = f64 ? "double" : "float";
   std::ostringstream os;
   os << kPrelude;
   emit_params(os, r, name, T);
   const size_t nl = r.leaves.size();
-  if (p.vec) {
-    emit_vec_body(os, r, p, kSingle, "blockIdx.x");
+  if (p.vec || p.quad) {
+    if (p.vec) emit_vec_body(os, r, p, kSingle, "blockIdx.x");
+    else emit_quad_body(os, r, p, T, kSingle, "blockIdx.x");
     os << "}\n";
   } else {
     os << "  const unsigned long n = " << p.n << "ul;\n";
@@ -627,38 +845,8 @@ std::string codegen(const Region& r, const Plan& p, const std::string& name, boo
   return os.str();
 }
 
-// The body of an indexed region run one-shot: block `block` owns elements
-// [kBlock * block, kBlock * block + kBlock), each decomposed into leaf offsets with
-// compile-time extents and strides.
-void emit_indexed_body(std::ostringstream& os, const Region& r, const Plan& p, const char* T,
-                       const Names& nm, const std::string& block) {
-  const size_t nl = r.leaves.size();
-  os << "  {\n  const unsigned long i = (unsigned long)" << block << " * " << kBlock
-     << "u + threadIdx.x;\n";
-  os << "  if (i < " << p.n << "ul) {\n";
-  os << "    unsigned long rest = i;\n";
-  for (size_t l = 0; l < nl; ++l) os << "    unsigned long o" << l << " = 0;\n";
-  for (size_t g = 0; g < p.groups.size(); ++g) {
-    os << "    {\n      const unsigned long q = rest / " << p.groups[g].extent
-       << "ul;\n      const unsigned long c = rest - q * " << p.groups[g].extent
-       << "ul;\n      rest = q;\n";
-    for (size_t l = 0; l < nl; ++l)
-      if (p.groups[g].stride[l])
-        os << "      o" << l << " += c * " << p.groups[g].stride[l] << "ul;\n";
-    os << "    }\n";
-  }
-  os << "    " << T << " res;\n    {\n";
-  emit_chain(os, r, "      ", "res", T, [&](int l) {
-    return nm.in + std::to_string(l) + "[o" + std::to_string(l) + "]";
-  });
-  for (size_t k = 0; k < r.outputs.size(); ++k)
-    os << "      " << nm.xo << k << "[i] = t" << r.node_of.at(r.outputs[k]) << ";\n";
-  os << "    }\n    " << nm.out << "[i] = res;\n  }\n  }\n";
-}
-
 // One kernel for several independent elementwise regions (realize_all):
-// region i owns workgroups [off_i, off_i + blocks_i), float4 lanes for a vec
-// plan, one element per lane otherwise.
+// region i owns workgroups [off_i, off_i + blocks_i), 16 bytes per lane.
 std::string codegen_multi(const std::vector<const Region*>& rs, const std::vector<const Plan*>& ps,
                           const std::vector<bool>& f64, const std::vector<uint64_t>& blocks,
                           const std::string& name) {
@@ -681,65 +869,113 @@ std::string codegen_multi(const std::vector<const Region*>& rs, const std::vecto
     os << (i ? "  else " : "  ") << "if (blockIdx.x < " << off + blocks[i] << "u)\n";
     const std::string block = "(blockIdx.x - " + std::to_string(off) + "u)";
     if (ps[i]->vec) emit_vec_body(os, *rs[i], *ps[i], region_names(i), block, stream_group);
-    else emit_indexed_body(os, *rs[i], *ps[i], f64[i] ? "double" : "float", region_names(i), block);
+    else
+      emit_quad_body(os, *rs[i], *ps[i], f64[i] ? "double" : "float", region_names(i), block,
+                     stream_group);
     off += blocks[i];
   }
   os << "}\n";
   return os.str();
 }
 
-// Row kernel for a region with reduce nodes (see RowPlan).
+// Row kernel for a region with reduce nodes (see RowPlan).  A lane's units
+// are listed part by part; unit k of the list is unit k.base + lane of the row.
 std::string codegen_rows(const Region& r, const RowPlan& rp, const std::string& name,
                          bool f64) {
+  struct Unit {
+    int64_t base;   // row unit of lane 0
+    int64_t at;     // base within the part
+    int64_t count;  // units of the part
+    bool every;     // inside the part for every lane
+  };
   const char* T = f64 ? "double" : "float";
-  const bool vo = rp.vec_order;
-  const int64_t NN = vo ? rp.N / 4 : rp.N;      // units a lane steps over
-  const int64_t TT = (NN + 63) / 64;            // units per lane
-  const int64_t E = vo ? TT * 4 : TT;           // elements per lane
-  const auto elem_col = [&](int64_t e) {        // column of element e, as code
+  const char* VT = f64 ? "lmp_d2" : "lmp_v4";
+  const char* comp[4] = {"x", "y", "z", "w"};
+  const int W = rp.W;
+  const int64_t L = rp.lanes;
+  const bool group = L > 64;  // a workgroup per row
+  std::vector<Unit> units;
+  std::vector<size_t> first;  // of each part, and the end
+  for (int64_t s = 0; s < rp.parts; ++s) {
+    const int64_t count = std::min(rp.seg, rp.units() - s * rp.seg);
+    first.push_back(units.size());
+    for (int64_t at = 0; at < count; at += L)
+      units.push_back(Unit{s * rp.seg + at, at, count, at + L <= count});
+  }
+  first.push_back(units.size());
+  const size_t E = units.size() * W;  // elements per lane
+  const auto elem_col = [&](size_t e) {  // column of element e, as code
     std::ostringstream c;
-    if (vo) c << "4u * (lane + " << 64 * (e / 4) << "u) + " << e % 4 << "u";
-    else c << "lane + " << 64 * e << "u";
+    c << W << "u * (lane + " << units[e / W].base << "u) + " << e % W << "u";
     return c.str();
   };
-  const auto ok_of = [&](int64_t e) { return "ok" + std::to_string(vo ? e / 4 : e); };
+  const auto ok = [&](size_t k) { return "ok" + std::to_string(k); };
   std::vector<bool> node_full(r.nodes.size());
   for (size_t m = 0; m < r.nodes.size(); ++m)
     node_full[m] = !is_reduce(r.nodes[m]) && static_cast<int64_t>(last_dim(r.nodes[m]->shape())) == rp.N;
+  // Nontemporal where all that a long-row kernel reads, or stores, is more than
+  // the MALL keeps from one kernel to the next (softmax over 10,000 classes with
+  // its loss, forward and backward, 2048 rows: 346 us with neither, 338 with the
+  // stores, 327 with both).
+  const size_t item = f64 ? sizeof(double) : sizeof(float);
+  size_t read = 0, written = 0;
+  for (size_t l = 0; l < r.leaves.size(); ++l)
+    if (rp.full[l]) read += r.leaves[l]->nbytes();
+  for (size_t m = 0; m < r.nodes.size(); ++m)
+    if (node_full[m] && (r.out_of.count(r.nodes[m]) || m + 1 == r.nodes.size()))
+      written += shape_numel(r.nodes[m]->shape()) * item;
+  const bool stream_in = group && read >= kStreamBytes,
+             stream_out = group && written > kStreamStoreBytes;
 
   std::ostringstream os;
   os << kPrelude;
-  emit_params(os, r, name, T);
-  os << "  const unsigned lane = threadIdx.x & 63u;\n";
-  os << "  const unsigned long row = (unsigned long)blockIdx.x * " << kBlock / 64
-     << "ul + (threadIdx.x >> 6);\n";
-  os << "  if (row >= " << rp.R << "ul) return;\n";
-  for (int64_t t = 0; t < TT; ++t)
-    os << "  const bool ok" << t << " = lane + " << 64 * t << "u < " << NN << "u;\n";
-  // Leaves.
-  for (size_t l = 0; l < r.leaves.size(); ++l) {
+  emit_params(os, r, name, T, rp.lanes);
+  os << "  const unsigned lane = threadIdx.x;\n";
+  os << "  const unsigned long row = blockIdx.x;\n";
+  if (group) {
+    size_t reduces = 0;
+    for (TensorImpl* n : r.nodes) reduces += is_reduce(n);
+    os << "  __shared__ " << T << " lmp_sh[" << reduces * rp.parts << "][" << L / 64 << "];\n";
+  }
+  for (size_t k = 0; k < units.size(); ++k)
+    if (!units[k].every)
+      os << "  const bool " << ok(k) << " = lane + " << units[k].at << "u < " << units[k].count
+         << "u;\n";
+  // Leaves: all before the first node in a wave's kernel; in a workgroup's
+  // before the first node that reads them, so a lane holds fewer values.
+  const auto load_leaf = [&](size_t l) {
     const std::string base = "in" + std::to_string(l) + " + row * " +
                              std::to_string(rp.row_stride[l]) + "ul";
     if (!rp.full[l]) {
       os << "  const " << T << " l" << l << " = *(" << base << ");\n";
-      continue;
+      return;
     }
-    if (rp.vec_load) {
-      for (int64_t t = 0; t < TT; ++t) {
-        os << "  const lmp_v4 q" << l << "_" << t << " = ok" << t
-           << " ? *reinterpret_cast<const lmp_v4*>(" << base << " + 4u * (lane + " << 64 * t
-           << "u)) : lmp_v4{0.0f, 0.0f, 0.0f, 0.0f};\n";
-        const char* comp[4] = {"x", "y", "z", "w"};
-        for (int c = 0; c < 4; ++c)
-          os << "  const " << T << " l" << l << "_" << 4 * t + c << " = q" << l << "_" << t
-             << "." << comp[c] << ";\n";
-      }
-    } else {
-      for (int64_t e = 0; e < E; ++e)
-        os << "  const " << T << " l" << l << "_" << e << " = " << ok_of(e) << " ? (" << base
-           << ")[" << elem_col(e) << "] : " << T << "(0);\n";
+    for (size_t k = 0; k < units.size() && rp.vec_load; ++k) {
+      const std::string q = "q" + std::to_string(l) + "_" + std::to_string(k);
+      const std::string ptr = "reinterpret_cast<const " + std::string(VT) + "*>(" + base + " + " +
+                              std::to_string(W) + "u * (lane + " + std::to_string(units[k].base) + "u))";
+      const std::string ld = stream_in ? "__builtin_nontemporal_load(" + ptr + ")" : "*" + ptr;
+      os << "  const " << VT << " " << q << " = ";
+      if (units[k].every) os << ld << ";\n";
+      else os << ok(k) << " ? " << ld << " : " << VT << "(0);\n";
+      for (int c = 0; c < W; ++c)
+        os << "  const " << T << " l" << l << "_" << W * k + c << " = " << q << "." << comp[c] << ";\n";
     }
-  }
+    for (size_t e = 0; e < E && !rp.vec_load; ++e) {
+      os << "  const " << T << " l" << l << "_" << e << " = ";
+      if (!units[e / W].every) os << ok(e / W) << " ? ";
+      os << "(" << base << ")[" << elem_col(e) << "]";
+      if (!units[e / W].every) os << " : " << T << "(0)";
+      os << ";\n";
+    }
+  };
+  std::vector<bool> loaded(r.leaves.size(), false);
+  const auto need_leaf = [&](size_t l) {
+    if (!loaded[l]) load_leaf(l);
+    loaded[l] = true;
+  };
+  if (!group)
+    for (size_t l = 0; l < r.leaves.size(); ++l) need_leaf(l);
   const auto arg = [&](const std::shared_ptr<TensorImpl>& in, int64_t e) {
     auto lt = r.leaf_of.find(in.get());
     if (lt != r.leaf_of.end())
@@ -748,16 +984,51 @@ std::string codegen_rows(const Region& r, const RowPlan& rp, const std::string& 
     const int k = r.node_of.at(in.get());
     return "v" + std::to_string(k) + (node_full[k] && e >= 0 ? "_" + std::to_string(e) : "");
   };
+  const auto store = [&](size_t m, const std::string& ptr) {
+    if (!node_full[m]) {
+      if (shape_numel(r.nodes[m]->shape()) == 1 && rp.R > 1)
+        os << "  if (lane == 0u && row == 0ul) " << ptr << "[0] = v" << m << ";\n";
+      else
+        os << "  if (lane == 0u) " << ptr << "[row] = v" << m << ";\n";
+      return;
+    }
+    const std::string obase = ptr + " + row * " + std::to_string(rp.N) + "ul";
+    for (size_t k = 0; k < units.size(); ++k) {
+      os << "  ";
+      if (!units[k].every) os << "if (" << ok(k) << ") ";
+      if (W == 1) {
+        os << "(" << obase << ")[" << elem_col(k) << "] = v" << m << "_" << k << ";\n";
+        continue;
+      }
+      std::string val = std::string(VT) + "{";
+      for (int c = 0; c < W; ++c)
+        val += (c ? ", v" : "v") + std::to_string(m) + "_" + std::to_string(W * k + c);
+      const std::string ptr = "reinterpret_cast<" + std::string(VT) + "*>(" + obase + " + " +
+                              std::to_string(W) + "u * (lane + " + std::to_string(units[k].base) + "u))";
+      if (stream_out) os << "__builtin_nontemporal_store(" << val << "}, " << ptr << ");\n";
+      else os << "*" << ptr << " = " << val << "};\n";
+    }
+  };
+  const auto store_if_output = [&](size_t m) {
+    auto it = r.out_of.find(r.nodes[m]);
+    if (it != r.out_of.end()) store(m, "xo" + std::to_string(it->second));
+    if (m + 1 == r.nodes.size()) store(m, "out");
+  };
+  size_t slot = 0;  // lmp_sh row of the next reduce node
   for (size_t m = 0; m < r.nodes.size(); ++m) {
     const auto& fn = r.nodes[m]->lazy_op();
+    for (const auto& in : fn->inputs)
+      if (auto lt = r.leaf_of.find(in.get()); lt != r.leaf_of.end())
+        need_leaf(static_cast<size_t>(lt->second));
     if (!is_reduce(r.nodes[m])) {
-      const int64_t count = node_full[m] ? E : 1;
+      const int64_t count = node_full[m] ? static_cast<int64_t>(E) : 1;
       for (int64_t e = 0; e < count; ++e) {
         std::vector<std::string> args;
         for (const auto& in : fn->inputs) args.push_back(arg(in, node_full[m] ? e : -1));
         os << "  const " << T << " v" << m << (node_full[m] ? "_" + std::to_string(e) : "")
            << " = " << substitute(fn->codegen_expr(), args) << ";\n";
       }
+      if (group) store_if_output(m);
       continue;
     }
     // Reduction in the eager kernels' order.
@@ -776,72 +1047,92 @@ std::string codegen_rows(const Region& r, const RowPlan& rp, const std::string& 
         default: return "(" + x + " < " + acc + " ? " + x + " : " + acc + ")";
       }
     };
-    const std::string P = "r" + std::to_string(m) + "_";
-    const int W = vo ? 4 : 1;  // components per accumulator
-    const auto acc = [&](int i, int c) { return P + "a" + std::to_string(i) + "_" + std::to_string(c); };
-    const auto src = [&](int64_t t, int c) { return arg(fn->inputs[0], vo ? 4 * t + c : t); };
     os << "  " << T << " v" << m << ";\n  {\n";
-    for (int i = 0; i < 4; ++i)
-      for (int c = 0; c < W; ++c) os << "    " << T << " " << acc(i, c) << " = " << id << ";\n";
-    os << "    unsigned " << P << "gd = 0u;\n";
-    for (int64_t g = 0; 4 * g + 3 < TT; ++g) {
-      os << "    if (lane + " << 64 * (4 * g + 3) << "u < " << NN << "u) {\n";
-      for (int i = 0; i < 4; ++i)
+    for (int64_t s = 0; s < rp.parts; ++s) {
+      const std::string P = "r" + std::to_string(m) + "_" + std::to_string(s) + "_";
+      const auto acc = [&](int i, int c) { return P + "a" + std::to_string(i) + "_" + std::to_string(c); };
+      const auto add = [&](const std::string& indent, int i, size_t k) {
         for (int c = 0; c < W; ++c)
-          os << "      " << acc(i, c) << " = " << comb(acc(i, c), src(4 * g + i, c)) << ";\n";
-      os << "      " << P << "gd = " << g + 1 << "u;\n    }\n";
-    }
-    for (int64_t t = 0; t < TT; ++t) {
-      os << "    if (" << t << "u >= 4u * " << P << "gd && ok" << t << ") {\n";
-      for (int c = 0; c < W; ++c)
-        os << "      " << acc(0, c) << " = " << comb(acc(0, c), src(t, c)) << ";\n";
-      os << "    }\n";
-    }
-    std::vector<std::string> b;
-    for (int c = 0; c < W; ++c)
-      b.push_back(comb(comb(acc(0, c), acc(1, c)), comb(acc(2, c), acc(3, c))));
-    os << "    " << T << " " << P << "v = ";
-    if (vo) {
-      os << T << "(0);\n";
-      for (int c = 0; c < 4; ++c)
-        os << "    const " << T << " " << P << "b" << c << " = " << b[c] << ";\n";
-      os << "    " << P << "v = " << comb(comb(P + "b0", P + "b1"), comb(P + "b2", P + "b3"))
+          os << indent << acc(i, c) << " = "
+             << comb(acc(i, c), arg(fn->inputs[0], static_cast<int64_t>(W * k + c))) << ";\n";
+      };
+      for (int i = 0; i < 4; ++i)
+        for (int c = 0; c < W; ++c) os << "    " << T << " " << acc(i, c) << " = " << id << ";\n";
+      // Units by fours into the four accumulators while the lane has all
+      // four, the rest into the first one.
+      size_t k = first[s];
+      const size_t end = first[s + 1];
+      for (; k + 4 <= end && units[k + 3].every; k += 4)
+        for (int i = 0; i < 4; ++i) add("    ", i, k + i);
+      if (k + 4 <= end) {
+        os << "    if (" << ok(k + 3) << ") {\n";
+        for (int i = 0; i < 4; ++i) add("      ", i, k + i);
+        os << "    } else {\n";
+        for (size_t t = k; t < k + 3; ++t) {
+          if (!units[t].every) os << "      if (" << ok(t) << ") {\n";
+          add("      ", 0, t);
+          if (!units[t].every) os << "      }\n";
+        }
+        os << "    }\n";
+      } else {
+        for (size_t t = k; t < end; ++t) {
+          if (!units[t].every) os << "    if (" << ok(t) << ") {\n";
+          add("    ", 0, t);
+          if (!units[t].every) os << "    }\n";
+        }
+      }
+      std::vector<std::string> b;
+      for (int c = 0; c < W; ++c) {
+        b.push_back(P + "b" + std::to_string(c));
+        os << "    const " << T << " " << b.back() << " = "
+           << comb(comb(acc(0, c), acc(1, c)), comb(acc(2, c), acc(3, c))) << ";\n";
+      }
+      os << "    " << T << " " << P << "v = "
+         << (W == 4 ? comb(comb(b[0], b[1]), comb(b[2], b[3])) : W == 2 ? comb(b[0], b[1]) : b[0])
          << ";\n";
-    } else {
-      os << b[0] << ";\n";
-    }
-    for (int off = 1; off <= 32; off <<= 1)
-      os << "    { const " << T << " o = lmp_swap<" << off << ">(" << P << "v); " << P
-         << "v = " << comb(P + "v", "o") << "; }\n";
-    // Every lane goes on with lane 0's result, the value the eager kernel
-    // stores (the lanes can differ where max/min tie +0 and -0).
-    os << "    v" << m << " = lmp_lane0(" << P << "v);\n  }\n";
-  }
-  os << "  // stores\n";
-  const auto store = [&](size_t m, const std::string& ptr) {
-    if (!node_full[m]) {
-      if (shape_numel(r.nodes[m]->shape()) == 1 && rp.R > 1)
-        os << "  if (lane == 0u && row == 0ul) " << ptr << "[0] = v" << m << ";\n";
+      for (int off = 1; off <= 32; off <<= 1)
+        os << "    { const " << T << " o = lmp_swap<" << off << ">(" << P << "v); " << P
+           << "v = " << comb(P + "v", "o") << "; }\n";
+      if (group)
+        os << "    if ((lane & 63u) == 0u) lmp_sh[" << slot + s << "][lane >> 6] = " << P << "v;\n";
       else
-        os << "  if (lane == 0u) " << ptr << "[row] = v" << m << ";\n";
-      return;
+        // Every lane goes on with lane 0's result, the value the eager kernel
+        // stores (the lanes can differ where max/min tie +0 and -0).
+        os << "    v" << m << " = lmp_lane0(" << P << "v);\n";
     }
-    const std::string obase = ptr + " + row * " + std::to_string(rp.N) + "ul";
-    if (vo) {
-      for (int64_t t = 0; t < TT; ++t)
-        os << "  if (ok" << t << ") *reinterpret_cast<lmp_v4*>(" << obase << " + 4u * (lane + "
-           << 64 * t << "u)) = lmp_v4{v" << m << "_" << 4 * t << ", v" << m << "_"
-           << 4 * t + 1 << ", v" << m << "_" << 4 * t + 2 << ", v" << m << "_"
-           << 4 * t + 3 << "};\n";
-    } else {
-      for (int64_t e = 0; e < E; ++e)
-        os << "  if (ok" << e << ") (" << obase << ")[" << elem_col(e) << "] = v" << m << "_"
-           << e << ";\n";
+    if (group) {
+      // The waves' results in order, then the parts' from the identity.
+      os << "    __syncthreads();\n";
+      const auto part = [&](int64_t s) {
+        std::string t = "lmp_sh[" + std::to_string(slot + s) + "][0]";
+        for (int64_t w = 1; w < L / 64; ++w) {
+          os << "    const " << T << " w" << s << "_" << w << " = "
+             << comb(t, "lmp_sh[" + std::to_string(slot + s) + "][" + std::to_string(w) + "]") << ";\n";
+          t = "w" + std::to_string(s) + "_" + std::to_string(w);
+        }
+        return t;
+      };
+      if (rp.parts == 1) {
+        const std::string t = part(0);
+        os << "    v" << m << " = " << t << ";\n";
+      } else {
+        os << "    v" << m << " = " << id << ";\n";
+        for (int64_t s = 0; s < rp.parts; ++s) {
+          const std::string t = part(s);
+          os << "    v" << m << " = " << comb("v" + std::to_string(m), t) << ";\n";
+        }
+      }
+      slot += static_cast<size_t>(rp.parts);
     }
-  };
-  for (size_t k = 0; k < r.outputs.size(); ++k)
-    store(static_cast<size_t>(r.node_of.at(r.outputs[k])), "xo" + std::to_string(k));
-  store(r.nodes.size() - 1, "out");
+    os << "  }\n";
+    if (group) store_if_output(m);
+  }
+  if (!group) {
+    os << "  // stores\n";
+    for (size_t k = 0; k < r.outputs.size(); ++k)
+      store(static_cast<size_t>(r.node_of.at(r.outputs[k])), "xo" + std::to_string(k));
+    store(r.nodes.size() - 1, "out");
+  }
   os << "}\n";
   return os.str();
 }
@@ -867,18 +1158,16 @@ struct Job {
   std::vector<size_t> shape;
   Storage out{0, DeviceType::HIP};  // empty until prepare() allocates or takes a target
   std::vector<Storage> extra;
-  // One lane per float4 (vec, one-shot), per row wave, or per element
-  // (grid-stride loop, one-shot up to 2^30 workgroups).
+  // One lane per unit (vec, quad: one-shot), one workgroup per row, or one
+  // lane per element (grid-stride loop, one-shot up to 2^30 workgroups).
   uint64_t blocks() const {
-    const uint64_t work = rp.ok ? uint64_t(rp.R) * 64 : p.vec ? p.nvec : p.n;
+    if (rp.ok) return uint64_t(rp.R);
+    const uint64_t work = p.vec || p.quad ? p.nvec : p.n;
     const uint64_t grid = (work + kBlock - 1) / kBlock;
     return std::max<uint64_t>(1, std::min<uint64_t>(grid, uint64_t(1) << 30));
   }
-  // Workgroups when run inside a group (one-shot for the indexed plan too).
-  uint64_t group_blocks() const {
-    const uint64_t work = p.vec ? p.nvec : p.n;
-    return std::max<uint64_t>(1, (work + kBlock - 1) / kBlock);
-  }
+  uint64_t group_blocks() const { return std::max<uint64_t>(1, (p.nvec + kBlock - 1) / kBlock); }
+  int threads() const { return rp.ok ? rp.lanes : kBlock; }
   void push_args(std::vector<void*>& ptrs) const {
     ptrs.push_back(out.data());
     for (const Storage& x : extra) ptrs.push_back(x.data());
@@ -964,7 +1253,7 @@ class HipFusionBackend : public lazy::LazyBackend {
       const size_t np = 1 + j.r.outputs.size() + j.r.leaves.size();
       // Row kernels, and regions large enough to fill the chip on their own
       // (2^20 workgroups is far past that), launch alone.
-      if (j.rp.ok || j.group_blocks() > (uint64_t(1) << 20)) {
+      if (j.rp.ok || !(j.p.vec || j.p.quad) || j.group_blocks() > (uint64_t(1) << 20)) {
         launch_single(j);
         continue;
       }
@@ -1040,7 +1329,7 @@ class HipFusionBackend : public lazy::LazyBackend {
       job.finish();
       return false;
     }
-    job.p = make_plan(r, job.shape, job.f64);
+    if (!job.rp.ok) job.p = make_plan(r, job.shape, job.f64);
     return true;
   }
 
@@ -1060,10 +1349,11 @@ class HipFusionBackend : public lazy::LazyBackend {
     return handle;
   }
 
-  void launch(void* handle, uint64_t grid, std::vector<void*>& ptrs) {
+  void launch(void* handle, uint64_t grid, int threads, std::vector<void*>& ptrs) {
     std::vector<void*> args(ptrs.size());
     for (size_t i = 0; i < ptrs.size(); ++i) args[i] = &ptrs[i];
-    hip_ok(lmp_jit_launch(handle, static_cast<uint32_t>(grid), kBlock, args.data()),
+    hip_ok(lmp_jit_launch(handle, static_cast<uint32_t>(grid), static_cast<uint32_t>(threads),
+                          args.data()),
            "lmp_jit_launch");
     ++backend_stats().fused_launches;
   }
@@ -1077,11 +1367,11 @@ class HipFusionBackend : public lazy::LazyBackend {
     std::vector<void*> ptrs;
     ptrs.reserve(r.leaves.size() + r.outputs.size() + 1);
     job.push_args(ptrs);
-    launch(handle, job.blocks(), ptrs);
+    launch(handle, job.blocks(), job.threads(), ptrs);
     backend_stats().fused_nodes += r.nodes.size();
     if (fusion_log())
       std::fprintf(stderr, "[lmp fusion] %s root %s nodes %zu leaves %zu outputs %zu\n",
-                   job.rp.ok ? "rows" : job.p.vec ? "vec" : "indexed",
+                   job.rp.ok ? "rows" : job.p.vec ? "vec" : job.p.quad ? "quad" : "indexed",
                    shape_text(job.shape).c_str(), r.nodes.size(), r.leaves.size(),
                    r.outputs.size());
     job.finish();
@@ -1110,7 +1400,7 @@ class HipFusionBackend : public lazy::LazyBackend {
                             [&] { return codegen_multi(rs, ps, f64, blocks, "lmp_fused"); });
     std::vector<void*> ptrs;
     for (const Job* j : group) j->push_args(ptrs);
-    launch(handle, grid, ptrs);
+    launch(handle, grid, kBlock, ptrs);
     backend_stats().fused_nodes += nodes;
     if (fusion_log())
       std::fprintf(stderr, "[lmp fusion] group of %zu regions, %zu nodes\n", group.size(),
@@ -1171,8 +1461,7 @@ std::string fused_group_source_for(const std::vector<TensorImpl*>& roots) {
     f64.push_back(root->type() == DataType::Float64);
     ps.push_back(make_plan(rs.back(), root->shape(), f64.back()));
     LMP_CHECK(!row_plan(rs.back()).ok) << "row regions are not grouped";
-    const uint64_t work = ps.back().vec ? ps.back().nvec : ps.back().n;
-    blocks.push_back(std::max<uint64_t>(1, (work + kBlock - 1) / kBlock));
+    blocks.push_back(std::max<uint64_t>(1, (ps.back().nvec + kBlock - 1) / kBlock));
   }
   std::vector<const Region*> rp;
   std::vector<const Plan*> pp;

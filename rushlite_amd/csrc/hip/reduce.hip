@@ -36,6 +36,7 @@
 
 #include "common.hpp"
 #include "ops.hpp"
+#include "row_split.hpp"
 
 namespace lmp_hip {
 
@@ -43,7 +44,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 namespace {
 
-constexpr int kBlock = 256;
+constexpr int kBlock = kRowLanes;
 constexpr int kWaves = kBlock / 64;
 
 #define LMP_WAVE_SWAP_SRC(...) __VA_ARGS__
@@ -455,14 +456,6 @@ bool packs(const void* p, uint64_t extent) {
   return kPackOf<T> > 1 && extent % kPackOf<T> == 0 && aligned16(p);
 }
 
-// Workgroups per row of a long row: enough to fill the chip twice over, more
-// than one only when the rows alone cannot.
-uint64_t row_parts(Runtime* rt, uint64_t rows, uint64_t units) {
-  const uint64_t target = uint64_t(rt->cu_count) * 8;
-  if (rows >= target) return 1;
-  return std::min<uint64_t>((target + rows - 1) / rows, std::max<uint64_t>(1, units / 1024));
-}
-
 template <int OP, typename T, int V, int G>
 int launch_small_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t units) {
   hipLaunchKernelGGL((row_reduce_small<OP, T, V, G>), dim3(blocks_for(rows * G)), dim3(kBlock), 0,
@@ -482,10 +475,9 @@ int reduce_rows_as(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len
     if (units <= 16) return launch_small_rows<OP, T, V, 16>(rt, out, in, rows, units);
     return launch_small_rows<OP, T, V, 32>(rt, out, in, rows, units);
   }
-  if (len >= 2048 && units <= kMaxU32Extent) {
-    uint64_t parts = row_parts(rt, rows, units);
+  if (len >= kLongRow && units <= kMaxU32Extent) {
+    const uint64_t parts = row_parts(uint64_t(rt->cu_count), rows, units);
     const uint64_t seg = (units + parts - 1) / parts;
-    parts = (units + seg - 1) / seg;
     if (rows * parts > 0x7fffffffull) return fail(LMP_ERR_UNSUPPORTED, "reduce: too many rows");
     T* dst = out;
     T* tmp = nullptr;
@@ -524,10 +516,10 @@ int reduce_rows_as(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len
 
 template <int OP, typename T>
 int reduce_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len) {
-  // float64 rows stay in units of one value up to 2048, as the fused row
-  // kernels take them.
+  // Short float64 rows stay in units of one value, as the fused row kernels
+  // take them.
   bool done = false;
-  const bool pack = packs<T>(in, len) && !(std::is_same_v<T, double> && len < 2048);
+  const bool pack = packs<T>(in, len) && !(std::is_same_v<T, double> && len < kLongRow);
   const int rc = pack ? reduce_rows_as<OP, T, kPackOf<T>>(rt, out, in, rows, len, &done)
                       : reduce_rows_as<OP, T, 1>(rt, out, in, rows, len, &done);
   if (done) return rc;
