@@ -380,6 +380,11 @@ std::vector<Group> coalesce(const std::vector<size_t>& shape,
   return g;
 }
 
+// Smaller outputs that are not whole float4s take one value per lane: their
+// kernels are bound by latency, and the shorter code (no row ends inside a
+// lane, no partial last unit) starts sooner.
+constexpr uint64_t kShortOutput = 1 << 14;
+
 struct Plan {
   bool vec = false;    // float4s of rows x cols with cols % 4 == 0
   bool quad = false;   // 16 bytes per lane, any layout
@@ -417,6 +422,7 @@ Plan make_plan(const Region& r, const std::vector<size_t>& shape, bool f64) {
     p.nvec = p.n / 4;
   } else {
     p.quad = true;
+    if (p.n < kShortOutput) p.W = 1;
     p.nvec = (p.n + p.W - 1) / p.W;
   }
   return p;
@@ -652,12 +658,13 @@ void emit_vec_body(std::ostringstream& os, const Region& r, const Plan& p, const
 void emit_quad_body(std::ostringstream& os, const Region& r, const Plan& p, const char* T,
                     const Names& nm, const std::string& block, bool stream_stores = false) {
   const int W = p.W;
-  const char* VT = W == 4 ? "lmp_v4" : "lmp_d2";
-  const char* comp[4] = {"x", "y", "z", "w"};
+  const char* VT = W == 4 ? "lmp_v4" : W == 2 ? "lmp_d2" : T;
+  const char* comp4[4] = {".x", ".y", ".z", ".w"};
+  const auto comp = [&](int e) { return W == 1 ? "" : comp4[e]; };
   const size_t nl = r.leaves.size(), G = p.groups.size();
   const bool tail = p.n % W != 0;
   const bool whole = G > 0 && p.groups[0].extent % W == 0;  // rows are whole units
-  const size_t item = W == 4 ? sizeof(float) : sizeof(double);
+  const size_t item = T[0] == 'f' ? sizeof(float) : sizeof(double);
   const auto flat = [&](size_t l) { return shape_numel(r.leaves[l]->shape()) == p.n; };
   const auto single = [&](size_t l) { return shape_numel(r.leaves[l]->shape()) == 1; };
   bool indexed = false;  // some leaf needs the position
@@ -735,10 +742,10 @@ void emit_quad_body(std::ostringstream& os, const Region& r, const Plan& p, cons
       if (tail) {
         os << "  else { " << s << " = " << VT << "(0); " << s << ".x = " << in << "[i0];";
         for (int e = 1; e + 1 < W; ++e)
-          os << " if (k" << e << ") " << s << "." << comp[e] << " = " << in << "[i0 + " << e << "u];";
+          os << " if (k" << e << ") " << s << comp(e) << " = " << in << "[i0 + " << e << "u];";
         os << " }\n";
       }
-      for (int e = 0; e < W; ++e) val[l][e] = s + "." + comp[e];
+      for (int e = 0; e < W; ++e) val[l][e] = s + comp(e);
     } else if (flat(l)) {
       for (int e = 0; e < W; ++e) {
         val[l][e] = s + "_" + std::to_string(e);
@@ -752,7 +759,7 @@ void emit_quad_body(std::ostringstream& os, const Region& r, const Plan& p, cons
       for (int e = 0; e < W; ++e) val[l][e] = s;
     } else if (whole && inner1 && rows_aligned) {
       os << "  const " << VT << " " << s << " = " << unit_load(offset(l, 0)) << ";\n";
-      for (int e = 0; e < W; ++e) val[l][e] = s + "." + comp[e];
+      for (int e = 0; e < W; ++e) val[l][e] = s + comp(e);
     } else if (inner0 && p.groups[0].extent >= W) {
       os << "  const unsigned long " << s << "f = " << offset(l, 0) << ", " << s
          << "g = " << offset(l, W - 1) << ";\n  const " << T << " " << s << "a = " << in << "[" << s
@@ -782,9 +789,9 @@ void emit_quad_body(std::ostringstream& os, const Region& r, const Plan& p, cons
   for (size_t k = 0; k < r.outputs.size(); ++k) os << "  " << VT << " y" << k << ";\n";
   for (int e = 0; e < W; ++e) {
     os << "  {\n";
-    emit_chain(os, r, "    ", std::string("o.") + comp[e], T, [&](int l) { return val[l][e]; });
+    emit_chain(os, r, "    ", std::string("o") + comp(e), T, [&](int l) { return val[l][e]; });
     for (size_t k = 0; k < r.outputs.size(); ++k)
-      os << "    y" << k << "." << comp[e] << " = t" << r.node_of.at(r.outputs[k]) << ";\n";
+      os << "    y" << k << comp(e) << " = t" << r.node_of.at(r.outputs[k]) << ";\n";
     os << "  }\n";
   }
   const bool stream_out = stream_stores || p.n * item > kStreamStoreBytes;
@@ -799,7 +806,7 @@ void emit_quad_body(std::ostringstream& os, const Region& r, const Plan& p, cons
     if (tail) {
       os << "  else { " << dst << "[i0] = " << x << ".x;";
       for (int e = 1; e + 1 < W; ++e)
-        os << " if (k" << e << ") " << dst << "[i0 + " << e << "u] = " << x << "." << comp[e] << ";";
+        os << " if (k" << e << ") " << dst << "[i0 + " << e << "u] = " << x << comp(e) << ";";
       os << " }\n";
     }
   };

@@ -25,12 +25,14 @@ def _same(a, b):
     assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
 
 
-# Output sizes around one unit, rows of one to a few values (several row ends
+# Small outputs (one value per lane), then sizes around one unit, rows of one to a few values (several row ends
 # in a unit), odd rows, whole-unit rows under 3-d and 4-d broadcasts.
 LAYOUTS = [((1,), (1,)), ((3,), (1,)), ((5,), (5,)), ((7, 1), (1, 3)), ((9, 3), (9, 1)), ((33, 5), (5,)),
            ((1, 2), (9, 1)), ((255, 7), (255, 1)), ((64, 130), (130,)), ((4, 1, 3), (1, 5, 3)), ((2, 3, 8), (3, 1)),
            ((5, 6, 8), (5, 1, 8)), ((3, 4, 12), (1, 4, 1)), ((2, 3, 4, 5), (3, 1, 5)), ((6, 1, 2, 1), (1, 5, 1, 4)),
-           ((1001, 37), (1001, 37)), ((70, 4, 6), (70, 1, 6))]
+           ((1001, 37), (1001, 37)), ((70, 4, 6), (70, 1, 6)), ((8003, 3), (8003, 1)), ((30001, 1), (1, 2)),
+           ((4001, 7), (7,)), ((40, 1, 30), (1, 17, 30)), ((60, 17, 20), (60, 1, 20)), ((50, 3, 128), (3, 1)),
+           ((3, 90, 2, 40), (90, 1, 40)), ((16385,), (1,)), ((20002,), (20002,))]
 
 
 @pytest.mark.parametrize("sa,sb", LAYOUTS, ids=str)
