@@ -15,7 +15,7 @@
 // owns 2 x 2 blocks of 16 x 16 accumulated by v_mfma_f64_16x16x4f64 (lane l
 // supplies A[l % 16][l / 16] and B[l / 16][l % 16]; accumulator register r
 // holds row 4r + l / 16, column l % 16).  K advances 16 at a time through two
-// LDS buffers with register prefetch of the next tile, one barrier per step.
+// LDS buffers with register prefetch of the next tiles, one barrier per step.
 // The integer kernel uses the same 64 x 64 tiles staged through LDS, each
 // thread owning a 4 x 4 block of C.
 #include <hip/hip_runtime.h>
@@ -45,6 +45,10 @@ struct TypedArgs {
   int lda, ldb, ldc;
   int accumulate;
   int vec;  // float64: both operands 16-byte aligned with even leading dimensions
+  // float64, 64 x 64 tiles: K tiles per split (blockIdx.y), and with several
+  // splits their partials, m * n values each.
+  int tiles_per_split;
+  double* part;
 };
 
 // Thread f's element of a [kTile x kBK] A tile (row-major in k when !TA) or a
@@ -209,13 +213,20 @@ __device__ __forceinline__ void f64_step_schedule() {
 // float64 on 64 x 64 tiles of 4 waves, each wave 2 x 2 blocks of 16 x 16, for
 // products whose 128 x 128 tiles do not cover the CUs.  Loads as in
 // gemm_f64_big (pairs of the [64 x 16] panels, unchecked for aligned tiles
-// inside C, checked otherwise, the same LDS tile either way); each unchecked
-// K step puts the 4 loads of the next tile one per MFMA at its start and the
-// LDS stores one per MFMA among its last MFMAs.  Measured against its
-// element-wise checked loads: 1024^3 71-77 -> 60-64 us, 1536^3 206-214 ->
-// 176-191 us (three orientations each).
+// inside C, checked otherwise, the same LDS tile either way).  A CU holds one
+// wave per SIMD here, so nothing covers a wait: a K step's MFMAs take 1024
+// cycles, about a load's latency, and the registers run two tiles ahead of
+// them (step t stores tile t + 1 to LDS and then issues the loads of tile
+// t + 2); each group of four MFMAs is issued behind the next group's LDS reads;
+// the last group of a tile runs past the barrier.  Two workgroups per CU in the
+// launch bounds keep the accumulators in VGPRs (64 moves a step otherwise).
+// 1024^3 58-60 -> 46.5-48 us (46 TFLOP/s; loads one tile ahead, 59% of the step
+// waiting, before), 1536^3 179 -> 150.  With fewer tiles than CUs K is split
+// over blockIdx.y, at least four K tiles each, into partials added in split
+// order: 512^3 29.3 -> 14.9 us, 200 x 200 x 2000 113 -> 14.9, 96 x 96 x 2047 119
+// -> 11.3 (unsplit before).
 template <bool TA, bool TB>
-__global__ __launch_bounds__(kThreads) void gemm_f64_mfma(TypedArgs g) {
+__global__ __launch_bounds__(kThreads, 2) void gemm_f64_mfma(TypedArgs g) {
   __shared__ double smem[2][2][kLds];  // [buffer][A|B], each [k][m or n], pitch kTile + 1
   const int tiles_n = (g.n + kTile - 1) / kTile;
   const int m0 = int(blockIdx.x / tiles_n) * kTile, n0 = int(blockIdx.x % tiles_n) * kTile;
@@ -243,68 +254,94 @@ __global__ __launch_bounds__(kThreads) void gemm_f64_mfma(TypedArgs g) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  // MFMA operands of the four k from 4 s on, and the MFMAs.
+  double af[2][2], bf[2][2];
+  auto read = [&](int cur, int s) {
+    const int kk = 4 * s + lk;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      af[s & 1][i] = smem[cur][0][kk * (kTile + 1) + wm * 32 + i * 16 + li];
+      bf[s & 1][i] = smem[cur][1][kk * (kTile + 1) + wn * 32 + i * 16 + li];
+    }
+  };
+  auto mma = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[i][j] =
+            __builtin_amdgcn_mfma_f64_16x16x4f64(af[s & 1][i], bf[s & 1][j], acc[i][j], 0, 0, 0);
+  };
+  static_assert(kBK == 16, "four groups of four k");
+  // The first three groups of a tile, each with the next one's reads in front.
   auto compute = [&](int cur) {
-    const double* As = smem[cur][0];
-    const double* Bs = smem[cur][1];
 #pragma unroll
-    for (int s = 0; s < kBK / 4; ++s) {
-      const int kk = 4 * s + lk;
-      double af[2], bf[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) af[i] = As[kk * (kTile + 1) + wm * 32 + i * 16 + li];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) bf[j] = Bs[kk * (kTile + 1) + wn * 32 + j * 16 + li];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
+    for (int s = 0; s < 3; ++s) {
+      read(cur, s + 1);
+      mma(s);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // LDS reads
+      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);  // MFMAs
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  const int k_tiles = (g.k + kBK - 1) / kBK;
-  // Steps kt < unchecked_end load tile kt + 1, which lies wholly inside K.
-  const int unchecked_end = inside ? g.k / kBK - 1 : 0;
-  if (inside) {
-    pa.load_unchecked(0, g.lda);
-    pb.load_unchecked(0, g.ldb);
-  } else {
-    load_checked(0);
-  }
+  const int kt0 = int(blockIdx.y) * g.tiles_per_split;
+  const int kt1 = min((g.k + kBK - 1) / kBK, kt0 + g.tiles_per_split);
+  const int whole = inside ? g.k / kBK : 0;  // tiles below it load unchecked
+  auto load = [&](int kt) {
+    if (kt < whole) {
+      pa.load_unchecked(kt * kBK, g.lda);
+      pb.load_unchecked(kt * kBK, g.ldb);
+    } else {
+      load_checked(kt * kBK);
+    }
+  };
+  load(kt0);
   store(0);
+  if (kt0 + 1 < kt1) load(kt0 + 1);
   __syncthreads();
-  int kt = 0;
-  for (; kt < unchecked_end; ++kt) {
-    const int cur = kt & 1;
-    pa.load_unchecked((kt + 1) * kBK, g.lda);
-    pb.load_unchecked((kt + 1) * kBK, g.ldb);
-    compute(cur);
+  // The last group of a tile is held past the barrier, over the next tile's
+  // first reads, its stores and the loads after it: each load has a whole step
+  // before its store, each operand a group of MFMAs.  Zeros before the first.
+#pragma unroll
+  for (int i = 0; i < 2; ++i) af[1][i] = bf[1][i] = 0.0;
+  int kt = kt0;
+  for (const int end = min(whole, kt1) - 2; kt < end; ++kt) {
+    const int cur = (kt - kt0) & 1;
+    read(cur, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(3);
     store(cur ^ 1);
-    // masks: 0x8 MFMA, 0x20 global load, 0x100 LDS read, 0x200 LDS write
-    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    }
-    __syncthreads();
-  }
-  for (; kt < k_tiles; ++kt) {
-    const int cur = kt & 1;
-    const bool more = kt + 1 < k_tiles;
-    if (more) load_checked((kt + 1) * kBK);
+    pa.load_unchecked((kt + 2) * kBK, g.lda);
+    pb.load_unchecked((kt + 2) * kBK, g.ldb);
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+    __builtin_amdgcn_sched_group_barrier(0x200, 4, 0);  // LDS writes
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x200, 4, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x020, 4, 0);  // global loads
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_barrier(0);
     compute(cur);
-    if (more) store(cur ^ 1);
     __syncthreads();
   }
+  for (; kt < kt1; ++kt) {
+    const int cur = (kt - kt0) & 1;
+    read(cur, 0);
+    mma(3);
+    if (kt + 1 < kt1) store(cur ^ 1);
+    if (kt + 2 < kt1) load(kt + 2);
+    compute(cur);
+    __syncthreads();
+  }
+  mma(3);
 
   double* C = static_cast<double*>(g.c);
+  int64_t ldc = g.ldc;
+  if (g.part) {
+    C = g.part + int64_t(blockIdx.y) * g.m * g.n;
+    ldc = g.n;
+  }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -314,11 +351,31 @@ __global__ __launch_bounds__(kThreads) void gemm_f64_mfma(TypedArgs g) {
       for (int r = 0; r < 4; ++r) {
         const int row = m0 + wm * 32 + i * 16 + 4 * r + lk;
         if (row < g.m && col < g.n) {
-          double* p = C + int64_t(row) * g.ldc + col;
-          *p = g.accumulate ? *p + acc[i][j][r] : acc[i][j][r];
+          double* p = C + row * ldc + col;
+          *p = g.accumulate && !g.part ? *p + acc[i][j][r] : acc[i][j][r];
         }
       }
     }
+}
+
+// C (+)= the partials of `splits` K splits, in split order.
+__global__ __launch_bounds__(kThreads) void fold_f64(TypedArgs g, int splits) {
+  const int64_t mn = int64_t(g.m) * g.n;
+  const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
+  if (i >= mn) return;
+  double v = g.part[i];
+  int s = 1;
+  for (; s + 8 <= splits; s += 8) {
+    double x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = g.part[(s + u) * mn + i];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v += x[u];
+  }
+  for (; s < splits; ++s) v += g.part[s * mn + i];
+  const int64_t row = i / g.n;
+  double* p = static_cast<double*>(g.c) + row * g.ldc + (i - row * g.n);
+  *p = g.accumulate ? *p + v : v;
 }
 
 template <bool TA, bool TB>
@@ -487,31 +544,60 @@ __global__ __launch_bounds__(kThreads) void gemm_int(TypedArgs g) {
     }
 }
 
+// The split of K on 64 x 64 tiles: none once there is a tile for every CU, else
+// enough workgroups to cover the CUs, four K tiles or more each.
+int f64_splits(Runtime* rt, int64_t tiles, int k) {
+  const int64_t k_tiles = (k + kBK - 1) / kBK;
+  if (tiles >= rt->cu_count) return 1;
+  return int(std::max<int64_t>(1, std::min<int64_t>((rt->cu_count + tiles - 1) / tiles, k_tiles / 4)));
+}
+
 template <typename T, bool TA, bool TB>
-void launch_typed(Runtime* rt, const TypedArgs& g) {
+int launch_typed(Runtime* rt, TypedArgs g) {
   const int64_t tiles = int64_t((g.m + kTile - 1) / kTile) * ((g.n + kTile - 1) / kTile);
   const int64_t big_tiles = int64_t((g.m + kBig - 1) / kBig) * ((g.n + kBig - 1) / kBig);
   if constexpr (std::is_same_v<T, double>) {
-    if (big_tiles >= rt->cu_count)
+    if (big_tiles >= rt->cu_count) {
       hipLaunchKernelGGL((gemm_f64_big<TA, TB>), dim3(uint32_t(big_tiles)), dim3(kThreads), 0,
                          rt->stream, g);
-    else
-      hipLaunchKernelGGL((gemm_f64_mfma<TA, TB>), dim3(uint32_t(tiles)), dim3(kThreads), 0,
-                         rt->stream, g);
+      LMP_LAUNCH_CHECK("gemm_f64_big");
+      return LMP_OK;
+    }
+    const int k_tiles = (g.k + kBK - 1) / kBK;
+    int splits = f64_splits(rt, tiles, g.k);
+    g.tiles_per_split = (k_tiles + splits - 1) / splits;
+    splits = (k_tiles + g.tiles_per_split - 1) / g.tiles_per_split;
+    const int64_t mn = int64_t(g.m) * g.n;
+    if (splits > 1) {
+      g.part = static_cast<double*>(scratch_alloc(size_t(splits) * size_t(mn) * sizeof(double)));
+      if (!g.part) {  // no room for the partials: unsplit
+        splits = 1;
+        g.tiles_per_split = k_tiles;
+      }
+    }
+    hipLaunchKernelGGL((gemm_f64_mfma<TA, TB>), dim3(uint32_t(tiles), uint32_t(splits)),
+                       dim3(kThreads), 0, rt->stream, g);
+    LMP_LAUNCH_CHECK("gemm_f64_mfma");
+    if (g.part) {
+      hipLaunchKernelGGL(fold_f64, dim3(uint32_t((mn + kThreads - 1) / kThreads)), dim3(kThreads),
+                         0, rt->stream, g, splits);
+      LMP_LAUNCH_CHECK("fold_f64");
+      scratch_free(g.part);  // stream-ordered: the fold reads it first
+    }
   } else {
     hipLaunchKernelGGL((gemm_int<T, TA, TB>), dim3(uint32_t(tiles)), dim3(kThreads), 0,
                        rt->stream, g);
+    LMP_LAUNCH_CHECK("gemm_int");
   }
+  return LMP_OK;
 }
 
 template <typename T>
 int dispatch_typed(Runtime* rt, bool ta, bool tb, const TypedArgs& g) {
-  if (!ta && !tb) launch_typed<T, false, false>(rt, g);
-  else if (!ta && tb) launch_typed<T, false, true>(rt, g);
-  else if (ta && !tb) launch_typed<T, true, false>(rt, g);
-  else launch_typed<T, true, true>(rt, g);
-  LMP_LAUNCH_CHECK("gemm (typed)");
-  return LMP_OK;
+  if (!ta && !tb) return launch_typed<T, false, false>(rt, g);
+  if (!ta && tb) return launch_typed<T, false, true>(rt, g);
+  if (ta && !tb) return launch_typed<T, true, false>(rt, g);
+  return launch_typed<T, true, true>(rt, g);
 }
 
 }  // namespace
@@ -548,7 +634,7 @@ extern "C" int lmp_k_gemm(int dtype, int trans_a, int trans_b, size_t m, size_t 
   const bool vec = reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(b) % 16 == 0 && lda % 2 == 0 && ldb % 2 == 0;
   TypedArgs g{a, b, c, int(m), int(n), int(k), int(lda), int(ldb), int(ldc),
-              accumulate ? 1 : 0, vec ? 1 : 0};
+              accumulate ? 1 : 0, vec ? 1 : 0, 0, nullptr};
   const bool ta = trans_a != 0, tb = trans_b != 0;
   switch (dtype) {
     case LMP_FLOAT64: return dispatch_typed<double>(rt, ta, tb, g);
