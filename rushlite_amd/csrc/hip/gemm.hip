@@ -1300,14 +1300,19 @@ __global__ __launch_bounds__(NT, MINB) void gemm_f32_lds(GemmArgs g) {
 
 // ------------------------------------------------------------------ rows
 //
-// M <= 32 with B transposed and enough columns to give every CU a block of
-// 32 (Linear's input gradient dY * W^T at a small batch: C[m, n] =
-// sum_k A[m, k] * Bs[n, k] with the weight stored as Bs [n, k]).  Column j of
-// C needs row j of Bs in full, so a workgroup that owns 32 columns reads 32
-// whole rows of Bs -- one contiguous span of memory -- over all of K: no
-// split of K, no partials, no fold.  (The split-K direct kernel instead reads
-// 4 KiB pieces of 128 rows 16 KiB apart.)  Its four waves take consecutive
-// quarters of K and add their 32x32 blocks through LDS in wave order.
+// M <= 32 with B transposed (Linear's input gradient dY * W^T at a small
+// batch: C[m, n] = sum_k A[m, k] * Bs[n, k] with the weight stored as Bs
+// [n, k]).  Column j of C needs row j of Bs, so a workgroup that owns 32 columns
+// reads 32 rows of Bs: whole ones, one contiguous span of memory, when
+// there are as many blocks as CUs, and otherwise a K range of them, into
+// partials that fold_splits adds in split order.  Bound by reading Bs.  (The
+// direct kernel, which ran the split case before, reads 32-byte pieces of 128
+// rows per instruction with a third of the bytes in flight: 32 x 4096 x 8192 65.5
+// us there, 32.0 here (4.2 TB/s); 8 x 4096 x 4096 32.7 and 17.3; 32 x 6000 x
+// 3000 58.3 and 27.9; 32 x 1024 x 1024 13.2 and 7.5; 20 x 8000 x 64 6.2 and
+// 4.0.)  The four waves take consecutive quarters of the K range and
+// add their 32x32 blocks through LDS in wave order; within a wave, MFMA step s
+// adds to accumulator s % ACCS, which shortens the chains of rounded sums.
 //
 // Operands move through wave-private LDS rings: per group of 32 k values a
 // 32 x 32 tile of A and one of Bs (4 KiB each), each filled by four
@@ -1338,13 +1343,14 @@ struct RowsArgs {
   const float* bias;  // per-column bias added to the output (or null)
   int relu;           // with a bias: ReLU after it
   int vec_out;        // C and the bias take 128-bit accesses
+  int k_per_wg;       // K range of one workgroup (a multiple of 32 * kRowsWaves)
 };
 
 constexpr int kRowsWaves = 4;
 constexpr int kRowsStages = 3;
 constexpr int kRowsTile = 32 * 32;  // floats of one operand tile
 
-template <int STAGES>
+template <int STAGES, int ACCS>
 __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_thin_rows(RowsArgs g) {
   constexpr int STAGE = 2 * kRowsTile;  // A tile, then B tile
   __shared__ __attribute__((aligned(1024))) float smem[kRowsWaves * STAGES * STAGE];
@@ -1352,8 +1358,8 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_thin_rows(RowsArgs g)
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int li = lane & 31, lh = lane >> 5;
   const int n0 = int(blockIdx.x) * 32;
-  const int part = ((g.k + kRowsWaves - 1) / kRowsWaves + 31) / 32 * 32;
-  const int kb = wave * part;
+  const int part = g.k_per_wg / kRowsWaves;
+  const int kb = int(blockIdx.y) * g.k_per_wg + wave * part;
   const int ke = min(g.k, kb + part);
   const int ntiles = kb < ke ? (ke - kb + 31) / 32 : 0;
   const int rot = ntiles ? int((blockIdx.x * 13u) % uint32_t(ntiles)) : 0;
@@ -1388,7 +1394,9 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_thin_rows(RowsArgs g)
       lds_dma16_nt(bsrc[q] && k0 + dk[q] < ke ? bsrc[q] + k0 : zero, st + kRowsTile + q * 256);
   };
 
-  v16f acc = v16f(0.0f);
+  v16f accs[ACCS];
+#pragma unroll
+  for (int i = 0; i < ACCS; ++i) accs[i] = v16f(0.0f);
 #pragma unroll
   for (int t = 0; t < STAGES - 1; ++t)
     if (t < ntiles) issue(t);
@@ -1412,8 +1420,14 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_thin_rows(RowsArgs g)
     }
 #pragma unroll
     for (int s = 0; s < 16; ++s)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[s / 4][s % 4], fb[s / 4][s % 4], acc, 0, 0, 0);
+      accs[s % ACCS] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[s / 4][s % 4], fb[s / 4][s % 4],
+                                                            accs[s % ACCS], 0, 0, 0);
   }
+#pragma unroll
+  for (int h = ACCS / 2; h > 0; h /= 2)
+#pragma unroll
+    for (int i = 0; i < h; ++i) accs[i] = accs[i] + accs[i + h];
+  const v16f acc = accs[0];
 
   // Waves' blocks [wave][r][lane] in LDS (over the rings, once every wave is
   // done with them), summed in wave order.  Thread t owns row t / 8 of the
@@ -1437,13 +1451,17 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_thin_rows(RowsArgs g)
     v[q] = s;
   }
   if (row >= g.m) return;
-  float* out = g.c + int64_t(row) * g.ldc;
+  const bool partial = gridDim.y > 1;
+  float* out = partial ? g.c + (int64_t(blockIdx.y) * g.m + row) * g.n
+                       : g.c + int64_t(row) * g.ldc;
   const int col = n0 + c4;
-  if (g.vec_out) {
+  const bool acc_out = !partial && g.accumulate;
+  const float* bias = partial ? nullptr : g.bias;
+  if (partial ? g.n % 4 == 0 : g.vec_out != 0) {
     if (col < g.n) {
       v4f* o = reinterpret_cast<v4f*>(out + col);
-      if (g.accumulate) *o = *o + v;
-      else if (g.bias) *o = lin_epi4(v, *reinterpret_cast<const v4f*>(g.bias + col), g.relu);
+      if (acc_out) *o = *o + v;
+      else if (bias) *o = lin_epi4(v, *reinterpret_cast<const v4f*>(bias + col), g.relu);
       else *o = v;
     }
     return;
@@ -1452,8 +1470,8 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_thin_rows(RowsArgs g)
   for (int q = 0; q < 4; ++q) {
     if (col + q < g.n) {
       float* o = out + col + q;
-      if (g.accumulate) *o = *o + v[q];
-      else *o = g.bias ? lin_epi(v[q], g.bias[col + q], g.relu) : v[q];
+      if (acc_out) *o = *o + v[q];
+      else *o = bias ? lin_epi(v[q], bias[col + q], g.relu) : v[q];
     }
   }
 }
@@ -1803,9 +1821,12 @@ int launch_short(Runtime* rt, GemmArgs g, bool* colsum_done) {
   return LMP_OK;
 }
 
-// M <= 32 with B transposed on the whole-rows kernel: one workgroup per 32
-// columns, no split of K.
-int launch_rows(Runtime* rt, const GemmArgs& g0) {
+// M <= 32 with B transposed on the rows kernel: one workgroup per 32 columns
+// and K split.  A CU holds one workgroup, so the split count is the one whose
+// rounds of workgroups take the fewest tile steps: a step of the whole chip
+// (4 MiB of B) is about 1 us, as are a round's start and end, and folding
+// partials costs about 4.
+int launch_rows(Runtime* rt, const GemmArgs& g0, const Workspace& ws) {
   RowsArgs r{};
   r.a = g0.a;
   r.b = g0.b;
@@ -1820,16 +1841,54 @@ int launch_rows(Runtime* rt, const GemmArgs& g0) {
   r.bias = g0.bias;
   r.relu = g0.relu;
   r.vec_out = g0.vec_out;
-  const dim3 grid{uint32_t((g0.n + 31) / 32), 1u, 1u};
-  hipLaunchKernelGGL(gemm_thin_rows<kRowsStages>, grid, dim3(64 * kRowsWaves), 0, rt->stream, r);
+  constexpr int kGrain = 32 * kRowsWaves;
+  const int64_t blocks = (int64_t(g0.n) + 31) / 32;
+  const int64_t k_tiles = (int64_t(g0.k) + kGrain - 1) / kGrain;  // a wave's tiles, unsplit
+  int64_t per = k_tiles, best = INT64_MAX;
+  const int64_t max_splits =
+      std::max<int64_t>(1, std::min<int64_t>(k_tiles / 2, 2 * rt->cu_count / blocks));
+  for (int64_t s = 1; s <= max_splits; ++s) {
+    const int64_t steps = (k_tiles + s - 1) / s;
+    const int64_t rounds = (blocks * s + rt->cu_count - 1) / rt->cu_count;
+    const int64_t cost = rounds * (steps + 1) + (s > 1 ? 4 : 0);
+    if (cost < best) {
+      best = cost;
+      per = steps;
+    }
+  }
+  const int splits = int((k_tiles + per - 1) / per);
+  r.k_per_wg = int(per) * kGrain;
+  float* part = nullptr;
+  if (splits > 1) {
+    const int wrc = ws.take(size_t(splits) * size_t(g0.m) * size_t(g0.n) * sizeof(float), &part);
+    if (wrc != LMP_OK) return wrc;
+    r.c = part;
+  }
+  const dim3 grid{uint32_t(blocks), uint32_t(splits), 1u};
+  // Eight sums per element where the direct kernel's shorter chains ran before
+  // (its error is the bound: 32 x 6000 x 3000 2.1e-7 there, 2.5e-7 with four
+  // sums, 1.8e-7 with eight); four where every CU has whole rows (5.7e-7 ->
+  // 2.9e-7 at 32 x 8192 x 4096; eight would cost 1-3% there).
+  if (blocks < rt->cu_count)
+    hipLaunchKernelGGL((gemm_thin_rows<kRowsStages, 8>), grid, dim3(64 * kRowsWaves), 0,
+                       rt->stream, r);
+  else
+    hipLaunchKernelGGL((gemm_thin_rows<kRowsStages, 4>), grid, dim3(64 * kRowsWaves), 0,
+                       rt->stream, r);
   LMP_LAUNCH_CHECK("gemm_thin_rows");
+  if (splits > 1) {
+    const int frc = launch_fold(rt, g0.c, part, g0.m, g0.n, g0.ldc, splits, g0.accumulate,
+                                g0.bias, g0.relu);
+    ws.give(part);  // stream-ordered: the fold reads it first
+    if (frc != LMP_OK) return frc;
+  }
   return LMP_OK;
 }
 
 // Kernel choice (measured on MI355X), in order: the tiny kernel for small
 // latency-bound products (K <= 512, at most 2^21 multiply-adds); the
-// persistent short-K kernel (A transposed, K <= 32); whole rows of B per
-// workgroup (M <= 32, B transposed, a 32-column block per CU); the
+// persistent short-K kernel (A transposed, K <= 32); rows of B per
+// workgroup (M <= 32, B transposed, K split when 32-column blocks leave CUs idle); the
 // register-direct kernel (M <= 32); the bf16 matrix cores (bf3_ok below, tiles
 // and split of K by bf3_plan); then the fp32 MFMAs: 32 x 256 tiles (M <= 64)
 // and, with 16-byte operand rows, the LDS-DMA configurations (256 x 256 when
@@ -1853,10 +1912,9 @@ Route gemm_route_f32(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok) {
     if (vec && g.vec_out && g.k <= kBK && short_tiles <= 0x7fffffff)
       return Route::Short;
   }
-  // M <= 32 with B transposed and a 32-column block for every CU: whole rows
-  // of B per workgroup, no split (config 3's dX: 46 -> 31-35 us cold).
+  // M <= 32 with B transposed: rows of B per workgroup.
   if constexpr (!TA && TB) {
-    if (direct_ok && g.m <= 32 && (g.n + 31) / 32 >= rt->cu_count) return Route::Rows;
+    if (direct_ok && g.m <= 32) return Route::Rows;
   }
   if (direct_ok && g.m <= 32) return Route::Direct;
   if (g.m <= 64) return Route::Skinny;
@@ -1912,10 +1970,12 @@ int launch_gemm(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok, const 
       if (g.colsum && colsum_done) *colsum_done = true;
       return launch_tiny<TA, TB>(rt, g);
     case Route::Short: return launch_short(rt, g, colsum_done);
-    case Route::Rows: return launch_rows(rt, g);
-    // With B transposed a wave's loads touch more cache lines per byte, so
-    // three fragments in flight instead of two.
-    case Route::Direct: return launch_direct<TA, TB, TB ? 3 : 2>(rt, g, ws);
+    case Route::Rows: return launch_rows(rt, g, ws);
+    // With B transposed (and A) a wave's loads touch more cache lines per byte,
+    // so three fragments in flight instead of two.
+    case Route::Direct:
+      if constexpr (TA || !TB) return launch_direct<TA, TB, TB ? 3 : 2>(rt, g, ws);
+      break;
     case Route::Bf3: return launch_bf3_planned<TA, TB>(rt, g, ws, colsum_done);
     case Route::Skinny: return launch_gemm_cfg<CfgSkinny, TA, TB>(rt, g, vec, ws);
     case Route::Small64: return launch_gemm_cfg<CfgSmall, TA, TB>(rt, g, vec, ws, 1);
