@@ -225,7 +225,9 @@ RowPlan row_plan(const Region& r) {
   p.N = static_cast<int64_t>(p.S.back());
   if (p.N < 2) return p;
   p.R = static_cast<int64_t>(shape_numel(p.S)) / p.N;
-  if (p.R > (int64_t(1) << 31)) return p;  // one wave per row, one-shot grid
+  // One wave, or for long rows four, per row in a one-shot grid of fewer than
+  // 2^32 threads.
+  if (p.R > int64_t(0xffffffffll) / (p.N < 2048 ? 64 : 256)) return p;
   std::vector<size_t> S1 = p.S;
   S1.back() = 1;
   for (TensorImpl* n : r.nodes) {
@@ -1166,12 +1168,12 @@ struct Job {
   Storage out{0, DeviceType::HIP};  // empty until prepare() allocates or takes a target
   std::vector<Storage> extra;
   // One lane per unit (vec, quad: one-shot), one workgroup per row, or one
-  // lane per element (grid-stride loop, one-shot up to 2^30 workgroups).
+  // lane per element (grid-stride loop, one-shot below 2^32 threads).
   uint64_t blocks() const {
     if (rp.ok) return uint64_t(rp.R);
     const uint64_t work = p.vec || p.quad ? p.nvec : p.n;
     const uint64_t grid = (work + kBlock - 1) / kBlock;
-    return std::max<uint64_t>(1, std::min<uint64_t>(grid, uint64_t(1) << 30));
+    return std::max<uint64_t>(1, std::min<uint64_t>(grid, 0xffffffffull / kBlock));
   }
   uint64_t group_blocks() const { return std::max<uint64_t>(1, (p.nvec + kBlock - 1) / kBlock); }
   int threads() const { return rp.ok ? rp.lanes : kBlock; }

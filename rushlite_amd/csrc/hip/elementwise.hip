@@ -35,7 +35,7 @@ namespace {
 // over [8192,8192] 176.2 -> 171.8 us, six eager ops 491.6 -> 476.8 us).
 constexpr int kBlock = 64;
 // Streaming kernels index float4s with 32 bits; one-shot grids need
-// nvec / kBlock workgroups, below the 2^30 cap of grid_for for nvec < 2^31.
+// nvec / kBlock workgroups, below the cap of grid_for for nvec < 2^31.
 constexpr uint64_t kMaxVec = 0x7fffffffull;
 
 // ------------------------------------------------------------ shape helpers
@@ -70,12 +70,12 @@ Coalesced coalesce(const lmp_bcast& d) {
   return c;
 }
 
-// One workgroup per `per_block` work items (one-shot), capped at 2^30
-// workgroups; kernels keep a grid-stride loop only for sizes past the cap.
+// One workgroup per `per_block` work items (one-shot), capped at what a grid
+// holds; kernels keep a grid-stride loop only for sizes past the cap.
 int grid_for(int64_t work_items, int per_block) {
   int64_t g = (work_items + per_block - 1) / per_block;
   if (g < 1) g = 1;
-  return static_cast<int>(std::min<int64_t>(g, int64_t(1) << 30));
+  return static_cast<int>(std::min<int64_t>(g, int64_t(kMaxGridThreads / uint64_t(per_block))));
 }
 
 bool aligned16(const void* p) {

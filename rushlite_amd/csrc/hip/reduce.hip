@@ -516,6 +516,18 @@ int reduce_rows_as(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len
 
 template <int OP, typename T>
 int reduce_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len) {
+  // A wave (long rows: a workgroup) per row, 2^31 threads a launch at most.
+  if ((rows + kWaves - 1) / kWaves > 0x7fffffffull)
+    return fail(LMP_ERR_UNSUPPORTED, "reduce: too many rows");
+  const uint64_t most = uint64_t(1) << (len >= kLongRow ? 23 : 25);
+  if (rows > most) {
+    const uint64_t launches = (rows + most - 1) / most, per = (rows + launches - 1) / launches;
+    for (uint64_t r = 0; r < rows; r += per) {
+      const int rc = reduce_rows<OP, T>(rt, out + r, in + r * len, std::min(per, rows - r), len);
+      if (rc != LMP_OK) return rc;
+    }
+    return LMP_OK;
+  }
   // Short float64 rows stay in units of one value, as the fused row kernels
   // take them.
   bool done = false;
@@ -524,7 +536,6 @@ int reduce_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len) {
                       : reduce_rows_as<OP, T, 1>(rt, out, in, rows, len, &done);
   if (done) return rc;
   const uint64_t blocks = (rows + kWaves - 1) / kWaves;
-  if (blocks > 0x7fffffffull) return fail(LMP_ERR_UNSUPPORTED, "reduce: too many rows");
   if constexpr (std::is_same_v<T, float>) {
     if (len % 4 == 0 && aligned16(in) && len / 4 <= kMaxU32Extent) {
       hipLaunchKernelGGL((row_reduce_wave_f32<OP>), dim3(uint32_t(blocks)), dim3(kBlock), 0,
@@ -536,6 +547,18 @@ int reduce_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len) {
   hipLaunchKernelGGL((row_reduce_wave<OP, T>), dim3(uint32_t(blocks)),
                      dim3(kBlock), 0, rt->stream, out, in, rows, len);
   LMP_LAUNCH_CHECK("row_reduce_wave");
+  return LMP_OK;
+}
+
+// One lane per output element, grid-striding, the axis folded in row order.
+template <int OP, typename T>
+int reduce_cols_flat(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t len,
+                     uint64_t inner) {
+  const uint64_t cap = uint64_t(rt->cu_count) * 64;
+  const uint64_t blocks = std::min<uint64_t>((outer * inner + kBlock - 1) / kBlock, cap);
+  hipLaunchKernelGGL((col_reduce_flat<OP, T>), dim3(uint32_t(blocks)), dim3(kBlock), 0, rt->stream,
+                     out, in, outer, len, inner);
+  LMP_LAUNCH_CHECK("col_reduce_flat");
   return LMP_OK;
 }
 
@@ -551,7 +574,7 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
   // the axis is short ([4096, 64, 33] fp32: 7.0 us, 7.6 us in strips; float64
   // 15.3 and 12.2).
   if ((len * units <= 128 || (n >= cus * 2 * kBlock && units * kUnit >= 128 && len <= 64 && kUnit == 4)) &&
-      n <= uint64_t(0x7fffffff) * kBlock) {
+      n <= kMaxGridThreads - kBlock) {
     hipLaunchKernelGGL((col_reduce_lane<OP, T, V>), dim3(blocks_for(n)), dim3(kBlock), 0,
                        rt->stream, out, in, n, uint32_t(units), uint32_t(len));
     LMP_LAUNCH_CHECK("col_reduce_lane");
@@ -588,7 +611,8 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
   const uint64_t chunk = (len + S - 1) / S;
   S = (len + chunk - 1) / chunk;
   const uint64_t blocks = strips * outer * S;
-  if (blocks > 0x7fffffffull) return fail(LMP_ERR_UNSUPPORTED, "reduce: too many columns");
+  if (blocks > kMaxGridThreads / kBlock)
+    return reduce_cols_flat<OP, T>(rt, out, in, outer, len, inner);
   T* dst = out;
   T* tmp = nullptr;
   if (S > 1) {
@@ -630,15 +654,8 @@ int reduce_cols(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t len,
   const uint64_t units = pack ? inner / kPackOf<T> : inner;
   if (units > kMaxU32Extent || len > kMaxU32Extent || outer > 65535) {
     // Extents past the tile kernel's 32-bit counters, and more than 65535
-    // outer slices: one lane per output element, grid-striding, the axis
-    // folded in row order.
-    const uint64_t n = outer * inner;
-    const uint64_t cap = uint64_t(rt->cu_count) * 64;
-    const uint64_t blocks = std::min<uint64_t>((n + kBlock - 1) / kBlock, cap);
-    hipLaunchKernelGGL((col_reduce_flat<OP, T>), dim3(uint32_t(blocks)), dim3(kBlock), 0,
-                       rt->stream, out, in, outer, len, inner);
-    LMP_LAUNCH_CHECK("col_reduce_flat");
-    return LMP_OK;
+    // outer slices.
+    return reduce_cols_flat<OP, T>(rt, out, in, outer, len, inner);
   }
   return pack ? reduce_cols_as<OP, T, kPackOf<T>>(rt, out, in, outer, len, inner)
               : reduce_cols_as<OP, T, 1>(rt, out, in, outer, len, inner);
