@@ -355,9 +355,11 @@ __global__ __launch_bounds__(kBlock) void col_reduce_tile(T* __restrict__ dst,
       for (int u = 0; u < kColUnroll - 1; ++u) acc[u] = combine_pack<OP>(acc[u], x[u]);
     }
   }
-  P a = acc[0];
 #pragma unroll
-  for (int u = 1; u < kColUnroll; ++u) a = combine_pack<OP>(a, acc[u]);
+  for (int w = kColUnroll / 2; w >= 1; w /= 2)
+#pragma unroll
+    for (int u = 0; u < w; ++u) acc[u] = combine_pack<OP>(acc[u], acc[u + w]);
+  P a = acc[0];
   __shared__ P lds[kBlock];
   lds[threadIdx.x] = a;
   for (uint32_t n = rg; n > 1;) {
