@@ -237,8 +237,9 @@ int lmp_k_reduce(int op, int dtype, void* out, const void* in, size_t outer,
 
 /* ----------------------------------------------------------------- matrix */
 
-/* C[m,n] (+)= op(A)[m,k] * op(B)[k,n], row-major, fp32, fp32 MFMA
- * accumulation.  trans_a != 0 means A is stored [k,m] (lda >= m); trans_b != 0
+/* C[m,n] (+)= op(A)[m,k] * op(B)[k,n], row-major, fp32 with fp32
+ * accumulation (fp32 MFMAs, or bf16 MFMAs on operands split into three bf16
+ * parts, no less exact; infinities, NaN and overflow as fp32 products).  trans_a != 0 means A is stored [k,m] (lda >= m); trans_b != 0
  * means B is stored [n,k] (ldb >= k).  accumulate != 0 adds into C.
  * Replaces matmul_cuda -> cudaMatMul (kernels.cu:83-110, matrix.cu:21-199);
  * the transposed forms replace the transpose-then-matmul pairs of
@@ -286,9 +287,9 @@ int lmp_k_linear_f32(int trans_a, int trans_b, size_t m, size_t n, size_t k,
  * together.  LinearBackward in the reference computes them apart: the bias
  * through AddBackward's grad-of-broadcast reduction (grad_utils.cpp:10-36)
  * and the weight through transpose + matmul (functions/matrix_ops.cpp:15-20).
- * The column sums ride in the GEMM's own launch on the tiny kernel (K <= 512,
- * at most 2^21 multiply-adds), on the LDS tiles when B is untransposed and K
- * is not split, and on the short-K kernel (A transposed, K <= 32); otherwise
+ * The column sums ride in the GEMM's own launches on the tiny kernel (K <= 512,
+ * at most 2^21 multiply-adds), on the bf16 matrix cores when B is untransposed,
+ * on the fp32 LDS tiles when K is not split, and on the short-K kernel (A transposed, K <= 32); otherwise
  * a second launch forms them after the GEMM (the dim-0 reduction for a
  * contiguous B, a strided column sum for any ldb).  Anything the second launch
  * needs is reserved before the first, so an error return leaves C and colsum
@@ -325,8 +326,9 @@ int lmp_k_gemm_colsum_masked_f32(int trans_a, size_t m, size_t n, size_t k,
  * grad_utils.cpp:10-36): two transposes, two matmuls and a reduction.  When
  * both products fit the tiny GEMM's 16 x 16 blocks (K <= 512, at most 2^21
  * multiply-adds, blocks of 32 x 32 short of a quarter of the CUs) they run as
- * one launch; otherwise lmp_k_gemm_colsum_f32 (dw, db) then lmp_k_gemm_f32
- * (dx).  Either way the same bits as those two calls.  Argument errors are
+ * one launch, and so do products that both take the bf16 matrix cores with one
+ * workgroup size; otherwise lmp_k_gemm_colsum_f32 (dw, db) then
+ * lmp_k_gemm_f32 (dx).  Either way the same bits as those two calls.  Argument errors are
  * returned before anything is written; after the first of the two calls only
  * running out of device memory can fail, which leaves dx unwritten. */
 int lmp_k_linear_backward_f32(size_t batch, size_t in, size_t out, const float* x, size_t ldx,
