@@ -8,6 +8,7 @@
 #include <string>
 
 #include "fastdiv.hpp"
+#include "gemm_plan.hpp"
 #include "lmp_hip.h"
 
 namespace lmp_hip {
@@ -58,11 +59,6 @@ constexpr uint64_t kStreamStoreBytes = uint64_t(128) << 20;
 // that every tile origin, fragment index and K-loop step (an extent plus at
 // most a few thousand) still fits the kernels' int arithmetic.
 constexpr size_t kGemmMaxExtent = (size_t(1) << 31) - 4096;
-
-// A grid holds fewer than 2^32 threads per dimension: a dispatch counts them in
-// 32 bits, and a longer one-shot launch comes out as what is left modulo 2^32
-// (2^33 + 64 threads as a single wave).
-constexpr uint64_t kMaxGridThreads = 0xffffffffull;
 
 // Scratch allocation for kernels that need a workspace (split-K partials,
 // two-pass reductions).  Memory comes from the pool and is returned to it

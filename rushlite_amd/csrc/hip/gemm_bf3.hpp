@@ -58,7 +58,6 @@ typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBf3K = 16;                               // k values per step
 constexpr float kBf3Scale = 16777216.0f;                // 2^24, on each operand
 constexpr float kBf3Unscale = 3.552713678800501e-15f;   // 2^-48, on the result
 
@@ -595,58 +594,17 @@ using Bf3Mid = Bf3Cfg<4, 2, 1, 2, 2, 1>;     // 128 x 128, 8 waves of 32 x 64
 using Bf3Flat = Bf3Cfg<1, 4, 2, 1, 2, 2>;    // 64 x 128, 4 waves of 64 x 32
 using Bf3Small = Bf3Cfg<2, 2, 1, 1, 2, 2>;   // 64 x 64, 4 waves of 32 x 32
 
-struct Bf3Plan {
-  int cfg = 0;  // index into kBf3Tiles
-  int splits = 1;
-};
+// kBf3Tiles is what these types are.
+template <class C>
+constexpr bool bf3_is(int cfg) {
+  return kBf3Tiles[cfg].bm == C::BM && kBf3Tiles[cfg].bn == C::BN &&
+         kBf3Tiles[cfg].threads == C::THREADS;
+}
+static_assert(bf3_is<Bf3Big>(0) && bf3_is<Bf3Wide>(1) && bf3_is<Bf3Mid>(2) &&
+              bf3_is<Bf3Flat>(3) && bf3_is<Bf3Small>(4));
 
-// Time of one 16-wide k step of a workgroup, in us: `alone` on its CU, and
-// `shared` per workgroup where several take turns (medians of a sweep of 25
-// shapes, random operands, on one MI355X).  A larger tile moves and splits
-// each value fewer times: 4096^3 takes 574, 637, 700, 792 and about 980 us on
-// the five, 512 x 1000 x 4096 (K split) 44.0, 34.4, 34.4, 36.7, 39.4 and
-// 256 x 1024 x 1024 25.9, 19.8, 15.9, 14.5, 13.7.
-struct Bf3Tile {
-  int bm, bn;
-  float alone, shared;
-};
-constexpr Bf3Tile kBf3Tiles[] = {{256, 256, 2.2f, 2.2f},
-                                 {256, 128, 1.25f, 1.25f},
-                                 {128, 128, 0.69f, 0.68f},
-                                 {64, 128, 0.42f, 0.39f},
-                                 {64, 64, 0.34f, 0.235f}};
-
-// Tiles and split of K with the least modelled time: workgroups go round the
-// CUs, each takes 4.5 us besides its steps (first loads, C), and a split costs
-// a second launch (2 us) and a round trip of the partials (5 TB/s).  The
-// partials stay within the fixed workspace whichever entry point is called, so
-// that all of them give the same bits; a split keeps at least 64 k.
 Bf3Plan bf3_plan(Runtime* rt, const GemmArgs& g) {
-  const int64_t steps = (g.k + kBf3K - 1) / kBf3K, mn = int64_t(g.m) * g.n;
-  const int64_t most =
-      std::min<int64_t>(std::max<int64_t>(1, steps / 4),
-                        int64_t(LMP_NOALLOC_SCRATCH_BYTES) / int64_t(sizeof(float)) /
-                            (mn + g.n + 8));  // room for column sums, asked for or not
-  Bf3Plan plan;
-  float best = 0.0f;
-  for (int c = 0; c < 5; ++c) {
-    const Bf3Tile& t = kBf3Tiles[c];
-    const int64_t tiles = int64_t((g.m + t.bm - 1) / t.bm) * ((g.n + t.bn - 1) / t.bn);
-    for (int s : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
-      if (s > 1 && s > most) break;
-      const float load = float((tiles * s + rt->cu_count - 1) / rt->cu_count);
-      const float per_step = std::max(t.alone, load * t.shared);
-      float us = 4.5f + float((steps + s - 1) / s) * per_step;
-      if (s > 1) us += 2.0f + float(s + 1) * float(mn) * (4.0f / 5e6f);
-      if (best == 0.0f || us < best) {
-        best = us;
-        plan.cfg = c;
-        plan.splits = s;
-      }
-      if (tiles * s > 8 * int64_t(rt->cu_count)) break;  // more splits only add partials
-    }
-  }
-  return plan;
+  return lmp_hip::bf3_plan(rt->cu_count, int64_t(LMP_NOALLOC_SCRATCH_BYTES), g.m, g.n, g.k);
 }
 
 // Calls f with the configuration's type.
@@ -721,17 +679,23 @@ int launch_bf3_as(Runtime* rt, GemmArgs g, const Bf3Plan& plan, const Workspace&
 template <bool TA, bool TB>
 int launch_bf3_planned(Runtime* rt, GemmArgs g, const Workspace& ws, bool* colsum_done) {
   if (TB) g.colsum = nullptr;  // the sums ride where B's rows run along n
+  const Bf3Plan plan = bf3_plan(rt, g);
+  if (plan.cfg < 0) return fail(LMP_ERR_UNSUPPORTED, "gemm: more tiles than a grid holds");
   if (g.colsum && colsum_done) *colsum_done = true;
-  return launch_bf3_as<TA, TB>(rt, g, bf3_plan(rt, g), ws);
+  return launch_bf3_as<TA, TB>(rt, g, plan, ws);
 }
 
 // A weight gradient (A transposed, with its column sums) and an input gradient
 // (B transposed) as one launch and, where either is split, one fold; false,
-// with nothing launched, if their workgroups differ in size.
+// with nothing launched, if their workgroups differ in size or are more than a
+// grid holds.
 bool launch_bf3_pair_planned(Runtime* rt, const GemmArgs& gw, const GemmArgs& gx, int* rc) {
   const Bf3Plan pw = bf3_plan(rt, gw), px = bf3_plan(rt, gx);
-  if ((pw.cfg <= 2) != (px.cfg <= 2)) return false;
+  if (pw.cfg < 0 || px.cfg < 0) return false;
+  const int threads = kBf3Tiles[pw.cfg].threads;
+  if (kBf3Tiles[px.cfg].threads != threads) return false;
   Bf3Args w = bf3_args(gw, pw), x = bf3_args(gx, px);
+  if (!bf3_pair_fits(bf3_workgroups(w), bf3_workgroups(x), threads)) return false;
   const Workspace ws{};
   if ((*rc = bf3_take_partials(w, ws)) != LMP_OK) return true;
   if ((*rc = bf3_take_partials(x, ws)) != LMP_OK) {

@@ -1,0 +1,84 @@
+// How the fp32 GEMMs are cut into workgroups: host code without HIP includes.
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+#include <iterator>
+
+namespace lmp_hip {
+
+// A grid holds fewer than 2^32 threads per dimension: a dispatch counts them in
+// 32 bits, and a longer one-shot launch comes out as what is left modulo 2^32
+// (2^33 + 64 threads as a single wave).
+constexpr uint64_t kMaxGridThreads = 0xffffffffull;
+
+// ---------------------------------------------- products on the bf16 matrix cores
+
+constexpr int kBf3K = 16;  // k values per step
+
+struct Bf3Plan {
+  int cfg = -1;  // index into kBf3Tiles; -1: no launch fits a grid
+  int splits = 1;
+};
+
+// Time of one 16-wide k step of a workgroup, in us: `alone` on its CU, and
+// `shared` per workgroup where several take turns (medians of a sweep of 25
+// shapes, random operands, on one MI355X).  A larger tile moves and splits
+// each value fewer times: 4096^3 takes 574, 637, 700, 792 and about 980 us on
+// the five, 512 x 1000 x 4096 (K split) 44.0, 34.4, 34.4, 36.7, 39.4 and
+// 256 x 1024 x 1024 25.9, 19.8, 15.9, 14.5, 13.7.
+struct Bf3Tile {
+  int bm, bn, threads;
+  float alone, shared;
+};
+constexpr Bf3Tile kBf3Tiles[] = {{256, 256, 512, 2.2f, 2.2f},
+                                 {256, 128, 512, 1.25f, 1.25f},
+                                 {128, 128, 512, 0.69f, 0.68f},
+                                 {64, 128, 256, 0.42f, 0.39f},
+                                 {64, 64, 256, 0.34f, 0.235f}};
+
+inline int64_t bf3_tiles(const Bf3Tile& t, int64_t m, int64_t n) {
+  return ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+}
+
+// Tiles and split of K with the least modelled time: workgroups go round the
+// CUs, each takes 4.5 us besides its steps (first loads, C), and a split costs
+// a second launch (2 us) and a round trip of the partials (5 TB/s).  The
+// partials stay within `scratch` bytes, the fixed workspace, whichever entry
+// point is called, so that all of them give the same bits; a split keeps at
+// least 64 k.  Launches that a grid cannot hold are left out.
+inline Bf3Plan bf3_plan(int64_t cus, int64_t scratch, int64_t m, int64_t n, int64_t k) {
+  const int64_t steps = (k + kBf3K - 1) / kBf3K, mn = m * n;
+  const int64_t most =
+      std::min<int64_t>(std::max<int64_t>(1, steps / 4),
+                        scratch / int64_t(sizeof(float)) /
+                            (mn + n + 8));  // room for column sums, asked for or not
+  Bf3Plan plan;
+  float best = 0.0f;
+  for (int c = 0; c < int(std::size(kBf3Tiles)); ++c) {
+    const Bf3Tile& t = kBf3Tiles[c];
+    const int64_t tiles = bf3_tiles(t, m, n);
+    for (int s : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+      if (s > 1 && s > most) break;
+      if (uint64_t(tiles) * uint64_t(s) > kMaxGridThreads / uint64_t(t.threads)) break;
+      const float load = float((tiles * s + cus - 1) / cus);
+      const float per_step = std::max(t.alone, load * t.shared);
+      float us = 4.5f + float((steps + s - 1) / s) * per_step;
+      if (s > 1) us += 2.0f + float(s + 1) * float(mn) * (4.0f / 5e6f);
+      if (plan.cfg < 0 || us < best) {
+        best = us;
+        plan.cfg = c;
+        plan.splits = s;
+      }
+      if (tiles * s > 8 * cus) break;  // more splits only add partials
+    }
+  }
+  return plan;
+}
+
+// Whether two planned products of `a` and `b` workgroups fit one grid.
+inline bool bf3_pair_fits(uint64_t a, uint64_t b, int threads) {
+  return a + b <= kMaxGridThreads / uint64_t(threads);
+}
+
+}  // namespace lmp_hip

@@ -1,0 +1,59 @@
+// Host-only checks of how the fp32 GEMMs are cut into workgroups.  Built and run
+// by tests/test_gemm_plan.py with g++; no GPU involved.
+#include <cstdio>
+
+#include "gemm_plan.hpp"
+
+using namespace lmp_hip;
+
+#define CHECK(c)                                                  \
+  do {                                                            \
+    if (!(c)) {                                                   \
+      std::printf("FAIL %s:%d %s\n", __FILE__, __LINE__, #c);     \
+      return 1;                                                   \
+    }                                                             \
+  } while (0)
+
+constexpr int64_t kTop = (int64_t(1) << 31) - 4097;  // the largest extent a GEMM takes
+constexpr int64_t kScratch = int64_t(32) << 20;
+
+// Every launch of the bf16 path has fewer than 2^32 threads, at any extents.
+int bf3_grids() {
+  const int64_t ms[] = {33, 512, 4096, int64_t(1) << 24, (int64_t(1) << 30) - 64, int64_t(1) << 30,
+                        (int64_t(1) << 30) + 64, kTop - 255, kTop};
+  const int64_t ns[] = {1, 64, 65, 128, 129, 4096};
+  for (int64_t m : ms)
+    for (int64_t n : ns)
+      for (int64_t k : {int64_t(33), int64_t(48), int64_t(1000), int64_t(1) << 20})
+        for (int flip = 0; flip < 2; ++flip) {
+          const int64_t a = flip ? n : m, b = flip ? m : n;
+          const Bf3Plan p = bf3_plan(256, kScratch, a, b, k);
+          if (p.cfg < 0) {  // only where no tile fits a grid
+            for (const Bf3Tile& t : kBf3Tiles)
+              CHECK(bf3_tiles(t, a, b) * t.threads > int64_t(kMaxGridThreads));
+            continue;
+          }
+          const Bf3Tile& t = kBf3Tiles[p.cfg];
+          CHECK(bf3_tiles(t, a, b) * p.splits * t.threads <= int64_t(kMaxGridThreads));
+        }
+  // What memory can hold is served: 2^30 + 64 rows of one column (33 values of k
+  // each), and the longest extent with up to a tile of the other.
+  CHECK(bf3_plan(256, kScratch, (int64_t(1) << 30) + 64, 1, 33).cfg >= 0);
+  CHECK(bf3_plan(256, kScratch, kTop, 64, 33).cfg >= 0);
+  CHECK(bf3_plan(256, kScratch, 64, kTop, 33).cfg >= 0);
+  return 0;
+}
+
+// Two products share a launch only where their workgroups together fit a grid.
+int bf3_pairs() {
+  CHECK(bf3_pair_fits(1, 1, 512));
+  const uint64_t most = kMaxGridThreads / 256;
+  CHECK(bf3_pair_fits(most - 5, 5, 256) && !bf3_pair_fits(most - 5, 6, 256));
+  return 0;
+}
+
+int main() {
+  if (bf3_grids() || bf3_pairs()) return 1;
+  std::printf("gemm plans ok\n");
+  return 0;
+}
