@@ -517,7 +517,6 @@ __device__ __forceinline__ int direct_row(int r, int lh) {
   return (r / 4) * 8 + lh * 4 + (r % 4);
 }
 
-constexpr int kDirectWaves = 4;
 
 template <bool TA, bool TB, int STAGES>
 __global__ __launch_bounds__(64 * kDirectWaves)
@@ -532,7 +531,7 @@ void gemm_direct(DirectArgs g) {
   const int n0 = int(blockIdx.x % g.n_blocks) * kDirectN;
   const int part = g.k_per_wg / KW;
   const int kb = int(blockIdx.y) * g.k_per_wg + wave * part;
-  const int ke = min(g.k, kb + part);
+  const int ke = k_range_end(kb, part, g.k);
 
   v16f acc[4];
 #pragma unroll
@@ -1346,7 +1345,6 @@ struct RowsArgs {
   int k_per_wg;       // K range of one workgroup (a multiple of 32 * kRowsWaves)
 };
 
-constexpr int kRowsWaves = 4;
 constexpr int kRowsStages = 3;
 constexpr int kRowsTile = 32 * 32;  // floats of one operand tile
 
@@ -1360,7 +1358,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_thin_rows(RowsArgs g)
   const int n0 = int(blockIdx.x) * 32;
   const int part = g.k_per_wg / kRowsWaves;
   const int kb = int(blockIdx.y) * g.k_per_wg + wave * part;
-  const int ke = min(g.k, kb + part);
+  const int ke = k_range_end(kb, part, g.k);
   const int ntiles = kb < ke ? (ke - kb + 31) / 32 : 0;
   const int rot = ntiles ? int((blockIdx.x * 13u) % uint32_t(ntiles)) : 0;
   float* ring = smem + wave * STAGES * STAGE;
@@ -1764,12 +1762,9 @@ int launch_direct(Runtime* rt, const GemmArgs& g0, const Workspace& ws, int spli
   d.bias = g0.bias;
   d.relu = g0.relu;
   d.n_blocks = (g0.n + kDirectN - 1) / kDirectN;
-  constexpr int kGrain = 8 * kDirectWaves;
-  const int max_splits = std::max(1, g0.k / (64 * kDirectWaves));
-  if (splits <= 0) splits = (rt->cu_count + d.n_blocks - 1) / d.n_blocks;
-  splits = std::max(1, std::min(splits, max_splits));
-  d.k_per_wg = ((g0.k + splits - 1) / splits + kGrain - 1) / kGrain * kGrain;
-  splits = (g0.k + d.k_per_wg - 1) / d.k_per_wg;
+  const KSplit ks = direct_split(rt->cu_count, d.n_blocks, g0.k, splits);
+  d.k_per_wg = ks.per_wg;
+  splits = ks.splits;
   float* part = nullptr;
   if (splits > 1) {
     const int wrc = ws.take(size_t(splits) * size_t(g0.m) * size_t(g0.n) * sizeof(float), &part);
@@ -1822,10 +1817,7 @@ int launch_short(Runtime* rt, GemmArgs g, bool* colsum_done) {
 }
 
 // M <= 32 with B transposed on the rows kernel: one workgroup per 32 columns
-// and K split.  A CU holds one workgroup, so the split count is the one whose
-// rounds of workgroups take the fewest tile steps: a step of the whole chip
-// (4 MiB of B) is about 1 us, as are a round's start and end, and folding
-// partials costs about 4.
+// and K split as rows_split has it.
 int launch_rows(Runtime* rt, const GemmArgs& g0, const Workspace& ws) {
   RowsArgs r{};
   r.a = g0.a;
@@ -1841,23 +1833,10 @@ int launch_rows(Runtime* rt, const GemmArgs& g0, const Workspace& ws) {
   r.bias = g0.bias;
   r.relu = g0.relu;
   r.vec_out = g0.vec_out;
-  constexpr int kGrain = 32 * kRowsWaves;
   const int64_t blocks = (int64_t(g0.n) + 31) / 32;
-  const int64_t k_tiles = (int64_t(g0.k) + kGrain - 1) / kGrain;  // a wave's tiles, unsplit
-  int64_t per = k_tiles, best = INT64_MAX;
-  const int64_t max_splits =
-      std::max<int64_t>(1, std::min<int64_t>(k_tiles / 2, 2 * rt->cu_count / blocks));
-  for (int64_t s = 1; s <= max_splits; ++s) {
-    const int64_t steps = (k_tiles + s - 1) / s;
-    const int64_t rounds = (blocks * s + rt->cu_count - 1) / rt->cu_count;
-    const int64_t cost = rounds * (steps + 1) + (s > 1 ? 4 : 0);
-    if (cost < best) {
-      best = cost;
-      per = steps;
-    }
-  }
-  const int splits = int((k_tiles + per - 1) / per);
-  r.k_per_wg = int(per) * kGrain;
+  const KSplit ks = rows_split(rt->cu_count, g0.n, g0.k);
+  const int splits = ks.splits;
+  r.k_per_wg = ks.per_wg;
   float* part = nullptr;
   if (splits > 1) {
     const int wrc = ws.take(size_t(splits) * size_t(g0.m) * size_t(g0.n) * sizeof(float), &part);

@@ -5,12 +5,67 @@
 #include <cstdint>
 #include <iterator>
 
+#include "fastdiv.hpp"
+
 namespace lmp_hip {
 
 // A grid holds fewer than 2^32 threads per dimension: a dispatch counts them in
 // 32 bits, and a longer one-shot launch comes out as what is left modulo 2^32
 // (2^33 + 64 threads as a single wave).
 constexpr uint64_t kMaxGridThreads = 0xffffffffull;
+
+// ------------------------------------------------------- products of up to 32 rows
+
+// K split over workgroups, `per_wg` values each; a workgroup's `waves` waves take
+// consecutive parts of its range.
+struct KSplit {
+  int splits = 1, per_wg = 0;
+};
+
+// One past the last k of a wave that takes `part` values from `kb` on: at most
+// k, and no more than kb for a wave past the end (kb + part may not fit an int).
+LMP_HD int k_range_end(int kb, int part, int k) {
+  const int left = k - kb;
+  return kb + (part < left ? part : left);
+}
+
+constexpr int kRowsWaves = 4;
+
+// Rows kernel (B transposed, one workgroup per 32 columns).  A CU holds one
+// workgroup, so the split count is the one whose rounds of workgroups take the
+// fewest tile steps: a step of the whole chip (4 MiB of B) is about 1 us, as
+// are a round's start and end, and folding partials costs about 4.
+inline KSplit rows_split(int64_t cus, int64_t n, int64_t k) {
+  constexpr int64_t kGrain = 32 * kRowsWaves;
+  const int64_t blocks = (n + 31) / 32;
+  const int64_t k_tiles = (k + kGrain - 1) / kGrain;  // a wave's tiles, unsplit
+  int64_t per = k_tiles, best = INT64_MAX;
+  const int64_t max_splits =
+      std::max<int64_t>(1, std::min<int64_t>(k_tiles / 2, 2 * cus / blocks));
+  for (int64_t s = 1; s <= max_splits; ++s) {
+    const int64_t steps = (k_tiles + s - 1) / s;
+    const int64_t rounds = (blocks * s + cus - 1) / cus;
+    const int64_t cost = rounds * (steps + 1) + (s > 1 ? 4 : 0);
+    if (cost < best) {
+      best = cost;
+      per = steps;
+    }
+  }
+  return {int((k_tiles + per - 1) / per), int(per * kGrain)};
+}
+
+constexpr int kDirectWaves = 4;
+
+// Register-direct kernel: `splits` workgroups (0: enough for the CUs) of 64 k or
+// more per wave for each of `blocks` column blocks.
+inline KSplit direct_split(int64_t cus, int64_t blocks, int64_t k, int64_t splits) {
+  constexpr int64_t kGrain = 8 * kDirectWaves;
+  const int64_t most = std::max<int64_t>(1, k / (64 * kDirectWaves));
+  if (splits <= 0) splits = (cus + blocks - 1) / blocks;
+  splits = std::max<int64_t>(1, std::min(splits, most));
+  const int64_t per = ((k + splits - 1) / splits + kGrain - 1) / kGrain * kGrain;
+  return {int((k + per - 1) / per), int(per)};
+}
 
 // ---------------------------------------------- products on the bf16 matrix cores
 

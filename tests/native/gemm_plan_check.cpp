@@ -52,8 +52,39 @@ int bf3_pairs() {
   return 0;
 }
 
+// The waves of the kernels for up to 32 rows cover K once: consecutive ranges,
+// none past the end (the last workgroup's may start close to 2^31).
+int covers(const KSplit& s, int waves, int64_t k) {
+  CHECK(s.splits >= 1 && s.per_wg > 0 && s.per_wg % waves == 0);
+  const int part = s.per_wg / waves;
+  int64_t at = 0;
+  for (int y = 0; y < s.splits; ++y)
+    for (int w = 0; w < waves; ++w) {
+      const int64_t kb64 = int64_t(y) * s.per_wg + int64_t(w) * part;
+      CHECK(kb64 < (int64_t(1) << 31));
+      const int kb = int(kb64), ke = k_range_end(kb, part, int(k));
+      if (ke <= kb) continue;  // a wave past the end
+      CHECK(kb == at);
+      at = ke;
+    }
+  CHECK(at == k);
+  return 0;
+}
+
+int thin_ranges() {
+  for (int64_t k : {int64_t(4), int64_t(128), int64_t(388), int64_t(8200), int64_t(1) << 30, kTop - 32768,
+                    kTop - 30000, kTop - 4096, kTop - 4, kTop})
+    for (int64_t n : {int64_t(1), int64_t(32), int64_t(33), int64_t(100), int64_t(1000), int64_t(4098),
+                      int64_t(8192), int64_t(8224), int64_t(100000)})
+      for (int64_t cus : {int64_t(256), int64_t(304), int64_t(64)}) {
+        if (covers(rows_split(cus, n, k), kRowsWaves, k)) return 1;
+        if (covers(direct_split(cus, (n + 127) / 128, k, 0), kDirectWaves, k)) return 1;
+      }
+  return 0;
+}
+
 int main() {
-  if (bf3_grids() || bf3_pairs()) return 1;
+  if (bf3_grids() || bf3_pairs() || thin_ranges()) return 1;
   std::printf("gemm plans ok\n");
   return 0;
 }
