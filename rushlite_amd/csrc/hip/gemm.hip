@@ -1891,11 +1891,13 @@ Route gemm_route_f32(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok) {
     if (vec && g.vec_out && g.k <= kBK && short_tiles <= 0x7fffffff)
       return Route::Short;
   }
-  // M <= 32 with B transposed: rows of B per workgroup.
+  // M <= 32 with B transposed: rows of B per workgroup, while a grid holds one
+  // for every 32 columns.
   if constexpr (!TA && TB) {
-    if (direct_ok && g.m <= 32) return Route::Rows;
+    if (direct_ok && g.m <= 32 && rows_fit(g.n)) return Route::Rows;
+  } else {
+    if (direct_ok && g.m <= 32) return Route::Direct;
   }
-  if (direct_ok && g.m <= 32) return Route::Direct;
   if (g.m <= 64) return Route::Skinny;
   if (vec) {
     const int64_t big_tiles = int64_t((g.m + LdsBig::BM - 1) / LdsBig::BM) *
@@ -2018,22 +2020,23 @@ bool aligned16(const void* p) {
 // sums could not ride in the GEMM.  B untransposed ([k, ldb]): one lane per
 // column, coalesced row by row.  B transposed (stored [n, ldb]): one wave per
 // output, lanes striding over the row, then a butterfly.  256 lanes per
-// workgroup; the grid is ceil(n / 256) or ceil(n / 4) workgroups.
+// workgroup; ceil(n / 256) or ceil(n / 4) workgroups in a grid_2d.
 __global__ __launch_bounds__(256) void colsum_strided_f32(float* __restrict__ out,
                                                           const float* __restrict__ b, int k,
                                                           int n, int ldb, int trans_b,
                                                           int accumulate) {
   // Indices in 64 bits: the last workgroup's lanes reach past n (and a lane's
   // last step past k), which for extents near 2^31 would not fit an int.
+  const int64_t block = int64_t(blockIdx.y) * gridDim.x + blockIdx.x;
   if (!trans_b) {
-    const int64_t j = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t j = block * 256 + threadIdx.x;
     if (j >= n) return;
     float s = 0.0f;
     for (int64_t r = 0; r < k; ++r) s += b[r * int64_t(ldb) + j];
     out[j] = accumulate ? out[j] + s : s;
     return;
   }
-  const int64_t j = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int64_t j = block * 4 + (threadIdx.x >> 6);
   const int lane = int(threadIdx.x & 63);
   if (j >= n) return;  // the whole wave leaves together
   const float* row = b + j * int64_t(ldb);
@@ -2050,7 +2053,8 @@ __global__ __launch_bounds__(256) void transpose_tiled(T* __restrict__ out,
                                                        const T* __restrict__ in,
                                                        int64_t m, int64_t n) {
   __shared__ T tile[64][65];
-  const int64_t r0 = int64_t(blockIdx.y) * 64, c0 = int64_t(blockIdx.x) * 64;
+  const int64_t r0 = int64_t(blockIdx.y) * 64;
+  const int64_t c0 = (int64_t(blockIdx.z) * gridDim.x + blockIdx.x) * 64;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4
 #pragma unroll
   for (int k = 0; k < 64; k += 4) {
@@ -2245,8 +2249,8 @@ extern "C" int lmp_k_gemm_colsum_f32(int trans_a, int trans_b, size_t m, size_t 
       if (rc == LMP_OK && colsum_accumulate) rc = lmp_k_add_inplace(LMP_FLOAT32, colsum, dst, n);
     } else {
       LMP_RUNTIME_OR_FAIL(rt);
-      const uint32_t grid = uint32_t(trans_b ? (n + 3) / 4 : (n + 255) / 256);
-      hipLaunchKernelGGL(colsum_strided_f32, dim3(grid), dim3(256), 0, rt->stream, colsum, b,
+      const Grid2 grid = grid_2d(trans_b ? (n + 3) / 4 : (n + 255) / 256, 256);
+      hipLaunchKernelGGL(colsum_strided_f32, dim3(grid.x, grid.y), dim3(256), 0, rt->stream, colsum, b,
                          int(k), int(n), int(ldb), trans_b ? 1 : 0, colsum_accumulate ? 1 : 0);
       LMP_LAUNCH_CHECK("colsum_strided_f32");
     }
@@ -2382,7 +2386,8 @@ extern "C" int lmp_k_transpose(int dtype, void* out, const void* in, size_t m,
   const uint64_t gx = (n + 63) / 64, gy = (m + 63) / 64;
   if (gx > 0x7fffffffull || gy > 65535)
     return fail(LMP_ERR_UNSUPPORTED, "transpose: matrix too large");
-  const dim3 grid{uint32_t(gx), uint32_t(gy), 1u};
+  const Grid2 cols = grid_2d(gx, 256);
+  const dim3 grid{cols.x, uint32_t(gy), cols.y};
   switch (dtype) {
 #define LMP_CASE(CODE, T)                                                     \
   case CODE:                                                                  \

@@ -14,6 +14,17 @@ namespace lmp_hip {
 // (2^33 + 64 threads as a single wave).
 constexpr uint64_t kMaxGridThreads = 0xffffffffull;
 
+// `blocks` workgroups over two dimensions of a grid, y past 1 only where x alone
+// would have too many threads; block y * x_extent + x may lie past the last one.
+struct Grid2 {
+  uint32_t x = 1, y = 1;
+};
+inline Grid2 grid_2d(uint64_t blocks, int threads) {
+  const uint64_t most = kMaxGridThreads / uint64_t(threads);
+  const uint64_t y = (blocks + most - 1) / most;
+  return {uint32_t((blocks + y - 1) / y), uint32_t(y)};
+}
+
 // ------------------------------------------------------- products of up to 32 rows
 
 // K split over workgroups, `per_wg` values each; a workgroup's `waves` waves take
@@ -30,6 +41,11 @@ LMP_HD int k_range_end(int kb, int part, int k) {
 }
 
 constexpr int kRowsWaves = 4;
+
+// A workgroup for every 32 of n columns fits a grid.
+inline bool rows_fit(int64_t n) {
+  return uint64_t(n + 31) / 32 <= kMaxGridThreads / (64 * kRowsWaves);
+}
 
 // Rows kernel (B transposed, one workgroup per 32 columns).  A CU holds one
 // workgroup, so the split count is the one whose rounds of workgroups take the

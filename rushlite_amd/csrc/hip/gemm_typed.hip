@@ -499,8 +499,10 @@ template <typename T, bool TA, bool TB>
 __global__ __launch_bounds__(kThreads) void gemm_int(TypedArgs g) {
   using U = typename IntAcc<T>::U;
   __shared__ T As[kLds], Bs[kLds];
-  const int tiles_n = (g.n + kTile - 1) / kTile;
-  const int m0 = int(blockIdx.x / tiles_n) * kTile, n0 = int(blockIdx.x % tiles_n) * kTile;
+  const uint32_t tiles_n = uint32_t(g.n + kTile - 1) / kTile;
+  const uint64_t tile = uint64_t(blockIdx.y) * gridDim.x + blockIdx.x;
+  if (tile / tiles_n >= uint32_t(g.m + kTile - 1) / kTile) return;  // the whole workgroup
+  const int m0 = int(tile / tiles_n) * kTile, n0 = int(tile % tiles_n) * kTile;
   const int tr = threadIdx.x / 16, tc = threadIdx.x % 16;  // rows tr + 16i, cols tc + 16j
   U acc[4][4];
 #pragma unroll
@@ -585,8 +587,9 @@ int launch_typed(Runtime* rt, TypedArgs g) {
       scratch_free(g.part);  // stream-ordered: the fold reads it first
     }
   } else {
-    hipLaunchKernelGGL((gemm_int<T, TA, TB>), dim3(uint32_t(tiles)), dim3(kThreads), 0,
-                       rt->stream, g);
+    const Grid2 grid = grid_2d(uint64_t(tiles), kThreads);
+    hipLaunchKernelGGL((gemm_int<T, TA, TB>), dim3(grid.x, grid.y), dim3(kThreads), 0, rt->stream,
+                       g);
     LMP_LAUNCH_CHECK("gemm_int");
   }
   return LMP_OK;

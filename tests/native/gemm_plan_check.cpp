@@ -83,8 +83,21 @@ int thin_ranges() {
   return 0;
 }
 
+// grid_2d: every block, fewer than 2^32 threads a dimension, less than one row over.
+int grids() {
+  for (uint64_t blocks : {uint64_t(1), uint64_t(1000), (uint64_t(1) << 24) - 1, uint64_t(1) << 24,
+                          (uint64_t(1) << 24) + 1, uint64_t(1) << 29, uint64_t(0x7fffffff)}) {
+    const Grid2 g = grid_2d(blocks, 256);
+    CHECK(uint64_t(g.x) * 256 <= kMaxGridThreads && g.y <= 65535);
+    CHECK(uint64_t(g.x) * g.y >= blocks && uint64_t(g.x) * g.y - blocks < g.x);
+    CHECK(g.y == 1 || blocks * 256 > kMaxGridThreads);
+  }
+  CHECK(rows_fit(8192) && rows_fit((int64_t(1) << 29) - 32) && !rows_fit(int64_t(1) << 29));
+  return 0;
+}
+
 int main() {
-  if (bf3_grids() || bf3_pairs() || thin_ranges()) return 1;
+  if (bf3_grids() || bf3_pairs() || thin_ranges() || grids()) return 1;
   std::printf("gemm plans ok\n");
   return 0;
 }

@@ -36,3 +36,45 @@ def test_row_sums_past_a_grid(hip, rows, cols):
     a.free()
     out.free()
     hip.check(L.lmp_rt_empty_cache())
+
+
+def _ends(hip, buf, n, dtype):
+    """A few values at the start, the middle and the end of n."""
+    got = []
+    for at in (0, n // 2, n - 8):
+        x = np.zeros(8, dtype)
+        hip.check(hip.lib().lmp_rt_memcpy_d2h(x.ctypes.data_as(C.c_void_p),
+                                              C.c_void_p(buf.ptr + x.itemsize * at), x.nbytes))
+        got.append(x)
+    return np.concatenate(got)
+
+
+@pytest.mark.parametrize("kind", ["int_gemm", "transpose", "thin_rows", "strided_column_sums"])
+def test_matrix_kernels_past_a_grid(hip, kind):
+    """One workgroup of 256 lanes per tile, row or block of columns, 2^32 threads
+    or more in all: ones, so every result is the number of terms."""
+    L, n = hip.lib(), {"thin_rows": (1 << 29) + 32, "strided_column_sums": (1 << 26) + 8}.get(kind, (1 << 30) + 64)
+    t, code = {"int_gemm": (np.int16, hip.INT16), "transpose": (np.bool_, hip.BOOL)}.get(kind, (np.float32, hip.FLOAT32))
+    rows = {"thin_rows": 4, "strided_column_sums": 8}.get(kind, 1)
+    big, out = hip.DeviceBuffer((n, rows), t), hip.DeviceBuffer((n,), t)
+    one = hip.DeviceBuffer.from_numpy(np.ones(8, t))
+    hip.check(L.lmp_k_fill(code, big.ptr, n * rows, 1.0))
+    hip.check(L.lmp_k_fill(code, out.ptr, n, 0.0))
+    bufs = [big, out, one]
+    if kind == "int_gemm":
+        hip.check(L.lmp_k_gemm(code, 0, 0, n, 1, 1, big.ptr, 1, one.ptr, 1, out.ptr, 1, 0))
+    elif kind == "transpose":
+        hip.check(L.lmp_k_transpose(code, out.ptr, big.ptr, 1, n))
+    elif kind == "thin_rows":
+        hip.check(L.lmp_k_gemm_f32(0, 1, 1, n, 4, one.ptr, 4, big.ptr, 4, out.ptr, n, 0))
+    else:
+        sums = hip.DeviceBuffer((n,), t)
+        bufs.append(sums)
+        hip.check(L.lmp_k_fill(code, sums.ptr, n, 0.0))
+        hip.check(L.lmp_k_gemm_colsum_f32(0, 1, 1, n, 4, one.ptr, 4, big.ptr, 8, out.ptr, n, 0, sums.ptr, 0))
+        assert np.all(_ends(hip, sums, n, t) == 4)
+    want = 4 if rows > 1 else 1
+    assert np.all(_ends(hip, out, n, t) == want)
+    for b in bufs:
+        b.free()
+    hip.check(L.lmp_rt_empty_cache())
