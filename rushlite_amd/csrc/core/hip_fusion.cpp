@@ -24,7 +24,8 @@
 // stores it, with the nontemporal hint for large outputs; other layouts, and
 // float64, produce 16 bytes per lane too, with the flat index decomposed once
 // and carried over the lane's values with compile-time extents (outputs of
-// 2^31 values or more: one value per lane in 64-bit arithmetic).  Kernels launch on the library stream without a
+// 2^33 values or more, 2^31 in these layouts: one value per lane in 64-bit
+// arithmetic).  Kernels launch on the library stream without a
 // device synchronisation (the reference synchronises every launch,
 // nvrtc_backend.cpp:135-141).
 #include <cstdio>
@@ -405,8 +406,9 @@ Plan make_plan(const Region& r, const std::vector<size_t>& shape, bool f64) {
   std::vector<std::vector<stride_t>> strides;
   for (TensorImpl* leaf : r.leaves) strides.push_back(padded_strides(leaf->shape(), shape.size()));
   p.groups = coalesce(shape, strides);
-  // 32-bit indices from here on; larger outputs use the indexed loop.
-  if (p.n >= (1ull << 31)) return p;
+  // 32-bit indices from here on, of float4s or of single values; larger outputs
+  // use the indexed loop.
+  if (p.n >= (f64 ? 1ull << 31 : 1ull << 33)) return p;
   p.W = f64 ? 2 : 4;
   for (size_t l = 0; l < r.leaves.size() && l < 64; ++l)
     if ((reinterpret_cast<uintptr_t>(r.leaves[l]->raw()) & 15u) == 0) p.aligned |= uint64_t(1) << l;
@@ -422,7 +424,7 @@ Plan make_plan(const Region& r, const std::vector<size_t>& shape, bool f64) {
     p.vec = true;
     p.cols4 = cols / 4;
     p.nvec = p.n / 4;
-  } else {
+  } else if (p.n < (1ull << 31)) {
     p.quad = true;
     if (p.n < kShortOutput) p.W = 1;
     p.nvec = (p.n + p.W - 1) / p.W;
@@ -599,11 +601,14 @@ void emit_vec_body(std::ostringstream& os, const Region& r, const Plan& p, const
   const bool rows = p.groups.size() == 2;
   os << "  {\n  const unsigned v = " << block << " * " << kBlock << "u + threadIdx.x;\n";
   os << "  if (v < " << p.nvec << "u) {\n";
+  // Units are counted in 32 bits; the column of one in rows of 2^32 values or
+  // more takes 64.
+  const char* C = uint64_t(p.cols4) > 0xffffffffull / 4 ? "unsigned long" : "unsigned";
   if (rows) {
     os << "  const unsigned r = v / " << p.cols4 << "u;\n";
-    os << "  const unsigned c = (v - r * " << p.cols4 << "u) * 4u;\n";
+    os << "  const " << C << " c = (" << C << ")(v - r * " << p.cols4 << "u) * 4u;\n";
   } else {
-    os << "  const unsigned r = 0u;\n  const unsigned c = v * 4u;\n";
+    os << "  const unsigned r = 0u;\n  const " << C << " c = (" << C << ")v * 4u;\n";
   }
   for (size_t l = 0; l < nl; ++l) {
     const bool contig = !p.groups.empty() && p.groups[0].stride[l] == 1;

@@ -82,6 +82,34 @@ int main() {
     const P r = bin(LMP_BIN_ADD, bin(LMP_BIN_MUL, a, a), b);
     check("a*a+b float4", r, "lmp_v4");
   }
+  // Large outputs: float4s are counted in 32 bits up to 2^33 values, rows of
+  // 2^32 values or more with 64-bit columns; other layouts stop at 2^31.
+  {
+    P a = leaf({size_t(1) << 16, size_t(1) << 16}), b = leaf({size_t(1) << 16, 1});
+    const P r = bin(LMP_BIN_ADD, bin(LMP_BIN_MUL, a, a), b);
+    check("a*a+b float4 of 2^32 values", r, "lmp_v4 o;");
+  }
+  {
+    P a = leaf({(size_t(1) << 32) + 8});
+    const P r = bin(LMP_BIN_ADD, a, a);
+    check("a+a float4 of a flat 2^32 + 8", r, "const unsigned long c = (unsigned long)v * 4u;");
+  }
+  {
+    P a = leaf({2, (size_t(1) << 32) - 4});
+    P b = leaf({2, 1});
+    const P r = bin(LMP_BIN_ADD, a, b);
+    check("a+b float4 of rows of 2^32 - 4", r, "const unsigned c = (unsigned)(v");
+  }
+  {
+    P a = leaf({(size_t(1) << 33)});
+    const P r = bin(LMP_BIN_ADD, a, a);
+    check("a+a of 2^33 values", r, "i += (unsigned long)gridDim.x");
+  }
+  {
+    P a = leaf({(size_t(1) << 31) + 1});
+    const P r = bin(LMP_BIN_ADD, a, a);
+    check("a+a of an odd 2^31 + 1", r, "i += (unsigned long)gridDim.x");
+  }
   {
     P a = leaf({4, 1, 3}), b = leaf({1, 5, 3});
     const P r = bin(LMP_BIN_MUL, a, b);

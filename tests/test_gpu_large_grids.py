@@ -78,3 +78,32 @@ def test_matrix_kernels_past_a_grid(hip, kind):
     for b in bufs:
         b.free()
     hip.check(L.lmp_rt_empty_cache())
+
+
+@pytest.mark.parametrize("shape", [((1 << 32) + 8,), (1 << 16, 1 << 15)], ids=str)
+def test_fused_chain_of_2_31_values_or_more(hip, shape):
+    """A captured chain over 8 GiB or more runs on the float4 plan: marks around
+    2^31, 2^32 and the ends come out at their own places, ones elsewhere."""
+    import rushlite_amd as rsl
+    n = int(np.prod([int(d) for d in shape], dtype=np.int64))
+    with rsl.no_grad():
+        a = rsl.ones(list(shape), device=rsl.device.hip, dtype=rsl.dtype.float32)
+        base = rsl._storage_ptr(a.data)
+        places = [p for p in (0, 4, (1 << 31) - 8, 1 << 31, (1 << 32) - 8, 1 << 32, n - 8) if 0 <= p <= n - 8]
+        for i, p in enumerate(places):
+            x = np.arange(8, dtype=np.float32) + 10 * (i + 1)
+            hip.check(hip.lib().lmp_rt_memcpy_h2d(C.c_void_p(base + 4 * p), x.ctypes.data_as(C.c_void_p), 32))
+        with rsl.capture_on():
+            y = a * a + a
+        assert "lmp_v4 o;" in rsl._fused_source(y)
+        y.realize()
+        want = np.ones(8, np.float32)
+        for p in places + [n // 2 + 64, n - 64]:
+            x, got = np.zeros(8, np.float32), np.zeros(8, np.float32)
+            hip.check(hip.lib().lmp_rt_memcpy_d2h(x.ctypes.data_as(C.c_void_p), C.c_void_p(base + 4 * p), 32))
+            hip.check(hip.lib().lmp_rt_memcpy_d2h(got.ctypes.data_as(C.c_void_p),
+                                                  C.c_void_p(rsl._storage_ptr(y.data) + 4 * p), 32))
+            assert np.array_equal(got, x * x + x), p
+        assert np.array_equal(x, want)  # the last place is an unmarked one
+    del a, y
+    hip.check(hip.lib().lmp_rt_empty_cache())
