@@ -4,12 +4,26 @@
 // the chip); v_mfma_f32_32x32x16_bf16 does 1024.  An fp32 value x scaled by
 // 2^24 is h + m + l exactly (h = bf16(x), m = bf16(x - h), l = x - h - m: 8
 // bits each, round to nearest), so
-//   a*b = ah*bh + ah*bm + am*bh + am*bm + ah*bl + al*bh + (terms below 2^-26)
+//   a*b = ah*bh + ah*bm + am*bh + am*bm + ah*bl + al*bh + (am*bl + al*bm + al*bl)
 // takes six bf16 MFMAs with fp32 accumulation: 2.5 PFLOP/s / 6 = 419 TFLOP/s.
-// The error against float64 is that of the accumulation: six roundings per 16
-// values of k here, eight or more on the fp32 MFMAs (4096^3, normal operands:
-// 1.01e-6 against 1.15e-6; 512^3: 3.5e-7 against 4.0e-7).  At K = 32 and
-// below the dropped terms show, and those products stay on the fp32 MFMAs.
+//
+// Error.  The terms left out are 2^-24 of a product at most (a = b = 1 + 2^-8 -
+// 2^-17 leaves out 2^-24.01, with one sign), 2^-26.5 rms.  The leading products
+// ah*bh accumulate apart from the five small ones, whose roundings are 2^-8 of
+// theirs, and the two sums meet at the end: one rounding of the sum per 16
+// values of k where an fp32 MFMA rounds once per value or two.  A single
+// product (a diagonal operand) is one rounding and the terms left out: rms
+// 2.6e-8, at most 2^-23, where an fp32 product has 2.5e-8 and 2^-24.  The
+// 256 x 256 tile has no registers for a second sum and adds all six to one, the
+// leading product last (first, a single product was 5.3e-8 rms off, at most
+// 2.8e-7; last 3.3e-8 and 1.6e-7).  Relative 2-norm of the error against
+// float64, fp32 MFMAs / this, K unsplit unless marked (splits fp32 / this):
+//                              normal           positive         one term 2^12
+//   512 x 512 x 33             1.0e-7  3.9e-8   8.7e-8  4.2e-8   1.0e-7  7.0e-8
+//   512 x 512 x 128            2.0e-7  6.5e-8   1.6e-7  6.2e-8   2.1e-7  9.1e-8
+//   1000 x 2047 x 1531 (1/2)   7.0e-7  1.6e-7   5.9e-7  1.1e-7   7.0e-7  1.8e-7
+//   512 x 4096 x 4096 (4/2)    5.7e-7  2.7e-7   2.2e-7  1.6e-7   5.8e-7  3.0e-7
+//   4096^3 (one sum)           1.2e-6  1.0e-6
 //
 // Range.  The scaling makes the split exact for every finite fp32 value,
 // subnormals included (the last bit of one, 2^-149, becomes 2^-125, a normal
@@ -20,13 +34,13 @@
 // unscaled operands (fallback below): infinities, NaN and overflow come out as
 // fp32 products give them, and no other value takes that path unnoticed.
 //
-// What bounds it: power.  4096^3 takes 575-607 us on normal operands (227-239
-// TFLOP/s = 1.36-1.43 PFLOP/s of bf16, where a bf16 product of 8192^3 through
-// the vendor library reached 1.26) and 395-420 us on zeros: the clock falls
+// What bounds it: power.  4096^3 takes 555-640 us on normal operands (215-248
+// TFLOP/s = 1.29-1.49 PFLOP/s of bf16, where a bf16 product of 8192^3 through
+// the vendor library reached 1.26) and 395-470 us on zeros: the clock falls
 // under the MFMAs of random operands.  The fp32 MFMA kernel it replaced took
 // 965 us (143 TFLOP/s); a Linear's backward of 1000 x 2047 x 1531 (odd rows,
-// register-staged fp32 tiles and a separate column reduction) 212 -> 84 us;
-// the two backward products of 512 x 4096 x 4096 281 -> 181 us.
+// register-staged fp32 tiles and a separate column reduction) 211 -> 90 us;
+// the two backward products of 512 x 4096 x 4096 268 -> 182 us.
 //
 // Structure.  A workgroup owns a BM x BN tile of C, its waves TM x TN blocks
 // of 32 x 32 each; K advances 16 at a time through two LDS stages with one
@@ -38,8 +52,8 @@
 // Each operand value is converted once per workgroup (13 VALU operations per
 // pair, spread over the MFMAs by hand: a pair, then MPC MFMAs), and a fragment
 // feeds TN (or TM) x 2 MFMAs per plane, so neither the VALU nor the LDS is
-// near its limit.  The last of the six products is held past the barrier: it
-// reads registers only and covers the first fragment reads of the next step.
+// near its limit.  The leading product is held past the barrier: it reads
+// registers only and covers the first fragment reads of the next step.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -88,10 +102,12 @@ __device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32
   l = pack_bf16(xr - bf16_low(m), yr - bf16_high(m));
 }
 
-// DEPTH: steps of loads in flight ahead of the one being split.
-template <int WM_, int WN_, int TM_, int TN_, int DEPTH_, int MINB_>
+// DEPTH: steps of loads in flight ahead of the one being split.  APART: the five
+// small products of a step accumulate apart from the leading one.
+template <int WM_, int WN_, int TM_, int TN_, int DEPTH_, int MINB_, bool APART_>
 struct Bf3Cfg {
   static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, DEPTH = DEPTH_, MINB = MINB_;
+  static constexpr bool APART = APART_;
   static constexpr int NW = WM * WN, THREADS = 64 * NW;
   static constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
   static constexpr int A_OCT = BM * 16 + 64, B_OCT = BN * 16 + 64;  // bytes
@@ -248,11 +264,15 @@ __device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char*
   pa.init(g.a, g.lda, m0, g.m, k_load, C::A_OCT);
   pb.init(g.b, g.ldb, n0, g.n, k_load, C::B_OCT);
 
-  v16f acc[TM][TN];
+  // The leading products, and (APART) the small ones.
+  v16f acc[TM][TN], low[C::APART ? TM : 1][C::APART ? TN : 1];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = v16f(0.0f);
+    for (int j = 0; j < TN; ++j) {
+      acc[i][j] = v16f(0.0f);
+      if constexpr (C::APART) low[i][j] = v16f(0.0f);
+    }
 
   const int a_at = lh * C::A_OCT + (wm * TM * 32 + li) * 16;
   const int b_at = 3 * C::A_PLANE + lh * C::B_OCT + (wn * TN * 32 + li) * 16;
@@ -267,11 +287,11 @@ __device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char*
     for (int j = 0; j < TN; ++j)
       fb[p][j] = *reinterpret_cast<const bf8*>(s + p * C::B_PLANE + b_at + j * 512);
   };
-  auto mma = [&](int p, int q) {
+  auto mma_leading = [&]() {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = mfma_bf16(fa[p][i], fb[q][j], acc[i][j]);
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma_bf16(fa[0][i], fb[0][j], acc[i][j]);
   };
 
   // The step with the end of K first (when 16 does not divide it), then the
@@ -298,12 +318,13 @@ __device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char*
     pb.load_all(d % C::DEPTH, adv);
     --ahead;
   }
-  // Product (1, 1) of the step before is held past the barrier; zeros at first.
+  // The leading product of the step before is held past the barrier; zeros at
+  // first.
 #pragma unroll
-  for (int i = 0; i < TM; ++i) fa[1][i] = bf8(0);
+  for (int i = 0; i < TM; ++i) fa[0][i] = bf8(0);
 #pragma unroll
-  for (int j = 0; j < TN; ++j) fb[1][j] = bf8(0);
-  constexpr int PA_OF[5] = {0, 0, 2, 1, 0}, PB_OF[5] = {0, 2, 0, 0, 1};
+  for (int j = 0; j < TN; ++j) fb[0][j] = bf8(0);
+  constexpr int PA_OF[5] = {1, 1, 0, 0, 2}, PB_OF[5] = {1, 0, 1, 2, 0};
   constexpr int PAIRS = PA::PAIRS + PB::PAIRS;
   constexpr int MPC = (5 * MM - MM / 2) / PAIRS > 0 ? (5 * MM - MM / 2) / PAIRS : 1;
   // One step: STAGE holds it, SET the next one.
@@ -316,21 +337,21 @@ __device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char*
       if (do_cs && t + 1 < steps) pb.add_cs(set);
     const int adv = advance();
     --ahead;
-    read_a(s, 0);
+    read_a(s, 1);
+    read_b(s, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mma_leading();
+    __builtin_amdgcn_sched_barrier(0);
     read_b(s, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(1, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    read_b(s, 2);
     uint32_t h[4], m[4], l[4];
 #pragma unroll
     for (int c = 0; c < PAIRS; ++c) {
       // The next product's fragments, half a product or more ahead of it.
       const int q0 = c * MPC, q1 = c == PAIRS - 1 ? 5 * MM : q0 + MPC;
       auto covers = [&](int q) { return q0 <= q && q < q1; };
-      if (covers(MM / 2)) read_a(s, 2);
-      if (covers(MM + MM / 2)) read_a(s, 1);
-      if (covers(3 * MM - 1)) read_b(s, 1);
+      if (covers(MM / 2)) read_a(s, 0);
+      if (covers(MM + MM / 2)) read_b(s, 2);
+      if (covers(3 * MM - 1)) read_a(s, 2);
       const bool of_a = c < PA::PAIRS;
       const int ca = of_a ? c : c - PA::PAIRS;
       const int it = of_a ? ca / (PA::W / 2) : ca / (PB::W / 2);
@@ -343,7 +364,11 @@ __device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char*
       for (int q = q0; q < q1; ++q)
         if (q < 5 * MM) {
           const int pp = q / MM, i = (q % MM) / TN, j = q % TN;
-          acc[i][j] = mfma_bf16(fa[PA_OF[pp]][i], fb[PB_OF[pp]][j], acc[i][j]);
+          v16f& sum = [&]() -> v16f& {
+            if constexpr (C::APART) return low[i][j];
+            else return acc[i][j];
+          }();
+          sum = mfma_bf16(fa[PA_OF[pp]][i], fb[PB_OF[pp]][j], sum);
         }
       if (of_a && pr == PA::W / 2 - 1) {
         pa.put(it, d, C::A_PLANE, h, m, l);
@@ -367,14 +392,18 @@ __device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char*
   static_assert(D == 1 || D == 2, "steps are unrolled by two");
 #define LMP_BF3_STEP(U) \
   step(std::integral_constant<int, (U) % 2>{}, std::integral_constant<int, ((U) + 1) % D>{}, t)
-  for (int t = 0;;) {
+  // (One way out of the loop: with two the compiler holds both accumulators
+  // twice.)
+  int t = 0;
+  while (t + 1 < steps) {
     LMP_BF3_STEP(0);
-    if (++t == steps) break;
+    ++t;
     LMP_BF3_STEP(1);
-    if (++t == steps) break;
+    ++t;
   }
+  if (t < steps) LMP_BF3_STEP(0);
 #undef LMP_BF3_STEP
-  mma(1, 1);
+  mma_leading();
   __syncthreads();
 
   // Column sums: the parts of a column (its items' k ranges) in k order.
@@ -408,7 +437,8 @@ __device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char*
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float v = acc[i][j][r];
+        float v = acc[i][j][r];
+        if constexpr (C::APART) v = v + low[i][j][r];
         top = max(top, __builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
         acc[i][j][r] = v * kBf3Unscale;
       }
@@ -588,17 +618,17 @@ __global__ __launch_bounds__(256) void fold_bf3(Bf3Fold a, Bf3Fold b) {
 
 // ------------------------------------------------------------------- host
 
-using Bf3Big = Bf3Cfg<2, 4, 4, 2, 1, 1>;     // 256 x 256, 8 waves of 128 x 64
-using Bf3Wide = Bf3Cfg<4, 2, 2, 2, 1, 1>;    // 256 x 128, 8 waves of 64 x 64
-using Bf3Mid = Bf3Cfg<4, 2, 1, 2, 2, 1>;     // 128 x 128, 8 waves of 32 x 64
-using Bf3Flat = Bf3Cfg<1, 4, 2, 1, 2, 2>;    // 64 x 128, 4 waves of 64 x 32
-using Bf3Small = Bf3Cfg<2, 2, 1, 1, 2, 2>;   // 64 x 64, 4 waves of 32 x 32
+using Bf3Big = Bf3Cfg<2, 4, 4, 2, 1, 1, false>;   // 256 x 256, 8 waves of 128 x 64
+using Bf3Wide = Bf3Cfg<4, 2, 2, 2, 1, 1, true>;   // 256 x 128, 8 waves of 64 x 64
+using Bf3Mid = Bf3Cfg<4, 2, 1, 2, 2, 4, true>;    // 128 x 128, 8 waves of 32 x 64, two a CU
+using Bf3Flat = Bf3Cfg<1, 4, 2, 1, 2, 2, true>;   // 64 x 128, 4 waves of 64 x 32
+using Bf3Small = Bf3Cfg<2, 2, 1, 1, 2, 2, true>;  // 64 x 64, 4 waves of 32 x 32
 
 // kBf3Tiles is what these types are.
 template <class C>
 constexpr bool bf3_is(int cfg) {
   return kBf3Tiles[cfg].bm == C::BM && kBf3Tiles[cfg].bn == C::BN &&
-         kBf3Tiles[cfg].threads == C::THREADS;
+         kBf3Tiles[cfg].threads == C::THREADS && kBf3Tiles[cfg].apart == C::APART;
 }
 static_assert(bf3_is<Bf3Big>(0) && bf3_is<Bf3Wide>(1) && bf3_is<Bf3Mid>(2) &&
               bf3_is<Bf3Flat>(3) && bf3_is<Bf3Small>(4));

@@ -93,20 +93,25 @@ struct Bf3Plan {
 };
 
 // Time of one 16-wide k step of a workgroup, in us: `alone` on its CU, and
-// `shared` per workgroup where several take turns (medians of a sweep of 25
-// shapes, random operands, on one MI355X).  A larger tile moves and splits
-// each value fewer times: 4096^3 takes 574, 637, 700, 792 and about 980 us on
-// the five, 512 x 1000 x 4096 (K split) 44.0, 34.4, 34.4, 36.7, 39.4 and
-// 256 x 1024 x 1024 25.9, 19.8, 15.9, 14.5, 13.7.
+// `shared` per workgroup where several take turns (fitted to a sweep of 66
+// products over every tile and split, random operands, on one MI355X: the plan
+// takes 0.4% more than the best of the sweep, 8% at worst).  A larger tile moves
+// and splits each value fewer times: 4096^3 takes 565-640, 650-680, 710-780,
+// 870 and about 980 us on the five, 512 x 1000 x 4096 (K split) 44, 37, 34, 37,
+// 38 and 256 x 1024 x 1024 25, 19, 16, 15.5, 14.
+// APART: the leading products of a value accumulate apart from the small ones,
+// one rounding of the sum a step (six without, which the largest tile's
+// accumulators leave no registers for).
 struct Bf3Tile {
   int bm, bn, threads;
+  bool apart;
   float alone, shared;
 };
-constexpr Bf3Tile kBf3Tiles[] = {{256, 256, 512, 2.2f, 2.2f},
-                                 {256, 128, 512, 1.25f, 1.25f},
-                                 {128, 128, 512, 0.69f, 0.68f},
-                                 {64, 128, 256, 0.42f, 0.39f},
-                                 {64, 64, 256, 0.34f, 0.235f}};
+constexpr Bf3Tile kBf3Tiles[] = {{256, 256, 512, false, 1.78f, 2.4f},
+                                 {256, 128, 512, true, 1.07f, 1.45f},
+                                 {128, 128, 512, true, 0.61f, 0.75f},
+                                 {64, 128, 256, true, 0.475f, 0.441f},
+                                 {64, 64, 256, true, 0.26f, 0.252f}};
 
 inline int64_t bf3_tiles(const Bf3Tile& t, int64_t m, int64_t n) {
   return ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
@@ -117,7 +122,10 @@ inline int64_t bf3_tiles(const Bf3Tile& t, int64_t m, int64_t n) {
 // a second launch (2 us) and a round trip of the partials (5 TB/s).  The
 // partials stay within `scratch` bytes, the fixed workspace, whichever entry
 // point is called, so that all of them give the same bits; a split keeps at
-// least 64 k.  Launches that a grid cannot hold are left out.
+// least 64 k.  Launches that a grid cannot hold are left out, and the tile with
+// one accumulator where it would not give every CU one: there the fp32 kernels
+// split K, and their shorter chains round less than its long one (2048^3: 5.7e-7
+// from float64 in two splits, 7.0e-7 here unsplit, 2.7e-7 with sums apart).
 inline Bf3Plan bf3_plan(int64_t cus, int64_t scratch, int64_t m, int64_t n, int64_t k) {
   const int64_t steps = (k + kBf3K - 1) / kBf3K, mn = m * n;
   const int64_t most =
@@ -130,7 +138,8 @@ inline Bf3Plan bf3_plan(int64_t cus, int64_t scratch, int64_t m, int64_t n, int6
     const Bf3Tile& t = kBf3Tiles[c];
     const int64_t tiles = bf3_tiles(t, m, n);
     for (int s : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
-      if (s > 1 && s > most) break;
+      if (s > 1 && (s > most || !t.apart)) break;
+      if (!t.apart && tiles < cus) break;
       if (uint64_t(tiles) * uint64_t(s) > kMaxGridThreads / uint64_t(t.threads)) break;
       const float load = float((tiles * s + cus - 1) / cus);
       const float per_step = std::max(t.alone, load * t.shared);

@@ -44,6 +44,21 @@ int bf3_grids() {
   return 0;
 }
 
+// The tile with one accumulator: whole K, and a tile for every CU.
+int bf3_sums_apart() {
+  for (int64_t m : {64, 512, 1000, 2048, 4000, 4096, 8192, 20000})
+    for (int64_t n : {64, 1000, 2048, 4096, 8192})
+      for (int64_t k : {33, 64, 512, 4096, 100000}) {
+        const Bf3Plan p = bf3_plan(256, kScratch, m, n, k);
+        CHECK(p.cfg >= 0);
+        const Bf3Tile& t = kBf3Tiles[p.cfg];
+        CHECK(t.apart || (p.splits == 1 && bf3_tiles(t, m, n) >= 256));
+      }
+  CHECK(!kBf3Tiles[bf3_plan(256, kScratch, 4096, 4096, 4096).cfg].apart);
+  CHECK(kBf3Tiles[bf3_plan(256, kScratch, 2048, 2048, 2048).cfg].apart);
+  return 0;
+}
+
 // Two products share a launch only where their workgroups together fit a grid.
 int bf3_pairs() {
   CHECK(bf3_pair_fits(1, 1, 512));
@@ -97,7 +112,7 @@ int grids() {
 }
 
 int main() {
-  if (bf3_grids() || bf3_pairs() || thin_ranges() || grids()) return 1;
+  if (bf3_grids() || bf3_sums_apart() || bf3_pairs() || thin_ranges() || grids()) return 1;
   std::printf("gemm plans ok\n");
   return 0;
 }

@@ -80,6 +80,46 @@ def test_against_float64(hip, m, n, k, ta, tb):
     assert np.array_equal(acc.view(np.uint32), (c0 + got).view(np.uint32))
 
 
+# K just above 32 and long, on tiles whose leading products accumulate apart, and
+# (last) the 256 x 256 tile's one sum.
+@pytest.mark.parametrize("m,n,k", [(200, 256, 33), (512, 512, 40), (2048, 2048, 2048), (4096, 4096, 65)], ids=str)
+@pytest.mark.parametrize("family", ["normal", "dominated", "spread", "constant", "single"])
+def test_error_by_operand_family(hip, family, m, n, k):
+    """Operands besides normal ones: one term of each row 2^12 times the others,
+    terms spread over 2^40, equal terms whose parts left out have one sign, and a
+    single product per element.
+
+    The running sum is rounded once per 16 k (six times in the one sum), each
+    rounding at most an ulp and 0.58 half-ulps rms; averaged over a walk that
+    starts at zero and over mantissas 0.41 sqrt(roundings) half-ulps of the
+    result, 0.6 with the margin.  A single product is one addition: half an ulp,
+    half of one for the parts left out, and in the one sum, where it is the last
+    of six, up to another for the alignment of the smaller summand."""
+    rng = np.random.default_rng(m + k)
+    big = m * n >= 1 << 24
+    a, b = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (k, n)))
+    if family == "dominated":
+        a[np.arange(m), rng.integers(0, k, m)] *= np.float32(4096)
+    elif family == "spread":
+        a *= np.exp2(rng.uniform(-20, 20, (m, k))).astype(np.float32)
+    elif family == "constant":
+        a[:], b[:] = np.float32(1 + 2.0 ** -8 - 2.0 ** -17), np.float32(1 + 2.0 ** -8 - 2.0 ** -17)
+    elif family == "single":
+        a = rng.random((m, k), dtype=np.float32) + 1
+        b = np.zeros((k, n), np.float32)
+        b[np.arange(n) % k, np.arange(n)] = rng.random(n, dtype=np.float32) + 1
+    want = a[:512].astype(np.float64) @ b.astype(np.float64)
+    got = _run(hip, np.ascontiguousarray(a.T), b, 1, 0)[:512]
+    err = np.abs(got - want)
+    roundings = -(-k // 16) * (6 if big else 1)
+    if family == "single":
+        assert np.max(err / np.abs(want)) <= (3 if big else 2) * U * (1 + 2.0 ** -6)
+    elif family == "constant":  # every rounding may have one sign
+        assert np.max(err / np.abs(want)) <= (2 * roundings + 2) * U
+    else:
+        assert np.linalg.norm(err) <= (0.6 * np.sqrt(roundings) + 1) * U * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("m,n,k", [(129, 127, 49), (1000, 1027, 1531), (200, 200, 2049), (300, 700, 260)],
                          ids=str)
 def test_column_sums(hip, m, n, k):
