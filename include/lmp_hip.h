@@ -238,9 +238,18 @@ int lmp_k_reduce(int op, int dtype, void* out, const void* in, size_t outer,
 /* ----------------------------------------------------------------- matrix */
 
 /* C[m,n] (+)= op(A)[m,k] * op(B)[k,n], row-major, fp32 with fp32
- * accumulation (fp32 MFMAs, or bf16 MFMAs on operands split into three bf16
- * parts, no less exact; infinities, NaN and overflow as fp32 products).  trans_a != 0 means A is stored [k,m] (lda >= m); trans_b != 0
- * means B is stored [n,k] (ldb >= k).  accumulate != 0 adds into C.
+ * accumulation: fp32 MFMAs, or, for most products with an operand transposed
+ * and k > 32, bf16 MFMAs on operands split into three bf16 parts.  The split
+ * leaves out at most 2^-24 of each term (2^-26.5 rms), so a sum of one term has
+ * up to 2^-23 relative error (rms 2.6e-8) where an fp32 product has 2^-24
+ * (2.5e-8); it rounds the running sum once per 16 k, so sums of several terms
+ * are closer to their float64 values than the fp32 MFMAs' (four times at 512 x
+ * 512 x 512, twice with one dominating term).  Outputs that fill the chip with
+ * 256 x 256 tiles round it six times per 16 k: a sum of one term has up to 1.5 x
+ * 2^-23 (rms 3.3e-8), 4096^3 is as close as with fp32 MFMAs.  Infinities, NaN and
+ * overflow are those of fp32 products.
+ * trans_a != 0 means A is stored [k,m] (lda >= m); trans_b != 0 means B is
+ * stored [n,k] (ldb >= k).  accumulate != 0 adds into C.
  * Replaces matmul_cuda -> cudaMatMul (kernels.cu:83-110, matrix.cu:21-199);
  * the transposed forms replace the transpose-then-matmul pairs of
  * MatrixMultiplicationBackward (functions/matrix_ops.cpp:8-24). */
@@ -288,9 +297,9 @@ int lmp_k_linear_f32(int trans_a, int trans_b, size_t m, size_t n, size_t k,
  * through AddBackward's grad-of-broadcast reduction (grad_utils.cpp:10-36)
  * and the weight through transpose + matmul (functions/matrix_ops.cpp:15-20).
  * The column sums ride in the GEMM's own launches on the tiny kernel (K <= 512,
- * at most 2^21 multiply-adds), on the bf16 matrix cores when B is untransposed,
- * on the fp32 LDS tiles when K is not split, and on the short-K kernel (A transposed, K <= 32); otherwise
- * a second launch forms them after the GEMM (the dim-0 reduction for a
+ * at most 2^21 multiply-adds), on the bf16 matrix cores (A transposed, B not), on
+ * the fp32 LDS tiles when K is not split, and on the short-K kernel (A
+ * transposed, K <= 32); otherwise a second launch forms them after the GEMM (the dim-0 reduction for a
  * contiguous B, a strided column sum for any ldb).  Anything the second launch
  * needs is reserved before the first, so an error return leaves C and colsum
  * unchanged.  accumulate / colsum_accumulate add into C / colsum instead of

@@ -5,8 +5,8 @@
 // materialised transpose (the reference transposes then multiplies,
 // functions/matrix_ops.cpp:8-24, with a SIMT kernel, matrix.cu:21-145).
 //
-// Most products with K > 32 run on the bf16 matrix cores instead, each operand
-// in three parts (gemm_bf3.hpp; bf3_ok says which).
+// Gradient products (an operand transposed) with K > 32 run on the bf16 matrix
+// cores instead, each operand in three parts (gemm_bf3.hpp; bf3_ok).
 //
 // Tiling.  A workgroup of 4 waves owns a BM x BN tile of C; the waves form a
 // WGM x WGN grid and each wave owns TM x TN blocks of 32x32, accumulated by
@@ -1920,20 +1920,20 @@ Route gemm_route_f32(Runtime* rt, const GemmArgs& g, bool vec, bool direct_ok) {
 
 // Whether the product may run on the bf16 matrix cores (in place of any fp32
 // kernel but the tiny, short-K and M <= 32 ones):
-//   K > 32, where the error against float64 is no larger than the fp32 MFMAs'
-//     (512 x 512 outputs, normal operands, unsplit: 7.4e-8 fp32 and 8.3e-8
-//     here at K = 16, 1.02e-7 and 1.04e-7 at 32, 1.44e-7 and 1.35e-7 at 64;
-//     4096^3: 1.15e-6 and 1.01e-6);
-//   not a forward product X * W (neither transposed) of up to 512 rows.  Those
-//     are a training step's, and any other rounding of them moves the ReLU
-//     inputs that lie within it of zero to the other side: a step of the wide
-//     net (512 rows) on these products as well took 690 us instead of 755 us,
-//     but its updated weights then differed by up to 1.7e-5 from the fp32
-//     kernels' (themselves 1.5e-5 from float64 for the same reason), more than
-//     the 1e-5 that perf/cases.py holds a training step to.
+//   K > 32 (the short-K kernel and one K tile of the fp32 kernels are bound by
+//     writing C; above it the error against float64 is below theirs at every K
+//     measured, 33 to 262144: gemm_bf3.hpp);
+//   an operand transposed: a Linear's gradients.  X * W, its forward, keeps its
+//     bits, whatever the number of rows.  A ReLU input within rounding of zero
+//     takes one side or the other, and one unit and row that changes sides moves
+//     the updated weights of a step by up to 1.2e-5 (512 rows, 4096 wide; seen at
+//     one seed in five with the forward products here), past the 1e-5 that
+//     another order of 32-bit sums may show.  It would be the better side: such a
+//     step is 2.7e-8 from float64 here where the fp32 products' is 1.2e-5 off, and
+//     faster (755 -> 688 us; 4096^3 960 -> 590).
 template <bool TA, bool TB>
 bool bf3_ok(const GemmArgs& g) {
-  return g.k > kBK && (TA || TB || g.m > 512);
+  return g.k > kBK && (TA || TB);
 }
 
 template <bool TA, bool TB>

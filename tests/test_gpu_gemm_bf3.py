@@ -1,6 +1,7 @@
 """The fp32 GEMM that runs on the bf16 matrix cores, each operand in three
-parts (K > 32 and M > 32, with an operand transposed or M > 512), through the C
-ABI: tile edges, K remainders, splits of K, unaligned rows, the whole range of
+parts (K > 32 and M > 32 with an operand transposed), through the C ABI, and
+beside it the forward product X * W of the same shapes, which stays on the fp32
+MFMAs: tile edges, K remainders, splits of K, unaligned rows, the whole range of
 fp32, and values that are not finite."""
 import numpy as np
 import pytest
@@ -64,7 +65,7 @@ def test_against_float64(hip, m, n, k, ta, tb):
     half-ulps of the result's (a missing part of a split, 2^-17 of a term, is
     over it).  Aligned and odd row pitches give the same bits."""
     if not ta and not tb:
-        m += 512  # up to 512 rows X * W stays on the fp32 MFMAs
+        m += 512  # the fp32 MFMAs, within the same bounds
     A, B, a64, b64 = _operands(m, n, k, ta, tb, m * 31 + n * 7 + k)
     want = a64 @ b64
     got = _run(hip, A, B, ta, tb)
@@ -185,3 +186,13 @@ def test_values_that_are_not_finite(hip, m, n, k, kind):
     scale = np.abs(np.where(np.isfinite(A), A, 0)).astype(np.float64) @ np.abs(B).astype(np.float64)
     # the fallback's fp32 products round once per value of k
     assert np.all(np.abs(got[fin] - want[fin]) <= (2 * k + 70) * U * scale[fin])
+
+
+@pytest.mark.parametrize("n,k", [(256, 64), (1000, 160), (77, 333)], ids=str)
+def test_forward_rows_keep_their_bits(hip, n, k):
+    """X * W rounds the same whatever its number of rows (sizes with one tile and
+    no split of K): the first rows of a longer batch are the shorter one's."""
+    A, B, _, _ = _operands(1600, n, k, 0, 0, n)
+    want = _run(hip, A[:512], B, 0, 0)
+    for m in (513, 640, 1600):
+        assert np.array_equal(_run(hip, A[:m], B, 0, 0)[:512].view(np.uint32), want.view(np.uint32)), m
