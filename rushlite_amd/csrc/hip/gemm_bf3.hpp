@@ -31,8 +31,13 @@
 // that, and every infinity and NaN of the operands, leaves a non-finite value
 // in the accumulator (an infinite h has m = NaN), so a workgroup that finds
 // one after its K loop computes its tile again with fp32 MFMAs on the
-// unscaled operands (fallback below): infinities, NaN and overflow come out as
-// fp32 products give them, and no other value takes that path unnoticed.
+// unscaled operands, staged through the same LDS (fallback below): infinities,
+// NaN and overflow come out as fp32 products give them, and no other value takes
+// that path unnoticed.  A tile that takes it costs both products: with every
+// operand NaN 4096^3 takes 1440-1530 us and 512 x 4096 x 4096 227 (fp32 MFMAs
+// alone 950 and 139; 2120-3140 and 740 with the second product's operands read
+// straight from memory).  Looking for non-finite operands in the first step
+// instead (1070 and 158) cost finite ones 1-5%.
 //
 // What bounds it: power.  4096^3 takes 555-640 us on normal operands (215-248
 // TFLOP/s = 1.29-1.49 PFLOP/s of bf16, where a bf16 product of 8192^3 through
@@ -199,6 +204,15 @@ struct Bf3Panel {
       *reinterpret_cast<u2*>(q + 2 * plane) = u2{l[0], l[1]};
     }
   }
+  // Stores the values themselves, [k][row] with R + 4 values per k.
+  __device__ __forceinline__ void store_values(float* lds) const {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int q = int(threadIdx.x) + i * THREADS, row = KMAJOR ? q / PER_ROW : q % R;
+#pragma unroll
+      for (int j = 0; j < W; ++j) lds[(k[i] + j) * (R + 4) + row] = v[0][i][j];
+    }
+  }
   __device__ __forceinline__ void store_all(int set, char* lds, int plane) const {
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
@@ -307,6 +321,8 @@ __device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char*
     pb.load_all(0, advance());
     --ahead;
   }
+  // A tile that meets an infinity or a NaN in its first step goes to the fallback
+  // at once (a diverged run's operands are NaN throughout).
   if constexpr (!TB)
     if (do_cs) pb.add_cs(0);
   pa.store_all(0, smem, C::A_PLANE);
@@ -429,47 +445,74 @@ __device__ __forceinline__ void gemm_bf3_tile(const Bf3Args& args, int id, char*
     }
   }
 
-  // Unscale; a value that is not finite sends the workgroup to the fallback.
+  // A sum that is not finite sends the workgroup to the fallback.
+  if constexpr (C::APART) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = acc[i][j] + low[i][j];
+  }
   uint32_t top = 0;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float v = acc[i][j][r];
-        if constexpr (C::APART) v = v + low[i][j][r];
-        top = max(top, __builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
-        acc[i][j][r] = v * kBf3Unscale;
-      }
+      for (int r = 0; r < 16; ++r)
+        top = max(top, __builtin_bit_cast(uint32_t, float(acc[i][j][r])) & 0x7fffffffu);
   if (top >= 0x7f800000u) *flag = 1;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = acc[i][j] * kBf3Unscale;
   __syncthreads();
   if (*flag) {
+    // fp32 MFMAs on the unscaled values, staged through the same LDS.
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = v16f(0.0f);
-    for (int k = 0; k < k_len; k += 2) {
-      const bool in = k + lh < k_len;
-      const int64_t kk = k_begin + k + (in ? lh : 0);
-      float xa[TM], xb[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int64_t r = min(m0 + (wm * TM + i) * 32 + li, g.m - 1);
-        const float x = g.a[TA ? kk * g.lda + r : r * g.lda + kk];
-        xa[i] = in ? x : 0.0f;
-      }
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t c = min(n0 + (wn * TN + j) * 32 + li, g.n - 1);
-        const float x = g.b[TB ? c * g.ldb + kk : kk * g.ldb + c];
-        xb[j] = in ? x : 0.0f;
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma_f32(xa[i], xb[j], acc[i][j]);
+    Bf3Panel<C::BM, C::THREADS, !TA, 1> qa;
+    Bf3Panel<C::BN, C::THREADS, TB, 1> qb;
+    qa.init(g.a, g.lda, m0, g.m, k_load, C::A_OCT);
+    qb.init(g.b, g.ldb, n0, g.n, k_load, C::B_OCT);
+    int whole = full;  // whole steps not loaded yet
+    if (left) {
+      qa.load_tail(0, k_begin - k_load + full * kBf3K, left);
+      qb.load_tail(0, k_begin - k_load + full * kBf3K, left);
+    } else {
+      --whole;
+      qa.load_all(0, whole > 0 ? kBf3K : 0);
+      qb.load_all(0, whole > 0 ? kBf3K : 0);
     }
+    constexpr int PITCH_A = C::BM + 4, PITCH_B = C::BN + 4;
+    static_assert(kBf3K * (PITCH_A + PITCH_B) * 4 <= C::STAGE, "a stage holds a step's values");
+#pragma unroll 1
+    for (int t = 0; t < steps; ++t) {
+      float* sa = reinterpret_cast<float*>(smem + (t & 1) * C::STAGE);
+      float* sb = sa + kBf3K * PITCH_A;
+      qa.store_values(sa);
+      qb.store_values(sb);
+      __syncthreads();
+      if (whole > 0) {
+        --whole;
+        qa.load_all(0, whole > 0 ? kBf3K : 0);
+        qb.load_all(0, whole > 0 ? kBf3K : 0);
+      }
+#pragma unroll
+      for (int k = 0; k < kBf3K; k += 2) {
+        float xa[TM], xb[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) xa[i] = sa[(k + lh) * PITCH_A + (wm * TM + i) * 32 + li];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) xb[j] = sb[(k + lh) * PITCH_B + (wn * TN + j) * 32 + li];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = mfma_f32(xa[i], xb[j], acc[i][j]);
+      }
+    }
+    __syncthreads();  // the epilogue writes over the stages
   }
 
   float* out = partial ? args.part + split * args.part_stride : g.c;

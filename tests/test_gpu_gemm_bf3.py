@@ -196,3 +196,20 @@ def test_forward_rows_keep_their_bits(hip, n, k):
     want = _run(hip, A[:512], B, 0, 0)
     for m in (513, 640, 1600):
         assert np.array_equal(_run(hip, A[:m], B, 0, 0)[:512].view(np.uint32), want.view(np.uint32)), m
+
+
+@pytest.mark.parametrize("m,n,k", [(300, 270, 200), (200, 200, 2049), (260, 130, 37), (1100, 1100, 50)], ids=str)
+@pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0), (1, 1)])
+def test_tiles_computed_again(hip, m, n, k, ta, tb):
+    """Rows near the top of the range send every tile to the fp32 products, in
+    each orientation, with K tails, short splits and odd pitches: within their
+    rounding (one per value of k) everywhere, C's other columns untouched."""
+    rng = np.random.default_rng(m + k)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    a[::29] *= np.float32(1e33)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    scale = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    A, B = (np.ascontiguousarray(a.T) if ta else a), (np.ascontiguousarray(b.T) if tb else b)
+    got = _run(hip, A, B, ta, tb)
+    assert np.all(np.abs(got - want) <= (k + 70) * U * scale)
+    assert np.array_equal(_run(hip, A, B, ta, tb, pad=(1, 3)).view(np.uint32), got.view(np.uint32))
