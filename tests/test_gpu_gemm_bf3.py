@@ -213,3 +213,38 @@ def test_tiles_computed_again(hip, m, n, k, ta, tb):
     got = _run(hip, A, B, ta, tb)
     assert np.all(np.abs(got - want) <= (k + 70) * U * scale)
     assert np.array_equal(_run(hip, A, B, ta, tb, pad=(1, 3)).view(np.uint32), got.view(np.uint32))
+
+
+@pytest.mark.parametrize("m,n,k", [(2048, 2048, 2048), (1024, 1027, 4096), (700, 900, 100), (300, 511, 257)], ids=str)
+@pytest.mark.parametrize("positive", [False, True], ids=["normal", "positive"])
+def test_column_sums_close_to_float64(hip, m, n, k, positive):
+    """The column sums, whole K and split: a step's 4 or 8 values add in up to
+    three levels, the steps' and splits' errors are kept, and up to four parts
+    meet, so eight independent roundings of 0.58 half-ulps rms at most, whatever
+    K is (a quarter more for the sample)."""
+    A, B, _, b64 = _operands(m, n, k, 1, 0, n)
+    if positive:
+        B, b64 = np.abs(B), np.abs(b64)
+    want = b64.sum(0)
+    for pad in ((0, 0), (1, 3)):
+        _, cs = _run(hip, A, B, 1, 0, pad=pad, colsum=True)
+        assert np.linalg.norm(cs - want) <= 1.25 * 0.58 * np.sqrt(8) * U * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("k", [100, 2049])
+def test_column_sums_that_are_not_finite(hip, k):
+    """Infinities and NaN in a column, sums that overflow, columns of the largest
+    magnitudes that cancel: as the plain sum has them."""
+    m, n = 200, 70
+    A, B, _, _ = _operands(m, n, k, 1, 0, 3)
+    big = np.float32(3e38)
+    B[k // 2, 3], B[k // 3, 4], B[5, 5], B[7, 6], B[9, 6] = np.inf, -np.inf, np.nan, np.inf, -np.inf
+    B[:, 8] = big
+    B[:, 9] = 0
+    B[[20, 90], 9] = big, -big
+    _, cs = _run(hip, A, B, 1, 0, colsum=True)
+    assert cs[3] == np.inf and cs[4] == -np.inf and np.isnan(cs[5]) and np.isnan(cs[6])
+    assert cs[8] == np.inf and cs[9] == 0
+    ok = np.ones(n, bool)
+    ok[[3, 4, 5, 6, 8]] = False
+    assert np.all(np.isfinite(cs[ok]))
