@@ -157,9 +157,9 @@ bool is_reduce(const TensorImpl* t) {
 // that length (row_reduce_wave_f32, row_reduce_wave, row_reduce_f32 or
 // row_reduce_block: four interleaved accumulators of 16-byte units or single
 // values, their pairwise combination, a wave butterfly and, for a workgroup,
-// the waves in order; a long row that the eager kernel splits over workgroups
-// is walked part by part), so a fused softmax equals the eager one bit for
-// bit.  Rows of more than kLaneValues values per lane are not fused.  A long
+// the four waves in order, or in pairs; a long row of float4s that the eager
+// kernel splits over workgroups is walked part by part), so a fused softmax equals
+// the eager one bit for bit.  Rows of more than kLaneValues values per lane are not fused.  A long
 // row's values stay in registers between its passes: softmax over 10,000
 // classes with its loss, forward and backward, 2048 rows: 604 -> 327 us (sixteen
 // kernels before, elementwise regions around eager reductions), what the 1.9 GB
@@ -250,10 +250,13 @@ RowPlan row_plan(const Region& r) {
   if (is_long)
     p.parts = static_cast<int64_t>(lmp_hip::row_parts(static_cast<uint64_t>(device_cus()),
                                                       static_cast<uint64_t>(p.R),
-                                                      static_cast<uint64_t>(p.units())));
+                                                      static_cast<uint64_t>(p.units()),
+                                                      p.W == 4 ? lmp_hip::RowUnits::Float4
+                                                               : lmp_hip::RowUnits::Other));
   p.seg = (p.units() + p.parts - 1) / p.parts;
   if (p.parts * ((p.seg + p.lanes - 1) / p.lanes) * p.W > (f32 ? kLaneValues : kLaneValues / 2))
     return p;
+  if (p.W != 4 && p.parts > 1) return p;  // (too long for the line above, as parts are cut now)
   p.vec_load = p.W > 1;
   for (TensorImpl* leaf : r.leaves) {
     const std::vector<stride_t> st = padded_strides(leaf->shape(), nd);
@@ -1115,16 +1118,18 @@ std::string codegen_rows(const Region& r, const RowPlan& rp, const std::string& 
         os << "    v" << m << " = lmp_lane0(" << P << "v);\n";
     }
     if (group) {
-      // The waves' results in order, then the parts' from the identity.
+      // The four waves' results in order (rows of float4s), then the parts' from
+      // the identity; in pairs for other rows, which have one part.
       os << "    __syncthreads();\n";
       const auto part = [&](int64_t s) {
-        std::string t = "lmp_sh[" + std::to_string(slot + s) + "][0]";
-        for (int64_t w = 1; w < L / 64; ++w) {
-          os << "    const " << T << " w" << s << "_" << w << " = "
-             << comb(t, "lmp_sh[" + std::to_string(slot + s) + "][" + std::to_string(w) + "]") << ";\n";
-          t = "w" + std::to_string(s) + "_" + std::to_string(w);
-        }
-        return t;
+        const std::string sh = "lmp_sh[" + std::to_string(slot + s) + "][";
+        const auto join = [&](const std::string& a, const std::string& b, const std::string& n) {
+          os << "    const " << T << " w" << s << "_" << n << " = " << comb(a, b) << ";\n";
+          return "w" + std::to_string(s) + "_" + n;
+        };
+        const std::string a = join(sh + "0]", sh + "1]", "1");
+        if (W != 4) return join(a, join(sh + "2]", sh + "3]", "2"), "3");
+        return join(join(a, sh + "2]", "2"), sh + "3]", "3");
       };
       if (rp.parts == 1) {
         const std::string t = part(0);

@@ -11,7 +11,8 @@
 //                      partials are folded by a second pass in fixed order.
 //   other long rows -> (odd lengths, other types) the same with units of
 //                      one value, or of 16 bytes where the type, length and
-//                      alignment allow.
+//                      alignment allow, in longer parts whose results are a row
+//                      of their own to reduce.
 //   short rows      -> one wave per row (softmax/loss rows like [512,1000]),
 //                      float4 loads when rows are 16-byte multiples, four
 //                      loads in flight per lane; rows of at most 32 units
@@ -227,8 +228,8 @@ __global__ __launch_bounds__(kBlock) void row_reduce_wave_f32(
 }
 
 // Long rows of any type: row_reduce_f32 with units of V values (len, a multiple
-// of V, counted in units).  [2048, 10001] fp32 (one wave a row before) 23.5 ->
-// 15.3 us, 5.35 TB/s.
+// of V, counted in units), the waves' results in pairs.  [2048, 10001] fp32 (one
+// wave a row before) 23.5 -> 15.3 us, 5.35 TB/s.
 template <int OP, typename T, int V>
 __global__ __launch_bounds__(kBlock) void row_reduce_block(T* __restrict__ out,
                                                            const T* __restrict__ in, uint32_t units,
@@ -250,7 +251,17 @@ __global__ __launch_bounds__(kBlock) void row_reduce_block(T* __restrict__ out,
 #pragma unroll
     for (int u = 0; u < 4; ++u) acc[u] = combine_pack<OP>(acc[u], x[u]);
   }
-  for (; i < end; i += kBlock) acc[0] = combine_pack<OP>(acc[0], src[i]);
+  {  // at most three units per lane remain: their loads go out together
+    P x[3];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      x[u] = identity_pack<OP, T, V>();
+      if (i + u * kBlock < end) x[u] = src[i + u * kBlock];
+    }
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+      if (i + u * kBlock < end) acc[0] = combine_pack<OP>(acc[0], x[u]);
+  }
   P a = combine_pack<OP>(combine_pack<OP>(acc[0], acc[1]), combine_pack<OP>(acc[2], acc[3]));
 #pragma unroll
   for (int w = 1; w < V; w *= 2)
@@ -260,12 +271,9 @@ __global__ __launch_bounds__(kBlock) void row_reduce_block(T* __restrict__ out,
   __shared__ T lds[kWaves];
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    T r = lds[0];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) r = R::combine(r, lds[w]);
-    out[blockIdx.x] = r;
-  }
+  static_assert(kWaves == 4, "two pairs");
+  if (threadIdx.x == 0)
+    out[blockIdx.x] = R::combine(R::combine(lds[0], lds[1]), R::combine(lds[2], lds[3]));
 }
 
 // Rows of at most 32 units, G = 8, 16 or 32 lanes each (64 / G rows per wave):
@@ -296,15 +304,15 @@ __global__ __launch_bounds__(kBlock) void row_reduce_small(T* __restrict__ out,
 }
 
 // Fold `parts` consecutive partials per output in order.
-template <int OP, typename T>
-__global__ __launch_bounds__(kBlock) void fold_parts(T* __restrict__ out,
-                                                     const T* __restrict__ part,
+template <int OP>
+__global__ __launch_bounds__(kBlock) void fold_parts(float* __restrict__ out,
+                                                     const float* __restrict__ part,
                                                      uint64_t n,
                                                      uint32_t parts) {
-  using R = Reducer<OP, T>;
+  using R = Reducer<OP, float>;
   const uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
   if (i >= n) return;
-  T acc = R::identity();
+  float acc = R::identity();
   for (uint32_t p = 0; p < parts; ++p) acc = R::combine(acc, part[i * parts + p]);
   out[i] = acc;
 }
@@ -466,6 +474,9 @@ int launch_small_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t 
   return LMP_OK;
 }
 
+template <int OP, typename T>
+int reduce_rows(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len);
+
 // Rows of V-value units: short ones several to a wave, long ones a workgroup
 // (or several) each; *done false where neither applies.
 template <int OP, typename T, int V>
@@ -478,7 +489,9 @@ int reduce_rows_as(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len
     return launch_small_rows<OP, T, V, 32>(rt, out, in, rows, units);
   }
   if (len >= kLongRow && units <= kMaxU32Extent) {
-    const uint64_t parts = row_parts(uint64_t(rt->cu_count), rows, units);
+    constexpr bool kFloat4 = std::is_same_v<T, float> && V == 4;
+    const uint64_t parts = row_parts(uint64_t(rt->cu_count), rows, units,
+                                     kFloat4 ? RowUnits::Float4 : RowUnits::Other);
     const uint64_t seg = (units + parts - 1) / parts;
     if (rows * parts > 0x7fffffffull) return fail(LMP_ERR_UNSUPPORTED, "reduce: too many rows");
     T* dst = out;
@@ -489,7 +502,7 @@ int reduce_rows_as(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len
       dst = tmp;
     }
     const dim3 grid{uint32_t(rows * parts)};
-    if constexpr (std::is_same_v<T, float> && V == 4) {
+    if constexpr (kFloat4) {
       // Enough workgroups in flight, and the nontemporal hint for inputs that
       // cannot stay in the MALL.
       if (rows * len * sizeof(T) >= kStreamBytes)
@@ -505,10 +518,18 @@ int reduce_rows_as(Runtime* rt, T* out, const T* in, uint64_t rows, uint64_t len
       LMP_LAUNCH_CHECK("row_reduce_block");
     }
     if (parts > 1) {
-      hipLaunchKernelGGL((fold_parts<OP, T>), dim3(blocks_for(rows)), dim3(kBlock), 0, rt->stream,
-                         out, tmp, rows, uint32_t(parts));
-      LMP_LAUNCH_CHECK("fold_parts");
-      scratch_free(tmp);
+      int rc = LMP_OK;
+      if constexpr (kFloat4) {
+        hipLaunchKernelGGL((fold_parts<OP>), dim3(blocks_for(rows)), dim3(kBlock), 0, rt->stream,
+                           out, tmp, rows, uint32_t(parts));
+        LMP_LAUNCH_CHECK("fold_parts");
+      } else {
+        // Parts of many rounds: few enough for a row reduction of their own (one
+        // lane adding 976 of them took 60 of the 64 us of [1, 1000001]).
+        rc = reduce_rows<OP, T>(rt, out, tmp, rows, parts);
+      }
+      scratch_free(tmp);  // stream-ordered: the second pass reads it first
+      return rc;
     }
     return LMP_OK;
   }

@@ -67,3 +67,32 @@ def test_reduce_extremes(hip, shape):
     assert np.array_equal(hip.reduce("max", d, 1).numpy(), want)
     want = np.fmin.reduce(a, axis=1, initial=-low, keepdims=True)
     assert np.array_equal(hip.reduce("min", d, 1).numpy(), want)
+
+
+@pytest.mark.parametrize("shape", [(256, 3001), (1000, 2049), (64, 32767), (3, 32768 * 2 + 1), (4, 200001), (1, 1000003)],
+                         ids=str)
+@pytest.mark.parametrize("dt", ["f32", "f64", "i32"])
+def test_long_rows_in_parts(hip, dt, shape):
+    """Long rows that are not fp32 float4s: one launch until a second part has 64
+    units a lane, then parts whose results are a row of their own.  The sums of
+    positive values: a lane's chain is 2^-10 of the row or less, so what rounds is
+    the joins, each level half the one after it (0.58 half-ulps rms times sqrt 2,
+    and a second set for the parts)."""
+    import ctypes as C
+    a = _data(dt, shape, sum(shape))
+    a = np.abs(a)
+    d = hip.DeviceBuffer.from_numpy(a.reshape(shape + (1,)))
+    n0, n1 = C.c_uint64(), C.c_uint64()
+    hip.check(hip.lib().lmp_rt_kernel_launch_count(C.byref(n0)))
+    got = hip.reduce("sum", d, 1).numpy().reshape(-1)
+    hip.check(hip.lib().lmp_rt_kernel_launch_count(C.byref(n1)))
+    assert n1.value - n0.value == (1 if shape[1] < 2 * 64 * 256 else 2)
+    if dt == "i32":
+        assert np.array_equal(got, a.sum(axis=1, dtype=np.int64).astype(np.int32))
+        return
+    want = a.astype(np.longdouble).sum(axis=1)
+    u = np.finfo(a.dtype).eps / 2
+    err = np.abs((got - want) / want).astype(np.float64)
+    # up to four outputs: the root mean square of as few is under twice the expected
+    bound = 0.58 * np.sqrt(2 * (1 if n1.value - n0.value == 1 else 2)) * u
+    assert np.sqrt(np.mean(err ** 2)) <= bound * (1.15 if shape[0] >= 64 else 2)
