@@ -20,7 +20,7 @@
 // Column case (inner > 1, e.g. sum over dim 0, the bias-gradient reduction):
 //   units of 16 bytes along the columns where the type, inner extent and
 //   alignment allow, one value otherwise.  A workgroup owns a strip of up to
-//   64 units of one outer slice (the strips of a slice evenly wide) and a chunk
+//   1 KiB of one outer slice (the strips of a slice evenly wide) and a chunk
 //   of the reduced axis; its 256 lanes are row groups that take every rg-th row
 //   (8 loads in flight per lane) and combine in LDS by halving in fixed order.
 //   The axis is cut into S chunks so the grid holds about four workgroups per
@@ -28,8 +28,8 @@
 //   axis that would need chunks (bias gradients: [batch, out] with a batch of a
 //   few hundred) takes narrower strips instead, down to 64 bytes, so there is
 //   no second launch.
-//   Slices of at most 128 units take a lane per output.  No atomics: results
-//   are deterministic.
+//   Slices of a few units, and short axes of many outputs, take a lane per
+//   output.  No atomics: results are deterministic.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -388,12 +388,12 @@ __global__ __launch_bounds__(kBlock) void col_reduce_tile(T* __restrict__ dst,
 template <int OP, typename T, int V>
 __global__ __launch_bounds__(kBlock) void col_reduce_lane(T* __restrict__ out,
                                                           const T* __restrict__ in, uint64_t n,
-                                                          uint32_t units, uint32_t len) {
+                                                          FastDiv by_units, uint32_t len) {
   using P = Pack<T, V>;
-  const uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;  // below 2^32: the launch's threads
   if (i >= n) return;
-  const uint64_t o = i / units, c = i - o * units;
-  const P* src = reinterpret_cast<const P*>(in) + o * len * units + c;
+  const uint32_t units = by_units.d, o = by_units.div(i), c = i - o * units;
+  const P* src = reinterpret_cast<const P*>(in) + uint64_t(o) * len * units + c;
   P acc[kColUnroll];
 #pragma unroll
   for (int u = 0; u < kColUnroll; ++u) acc[u] = identity_pack<OP, T, V>();
@@ -415,9 +415,11 @@ __global__ __launch_bounds__(kBlock) void col_reduce_lane(T* __restrict__ out,
 
 // Column reduction with one lane per output element (o, c) of [outer, inner],
 // grid-striding over them: the axis is folded sequentially from the identity
-// (eight loads in flight, combined in row order).  Used when outer exceeds
-// the grid's z extent, where the kernels above would need one z slice per
-// outer index (reduct.cu:166-182 grid-strides over any output count too).
+// (eight loads in flight, combined in row order).  For more than 65535 outer
+// slices, whose results are the sequential fold's bit for bit, as
+// cpu/reduct.cpp:15-19 forms them, and for what the kernels above do not count:
+// extents of 2^31 or more, or more workgroups than a grid holds
+// (reduct.cu:166-182 grid-strides over any output count too).
 template <int OP, typename T>
 __global__ __launch_bounds__(kBlock) void col_reduce_flat(T* __restrict__ out,
                                                           const T* __restrict__ in,
@@ -592,36 +594,59 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
   const uint64_t units = inner / V, cus = uint64_t(rt->cu_count);
   const uint64_t n = outer * units;
   // A lane per output where a slice is too short to share a workgroup
-  // ([30000, 16, 16] fp32 34.6 -> 6.0 us), or where the outputs give every CU
-  // two workgroups of lanes of one 4-byte value, rows are 128 bytes or more and
-  // the axis is short ([4096, 64, 33] fp32: 7.0 us, 7.6 us in strips; float64
-  // 15.3 and 12.2).
-  if ((len * units <= 128 || (n >= cus * 2 * kBlock && units * kUnit >= 128 && len <= 64 && kUnit == 4)) &&
-      n <= kMaxGridThreads - kBlock) {
+  // ([30000, 16, 16] fp32 34.6 -> 6.0 us, [5912, 21, 16] float64 8.3 -> 4.2), or
+  // where the outputs give every CU two workgroups of lanes, rows are 128 bytes
+  // or more and the axis is short: 64 values of 4 bytes ([4096, 64, 33] fp32: 7.0
+  // us, 7.6 us in strips; float64 15.3 and 12.2), 16 units of more ([64, 1,
+  // 151296] float64 63 us in strips, 25.3 so).
+  const bool lanes = (len <= 32 && len * units <= 256) || (len * units <= 128 && n >= 8192) ||
+                     (n >= cus * 2 * kBlock && units * kUnit >= 128 &&
+                      len <= (kUnit == 4 ? 64 : 16));
+  if (lanes && n <= kMaxGridThreads - kBlock) {
     hipLaunchKernelGGL((col_reduce_lane<OP, T, V>), dim3(blocks_for(n)), dim3(kBlock), 0,
-                       rt->stream, out, in, n, uint32_t(units), uint32_t(len));
+                       rt->stream, out, in, n, FastDiv(uint32_t(units)), uint32_t(len));
     LMP_LAUNCH_CHECK("col_reduce_lane");
     return LMP_OK;
   }
-  // Strips of equal width, at most 64 units; narrower (256 bytes or more) for an
-  // axis of 128 rows or more while there are not four workgroups per CU
-  // ([16384,16384]: 176 us at 4/CU, 196 us at 8/CU; [256, 197, 768] at 3/CU 31.7
-  // us, at 4/CU 28.8; but [64, 151296] 7.5 us at 2.3/CU, 8.2 at 4/CU).
+  // Strips of equal width, 1 KiB and 256 units at most.  Strips of 16-byte units may be
+  // narrower (256 bytes or more) for an axis of 128 rows or more where that
+  // gives four workgroups per CU ([16384,16384]: 176 us at 4/CU, 196 us at 8/CU;
+  // [256, 197, 768] at 3/CU 31.7 us, at 4/CU 28.8; but [64, 151296] 7.5 us at
+  // 2.3/CU, 8.2 at 4/CU); they start on 128-byte lines where they are longer than
+  // one ([205, 128, 1152] fp32 19.8 -> 18.5 us, [25, 314, 1344] float64 18.1 ->
+  // 14.0), and are a power of two wide where that divides the row, so that the row
+  // groups meet in even pairs ([256, 197, 768] 3.95e-8 -> 3.81e-8 from float64).
+  // Strips of single values stay 1 KiB: [16, 576, 3135] fp32 27.5 -> 22.8 us, [15,
+  // 7424, 67] 12.8 -> 7.6, [14, 1004, 1269] float64 33.4 -> 25.9 against 256 bytes.
   const uint64_t target = cus * 4;
+  const uint64_t widest = std::min<uint64_t>(kBlock, 1024 / kUnit);  // a lane per unit at least
   const auto width = [&](uint64_t count) { return (units + count - 1) / count; };
-  uint64_t strips = (units + 63) / 64, S = 1;
-  while (len >= 128 && strips * outer < target && width(strips + 1) * kUnit >= 256) ++strips;
+  uint64_t strips = (units + widest - 1) / widest, S = 1;
+  if (kUnit == 16 && len >= 128)
+    while (strips * outer < target && width(strips + 1) * kUnit >= 256) ++strips;
   uint64_t cw = width(strips);
+  if (kUnit == 16 && cw > 8) {
+    const uint64_t lines = std::min(widest, (cw + 7) / 8 * 8), last = units % lines;
+    if (last == 0 || last >= lines / 2) cw = lines;  // no nearly empty last strip
+    uint64_t p = 16;
+    while (p * 2 <= cw) p *= 2;
+    if (p <= cw && units % p == 0) cw = p;
+  }
   strips = (units + cw - 1) / cw;
   if (strips * outer < target) {
     // One pass for an axis of at most 4096 rows, with strips of 64 bytes or
     // more until there are 128 workgroups, while a workgroup reads at most 128
     // KiB (more than that costs more than a second launch: [4096, 4096] 25 us
-    // in one pass, 15 us in two); the partials of a first pass always.
+    // in one pass, 15 us in two), or 256 KiB where there is one for every CU or
+    // the whole is 8 MiB at most ([3000, 256] fp32 7.4 us in two passes, 5.3 in
+    // one); the partials of a first pass always.
     uint64_t narrow = cw;
-    while (narrow * kUnit >= 128 && (units + narrow - 1) / narrow * outer < 128)
-      narrow = (narrow + 1) / 2;
-    if (second || (len <= kStripMaxLen && len * narrow * kUnit <= (128 << 10))) {
+    constexpr uint64_t least = 64 / kUnit;
+    while (narrow > least && (units + narrow - 1) / narrow * outer < 128)
+      narrow = std::max(least, (narrow + 1) / 2);
+    const uint64_t groups = (units + narrow - 1) / narrow * outer;
+    const bool more = groups >= cus || outer * len * inner * sizeof(T) <= (8 << 20);
+    if (second || (len <= kStripMaxLen && len * narrow * kUnit <= (more ? 256u << 10 : 128u << 10))) {
       cw = narrow;
       strips = (units + cw - 1) / cw;
     } else {
@@ -675,11 +700,10 @@ int reduce_cols(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t len,
   const bool lanes = sizeof(T) == 4 && len <= 64 && inner >= 32 && per_cu >= 2 && per_cu < 8;
   const bool pack = !lanes && packs<T>(in, inner) && aligned16(out);
   const uint64_t units = pack ? inner / kPackOf<T> : inner;
-  if (units > kMaxU32Extent || len > kMaxU32Extent || outer > 65535) {
-    // Extents past the tile kernel's 32-bit counters, and more than 65535
-    // outer slices.
+  // Extents past the tile kernel's 32-bit counters; more than 65535 outer slices
+  // (in row order, which callers can hold against the sequential fold).
+  if (units > kMaxU32Extent || len > kMaxU32Extent || outer > 65535)
     return reduce_cols_flat<OP, T>(rt, out, in, outer, len, inner);
-  }
   return pack ? reduce_cols_as<OP, T, kPackOf<T>>(rt, out, in, outer, len, inner)
               : reduce_cols_as<OP, T, 1>(rt, out, in, outer, len, inner);
 }

@@ -96,3 +96,34 @@ def test_long_rows_in_parts(hip, dt, shape):
     # up to four outputs: the root mean square of as few is under twice the expected
     bound = 0.58 * np.sqrt(2 * (1 if n1.value - n0.value == 1 else 2)) * u
     assert np.sqrt(np.mean(err ** 2)) <= bound * (1.15 if shape[0] >= 64 else 2)
+
+
+# The columns' rules at their edges: a lane per output for short axes and few
+# units, strips that end inside a 128-byte line or leave a short last one, power
+# of two widths, strips of single values of 1 KiB and less, one pass up to 256
+# KiB a workgroup, 65535 outer slices and more.
+MORE_COLS = [(300, 1, 300), (2100, 16, 64), (2100, 17, 64), (8200, 40, 3), (2800, 32, 8), (3, 33, 8), (2, 200, 130),
+             (1, 300, 1544), (5, 300, 600), (29, 2752, 24), (1, 3000, 256), (2, 130, 1100), (6, 700, 1027),
+             (65535, 5, 6), (65536, 5, 6), (65535, 33, 20)]
+
+
+@pytest.mark.parametrize("shape", MORE_COLS, ids=str)
+@pytest.mark.parametrize("dt", ["f32", "f64", "i32", "i16", "bool"])
+def test_reduce_column_rules(hip, dt, shape):
+    test_reduce_shapes(hip, dt, shape)
+
+
+@pytest.mark.parametrize("shape,launches", [((1, 3000, 256), 1), ((6, 3937, 64), 1), ((1, 4096, 4096), 2)], ids=str)
+def test_column_sums_in_one_pass(hip, shape, launches):
+    """A short axis of small slices in one launch; the sums' joins (0.58 half-ulps
+    rms a level, six or fewer count) bound the error of positive values."""
+    import ctypes as C
+    a = np.abs(_data("f32", shape, 5)) + np.float32(0.5)
+    d = hip.DeviceBuffer.from_numpy(a)
+    n0, n1 = C.c_uint64(), C.c_uint64()
+    hip.check(hip.lib().lmp_rt_kernel_launch_count(C.byref(n0)))
+    got = hip.reduce("sum", d, 1).numpy()
+    hip.check(hip.lib().lmp_rt_kernel_launch_count(C.byref(n1)))
+    assert n1.value - n0.value == launches
+    want = a.sum(axis=1, keepdims=True, dtype=np.float64)
+    assert np.linalg.norm(got - want) <= 0.58 * np.sqrt(6) * 2.0 ** -24 * np.linalg.norm(want)
