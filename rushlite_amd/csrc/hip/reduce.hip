@@ -609,10 +609,12 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
     return LMP_OK;
   }
   // Strips of equal width, 1 KiB and 256 units at most.  Strips of 16-byte units may be
-  // narrower (256 bytes or more) for an axis of 128 rows or more where that
-  // gives four workgroups per CU ([16384,16384]: 176 us at 4/CU, 196 us at 8/CU;
+  // narrower (256 bytes or more) for an axis of 128 rows or more until there are
+  // four workgroups per CU ([16384,16384]: 176 us at 4/CU, 196 us at 8/CU;
   // [256, 197, 768] at 3/CU 31.7 us, at 4/CU 28.8; but [64, 151296] 7.5 us at
-  // 2.3/CU, 8.2 at 4/CU); they start on 128-byte lines where they are longer than
+  // 2.3/CU, 8.2 at 4/CU), where rows are a whole number of 256 bytes ([8192, 4096]
+  // fp32 30.4 us in chunks of 1 KiB strips, 23.0 so; [10000, 10000] 68.1 and 77.5,
+  // [20000, 3000] 40.9 and 51.7, narrow strips lying across lines); they start on 128-byte lines where they are longer than
   // one ([205, 128, 1152] fp32 19.8 -> 18.5 us, [25, 314, 1344] float64 18.1 ->
   // 14.0), and are a power of two wide where that divides the row, so that the row
   // groups meet in even pairs ([256, 197, 768] 3.95e-8 -> 3.81e-8 from float64).
@@ -622,7 +624,7 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
   const uint64_t widest = std::min<uint64_t>(kBlock, 1024 / kUnit);  // a lane per unit at least
   const auto width = [&](uint64_t count) { return (units + count - 1) / count; };
   uint64_t strips = (units + widest - 1) / widest, S = 1;
-  if (kUnit == 16 && len >= 128)
+  if (kUnit == 16 && len >= 128 && units % 16 == 0)
     while (strips * outer < target && width(strips + 1) * kUnit >= 256) ++strips;
   uint64_t cw = width(strips);
   if (kUnit == 16 && cw > 8) {
