@@ -323,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void fold_parts(float* __restrict__ out,
 // rg * i, eight loads in flight.  dst layout [outer, S, units] (S == 1 writes
 // the final result).  HBM-bound: sum over the middle axis of [256, 197, 768]
 // 51.6 -> 28.8 us (5.4 TB/s; fp32 strips were sized without the outer extent:
-// 64-byte rows), over dim 0 of [16384, 16384] 160 -> 157 us (6.8 TB/s), float64
+// 64-byte rows), over dim 0 of [16384, 16384] 158.5 us (6.8 TB/s; 159 before), float64
 // 352 -> 317 us and int32 184 -> 164 us (units of one value before), of
 // [200000, 64] fp32 59 -> 14 us, float64 272 -> 21 us (the partials folded by one
 // lane per column), [16384, 3] 27.6 -> 6.5 us (three lanes of 256).
@@ -593,13 +593,13 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
   constexpr uint64_t kUnit = sizeof(T) * V;
   const uint64_t units = inner / V, cus = uint64_t(rt->cu_count);
   const uint64_t n = outer * units;
-  // A lane per output where a slice is too short to share a workgroup
-  // ([30000, 16, 16] fp32 34.6 -> 6.0 us, [5912, 21, 16] float64 8.3 -> 4.2), or
-  // where the outputs give every CU two workgroups of lanes, rows are 128 bytes
-  // or more and the axis is short: 64 values of 4 bytes ([4096, 64, 33] fp32: 7.0
-  // us, 7.6 us in strips; float64 15.3 and 12.2), 16 units of more ([64, 1,
-  // 151296] float64 63 us in strips, 25.3 so).
-  const bool lanes = (len <= 32 && len * units <= 256) || (len * units <= 128 && n >= 8192) ||
+  // A lane per output where a slice is too short to share a workgroup ([30000, 16,
+  // 16] fp32 34.6 -> 6.0 us, [5912, 21, 16] float64 8.3 -> 4.2) and there are many
+  // ([49, 21, 48] is 588 lanes: 3 us longer so), or where the outputs give every CU
+  // two workgroups of lanes, rows are 128 bytes or more and the axis is short: 64
+  // values of 4 bytes ([4096, 64, 33] fp32: 7.0 us, 7.6 us in strips; float64 15.3
+  // and 12.2), 16 units of more ([64, 1, 151296] float64 63 us in strips, 25.3 so).
+  const bool lanes = (len * units <= (len <= 32 ? 256 : 128) && n >= 8192) ||
                      (n >= cus * 2 * kBlock && units * kUnit >= 128 &&
                       len <= (kUnit == 4 ? 64 : 16));
   if (lanes && n <= kMaxGridThreads - kBlock) {
@@ -608,28 +608,36 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
     LMP_LAUNCH_CHECK("col_reduce_lane");
     return LMP_OK;
   }
-  // Strips of equal width, 1 KiB and 256 units at most.  Strips of 16-byte units may be
-  // narrower (256 bytes or more) for an axis of 128 rows or more until there are
-  // four workgroups per CU ([16384,16384]: 176 us at 4/CU, 196 us at 8/CU;
-  // [256, 197, 768] at 3/CU 31.7 us, at 4/CU 28.8; but [64, 151296] 7.5 us at
-  // 2.3/CU, 8.2 at 4/CU), where rows are a whole number of 256 bytes ([8192, 4096]
-  // fp32 30.4 us in chunks of 1 KiB strips, 23.0 so; [10000, 10000] 68.1 and 77.5,
-  // [20000, 3000] 40.9 and 51.7, narrow strips lying across lines); they start on 128-byte lines where they are longer than
-  // one ([205, 128, 1152] fp32 19.8 -> 18.5 us, [25, 314, 1344] float64 18.1 ->
-  // 14.0), and are a power of two wide where that divides the row, so that the row
-  // groups meet in even pairs ([256, 197, 768] 3.95e-8 -> 3.81e-8 from float64).
+  // Strips of equal width, 1 KiB and 256 units at most.  Strips of 16-byte units
+  // may be narrower for an axis of 128 rows or more until there are four
+  // workgroups per CU ([16384,16384]: 176 us at 4/CU, 196 us at 8/CU; [256, 197,
+  // 768] at 3/CU 31.7 us, at 4/CU 28.8; but [64, 151296] 7.5 us at 2.3/CU, 8.2 at
+  // 4/CU), where rows are a whole number of 256 bytes ([10000, 10000] fp32 68.1 us
+  // in strips of 1 KiB, 77.5 narrower ones lying across lines, [20000, 3000] 40.9
+  // and 51.7).  512 bytes are the least: [256, 65536] 11.9 us (256 bytes: 15.7),
+  // [192, 28928] 6.0 (10.3), [16384, 16384] 158 to 161 us wherever it starts (157
+  // to 169; 1 KiB: 161 to 168); 256 bytes below 256 MiB where rows are 8 KiB or
+  // less or there are four slices ([16384, 1024] 15.3 us, 17.6 with 512; [28, 145,
+  // 1984] 6.0 and 7.1, [8, 252, 2240] 4.3 and 6.5).  Where rows are whole 128-byte
+  // lines, strips longer than one start on them ([205, 128, 1152] fp32 19.8 -> 18.5
+  // us, [25, 314, 1344] float64 18.1 -> 14.0; else that only leaves lanes idle:
+  // [49, 7692, 48] fp32 15.1 us, 17.9 so).  They are a power of two wide where that
+  // divides the row, so that the row groups meet in even pairs ([256, 197, 768]
+  // 3.95e-8 -> 3.81e-8 from float64).
   // Strips of single values stay 1 KiB: [16, 576, 3135] fp32 27.5 -> 22.8 us, [15,
   // 7424, 67] 12.8 -> 7.6, [14, 1004, 1269] float64 33.4 -> 25.9 against 256 bytes.
-  const uint64_t target = cus * 4;
+  const uint64_t target = cus * 4, bytes = outer * len * inner * sizeof(T);
   const uint64_t widest = std::min<uint64_t>(kBlock, 1024 / kUnit);  // a lane per unit at least
+  const uint64_t slim =
+      (outer >= 4 || units * kUnit <= (8 << 10)) && bytes < kStreamBytes ? 256 : 512;
   const auto width = [&](uint64_t count) { return (units + count - 1) / count; };
   uint64_t strips = (units + widest - 1) / widest, S = 1;
   if (kUnit == 16 && len >= 128 && units % 16 == 0)
-    while (strips * outer < target && width(strips + 1) * kUnit >= 256) ++strips;
+    while (strips * outer < target && width(strips + 1) * kUnit >= slim) ++strips;
   uint64_t cw = width(strips);
   if (kUnit == 16 && cw > 8) {
     const uint64_t lines = std::min(widest, (cw + 7) / 8 * 8), last = units % lines;
-    if (last == 0 || last >= lines / 2) cw = lines;  // no nearly empty last strip
+    if (units % 8 == 0 && (last == 0 || last >= lines / 2)) cw = lines;  // no nearly empty last strip
     uint64_t p = 16;
     while (p * 2 <= cw) p *= 2;
     if (p <= cw && units % p == 0) cw = p;
@@ -640,15 +648,23 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
     // more until there are 128 workgroups, while a workgroup reads at most 128
     // KiB (more than that costs more than a second launch: [4096, 4096] 25 us
     // in one pass, 15 us in two), or 256 KiB where there is one for every CU or
-    // the whole is 8 MiB at most ([3000, 256] fp32 7.4 us in two passes, 5.3 in
-    // one); the partials of a first pass always.
+    // the whole is 16 MiB at most ([3000, 256] fp32 7.4 us in two passes, 5.3 in
+    // one; [3111, 1024] 7.9 and 5.9), down to a line per row ([896, 8192] 8.2 us
+    // in two passes, 5.9 in one) or to two lines' length where rows are no whole
+    // lines ([3, 500, 5000] float64 14.2 and 12.3); the partials of a first pass
+    // always.
     uint64_t narrow = cw;
-    constexpr uint64_t least = 64 / kUnit;
-    while (narrow > least && (units + narrow - 1) / narrow * outer < 128)
-      narrow = std::max(least, (narrow + 1) / 2);
-    const uint64_t groups = (units + narrow - 1) / narrow * outer;
-    const bool more = groups >= cus || outer * len * inner * sizeof(T) <= (8 << 20);
-    if (second || (len <= kStripMaxLen && len * narrow * kUnit <= (more ? 256u << 10 : 128u << 10))) {
+    constexpr uint64_t least = 64 / kUnit, line = 128 / kUnit;
+    const auto groups = [&] { return (units + narrow - 1) / narrow * outer; };
+    const bool lined = units % 8 == 0;
+    const auto fits = [&] {
+      const bool more = groups() >= cus || bytes <= (16 << 20);
+      return groups() >= target || len * narrow * kUnit <= (more ? 256u << 10 : 128u << 10);
+    };
+    while (narrow > least && groups() < 128) narrow = std::max(least, (narrow + 1) / 2);
+    while (kUnit == 16 && narrow >= (lined ? 2 : 4) * line && !fits())
+      narrow = lined ? (narrow / 2 + line - 1) / line * line : (narrow + 1) / 2;
+    if (second || (len <= kStripMaxLen && fits())) {
       cw = narrow;
       strips = (units + cw - 1) / cw;
     } else {
@@ -673,7 +689,7 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
   const FastDiv dcw{uint32_t(cw)}, dst_strips{uint32_t(strips)}, dS{uint32_t(S)};
   bool nt = false;
   if constexpr (kUnit == 16) {
-    nt = outer * len * inner * sizeof(T) >= kStreamBytes;
+    nt = bytes >= kStreamBytes;
     if (nt)
       hipLaunchKernelGGL((col_reduce_tile<OP, T, V, true>), dim3(uint32_t(blocks)), dim3(kBlock),
                          0, rt->stream, dst, in, uint32_t(units), uint32_t(len), uint32_t(chunk),

@@ -101,9 +101,11 @@ def test_long_rows_in_parts(hip, dt, shape):
 # The columns' rules at their edges: a lane per output for short axes and few
 # units, strips that end inside a 128-byte line or leave a short last one, power
 # of two widths, strips of single values of 1 KiB and less, one pass up to 256
-# KiB a workgroup, 65535 outer slices and more.
+# KiB a workgroup and down to a line (whole lines) or two (others), 512-byte and
+# 256-byte strips in parts, 65535 outer slices and more.
 MORE_COLS = [(300, 1, 300), (2100, 16, 64), (2100, 17, 64), (8200, 40, 3), (2800, 32, 8), (3, 33, 8), (2, 200, 130),
              (1, 300, 1544), (5, 300, 600), (29, 2752, 24), (1, 3000, 256), (2, 130, 1100), (6, 700, 1027),
+             (1, 896, 8192), (1, 192, 6400), (3, 500, 2500), (4, 4200, 512), (1, 4200, 2304), (49, 777, 48),
              (65535, 5, 6), (65536, 5, 6), (65535, 33, 20)]
 
 
@@ -113,7 +115,8 @@ def test_reduce_column_rules(hip, dt, shape):
     test_reduce_shapes(hip, dt, shape)
 
 
-@pytest.mark.parametrize("shape,launches", [((1, 3000, 256), 1), ((6, 3937, 64), 1), ((1, 4096, 4096), 2)], ids=str)
+@pytest.mark.parametrize("shape,launches", [((1, 3000, 256), 1), ((6, 3937, 64), 1), ((1, 3111, 1024), 1),
+                                            ((1, 896, 8192), 1), ((1, 4096, 4096), 2)], ids=str)
 def test_column_sums_in_one_pass(hip, shape, launches):
     """A short axis of small slices in one launch; the sums' joins (0.58 half-ulps
     rms a level, six or fewer count) bound the error of positive values."""
