@@ -269,7 +269,9 @@ int lmp_k_gemm_f32(int trans_a, int trans_b, size_t m, size_t n, size_t k,
  * device, reserved when the library's code object loads there and held until
  * the process ends) instead of the pool.  A product whose partials would not
  * fit fails with LMP_ERR_UNSUPPORTED (lmp_k_gemm_f32 serves it); config 4's
- * largest split (512 x 4096, K split four ways) uses exactly 32 MiB.  Calls
+ * largest split (512 x 4096, K split four ways) uses exactly 32 MiB.  Which
+ * products are refused is set by the fp32 kernels' split of K, also where the
+ * bf16 matrix cores run the product, whose own partials always fit.  Calls
  * allocate nothing and free nothing, and need nothing cleared between them
  * (every partial is written before it is read).  All calls on one GPU share
  * its workspace: calls whose kernels overlap on that GPU (graphs holding

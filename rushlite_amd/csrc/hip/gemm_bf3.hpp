@@ -44,7 +44,7 @@
 // the vendor library reached 1.26) and 395-470 us on zeros: the clock falls
 // under the MFMAs of random operands.  The fp32 MFMA kernel it replaced took
 // 965 us (143 TFLOP/s); a Linear's backward of 1000 x 2047 x 1531 (odd rows,
-// register-staged fp32 tiles and a separate column reduction) 211 -> 90 us;
+// register-staged fp32 tiles and a separate column reduction) 211 -> 84 us;
 // the two backward products of 512 x 4096 x 4096 268 -> 182 us.
 //
 // Structure.  A workgroup owns a BM x BN tile of C, its waves TM x TN blocks
