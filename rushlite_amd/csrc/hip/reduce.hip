@@ -597,11 +597,15 @@ int reduce_cols_as(Runtime* rt, T* out, const T* in, uint64_t outer, uint64_t le
   // 16] fp32 34.6 -> 6.0 us, [5912, 21, 16] float64 8.3 -> 4.2) and there are many
   // ([49, 21, 48] is 588 lanes: 3 us longer so), or where the outputs give every CU
   // two workgroups of lanes, rows are 128 bytes or more and the axis is short: 64
-  // values of 4 bytes ([4096, 64, 33] fp32: 7.0 us, 7.6 us in strips; float64 15.3
-  // and 12.2), 16 units of more ([64, 1, 151296] float64 63 us in strips, 25.3 so).
+  // values of 4 bytes ([60000, 8, 50] fp32 35.6 us in strips, 18.3 so), but for
+  // slices of one strip that give a workgroup over three values a lane ([10000,
+  // 20, 250] 29.9 us in strips, 35.8 by lanes, [25600, 16, 62] 17.7 and 18.5, [4096,
+  // 64, 33] 6.2 and 7.1; [20000, 24, 34] 14.3 and 12.2), or 16 units of other sizes
+  // ([64, 1, 151296] float64 63 us in strips, 25.3 so).
   const bool lanes = (len * units <= (len <= 32 ? 256 : 128) && n >= 8192) ||
                      (n >= cus * 2 * kBlock && units * kUnit >= 128 &&
-                      len <= (kUnit == 4 ? 64 : 16));
+                      len <= (kUnit == 4 ? 64 : 16) &&
+                      (kUnit != 4 || units > kBlock || len * units <= 7 * kBlock / 2));
   if (lanes && n <= kMaxGridThreads - kBlock) {
     hipLaunchKernelGGL((col_reduce_lane<OP, T, V>), dim3(blocks_for(n)), dim3(kBlock), 0,
                        rt->stream, out, in, n, FastDiv(uint32_t(units)), uint32_t(len));

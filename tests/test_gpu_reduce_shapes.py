@@ -99,13 +99,15 @@ def test_long_rows_in_parts(hip, dt, shape):
 
 
 # The columns' rules at their edges: a lane per output for short axes and few
-# units, strips that end inside a 128-byte line or leave a short last one, power
-# of two widths, strips of single values of 1 KiB and less, one pass up to 256
-# KiB a workgroup and down to a line (whole lines) or two (others), 512-byte and
-# 256-byte strips in parts, 65535 outer slices and more.
+# units, a workgroup a slice from three and a half values a lane on, strips that
+# end inside a 128-byte line or leave a short last one, power of two widths,
+# strips of single values of 1 KiB and less, one pass up to 256 KiB a workgroup
+# and down to a line (whole lines) or two (others), 512-byte and 256-byte strips
+# in parts, 65535 outer slices and more.
 MORE_COLS = [(300, 1, 300), (2100, 16, 64), (2100, 17, 64), (8200, 40, 3), (2800, 32, 8), (3, 33, 8), (2, 200, 130),
              (1, 300, 1544), (5, 300, 600), (29, 2752, 24), (1, 3000, 256), (2, 130, 1100), (6, 700, 1027),
              (1, 896, 8192), (1, 192, 6400), (3, 500, 2500), (4, 4200, 512), (1, 4200, 2304), (49, 777, 48),
+             (2600, 18, 51), (2600, 17, 51), (2100, 64, 63),
              (65535, 5, 6), (65536, 5, 6), (65535, 33, 20)]
 
 
